@@ -123,9 +123,10 @@ struct RasterArgs {
     int B, T, H, W;
     float sigma;
     // Wave-uniform quotients, divided once on the host (IEEE, as the kernels
-    // would): rsig = 1 / max(sigma, 1e-8), lscale = 2 / (3 H W) (dL/dpixel).
+    // would): rsig = 1 / max(sigma, 1e-8), nl2 = -log2(e) / max(sigma, 1e-8)
+    // (the exponent of the fast coverage), lscale = 2 / (3 H W) (dL/dpixel).
     // Set with set_sizes, which also fills B, T, H, W and sigma.
-    float rsig, lscale;
+    float rsig, nl2, lscale;
     const float* rec;      // B*T*REC
     const float* bg;       // B*3
     const float* target;   // B*H*W*3 (MODE_LOSS)
@@ -185,6 +186,7 @@ inline void set_sizes(RasterArgs& a, int B, int T, int H, int W, float sigma) {
     a.W = W;
     a.sigma = sigma;
     a.rsig = 1.0f / std::fmax(sigma, 1e-8f);
+    a.nl2 = (float)(-1.4426950408889634 / (double)std::fmax(sigma, 1e-8f));
     a.lscale = 2.0f / (float)(3 * (size_t)W * H);
 }
 

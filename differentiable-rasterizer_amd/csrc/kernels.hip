@@ -572,36 +572,39 @@ __device__ inline TileEnt ent_at(const TileEnt* __restrict__ te, int i) {
                                              (uint32_t)i * (uint32_t)sizeof(TileEnt));
 }
 
-// Field i0, i1 or i2 of the record for a per-lane e in {0, 1, 2}: the bits of
-// f_e as f0 ^ ((f0 ^ f1) & m1) ^ ((f0 ^ f2) & m2), m1 and m2 the lane masks of
-// e == 1 and e == 2 (its two bits, sign-extended). The two xors of scalar
-// fields are scalar; per lane it is two ands and a three-way xor, where a
-// select among scalar fields needs each field copied into a vector register
-// first (a vector instruction reads one scalar register at most): -0.8 us of
-// ~88 against the selects at B=16 256x256 T=128.
-__device__ inline float pick3_lane(const Rec& r, int e, int i0, int i1, int i2) {
-    const uint32_t b0 = __float_as_uint(r.f(i0));
-    const uint32_t x1 = b0 ^ __float_as_uint(r.f(i1)), x2 = b0 ^ __float_as_uint(r.f(i2));
-    const uint32_t m1 = (uint32_t)__builtin_amdgcn_sbfe(e, 0, 1), m2 = (uint32_t)__builtin_amdgcn_sbfe(e, 1, 1);
-    return __uint_as_float(b0 ^ (x1 & m1) ^ (x2 & m2));
-}
-
 struct Pix {
     float px, py;
 };
 
-// raster.rs:79-87; both branches are formed and the sign picks one.
+// The wave's lanes for which `c` holds (inactive lanes 0). HIP's __ballot widens
+// the condition to an integer and compares it again, two vector instructions
+// more per call than the builtin, which takes the compare's lane mask as is.
+__device__ inline uint64_t lane_mask(bool c) { return __builtin_amdgcn_ballot_w64(c); }
+__device__ inline bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// All lanes where bit `bit` of the wave-uniform v is set, else none.
+__device__ inline uint64_t all_lanes_if(uint32_t v, int bit) {
+    const uint32_t m = (uint32_t)((int32_t)(v << (31 - bit)) >> 31);
+    return (uint64_t)m << 32 | m;
+}
+
+// The softness as the sweeps use it: max(sigma, 1e-8), its reciprocal, and
+// -log2(e) / max(sigma, 1e-8).
+struct Soft {
+    float sig, rsig, nl2;
+};
+
+// raster.rs:79-87 of sd / sigma. The reference's two branches are one function,
+// 1 / (1 + e^-x): formed from one hardware exponential it is as exact on both
+// sides (1 + e^-x rounds once, and where e^-x overflows the result is 0), in
+// five instructions instead of nine with both branches and a select.
 template <bool FAST>
-__device__ inline float sigmoid_f(float x) {
-    if (FAST) {
-        float e = __expf(-fabsf(x));
-        float s = __builtin_amdgcn_rcpf(1.0f + e);
-        return x >= 0.0f ? s : e * s;
-    } else {
-        if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
-        float e = expf(x);
-        return e / (1.0f + e);
-    }
+__device__ inline float coverage_of(float sd, const Soft& so) {
+    if (FAST) return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sd * so.nl2));
+    const float x = sd / so.sig;
+    if (x >= 0.0f) return 1.0f / (1.0f + expf(-x));
+    const float e = expf(x);
+    return e / (1.0f + e);
 }
 
 // The exact-path geometry of one (pixel, triangle) pair: raster.rs:96-134 and
@@ -612,13 +615,28 @@ __device__ inline float sigmoid_f(float x) {
 // projection quotient from a refined reciprocal and takes the hardware square
 // root; otherwise both are IEEE operations. The choice is made per triangle,
 // outside this function, by a wave-uniform branch.
+//
+// The nearest point is kept as the reference rounds it, a + t (b - a): the
+// distance has formed t (b - a) for every edge already, so each edge's point is
+// two adds more, and the nearest edge's is two selects a coordinate. Choosing
+// the edge's vertex and vector per lane and forming the point again took twice
+// that (a scalar field must be copied into a vector register before a select).
+// Which edge is nearest and which side the pixel is on are wave masks, so that
+// neither costs a vector register or a compare where it is used. The sweeps are
+// bound by vector issue (3.2 cycles an instruction and SIMD at B=16 256x256
+// T=512), so their time follows the count: a three-edge entry went from ~82 to
+// 68 vector instructions here in the forward sweep and from ~105 to 84 in the
+// backward, its vertex terms from 61 to 47 with their reduction. Whole calls:
+// B=16 256x256 T=512 sigma 0.01 249 -> 220 us, B=16 256x256 T=128 95.8 -> 90.7
+// (through autograd), B=8 256x256 T=512 small 33.6 -> 31.5, B=1 383x509 T=400
+// 43.8 -> 40.1, B=16 128x128 T=128 66.7 -> 63.6.
 struct Geo {
-    float sd;      // signed distance, positive inside
-    float dist;    // |nearest segment distance|
-    float t;       // clamped projection parameter on the nearest edge
-    float ax, ay;  // first vertex of the nearest edge
-    float ex, ey;  // its edge vector b - a
-    int edge;      // nearest edge index, first minimum wins (grad.rs:236-242)
+    float dist;          // |nearest segment distance|
+    float t;             // clamped projection parameter on the nearest edge
+    float cpx, cpy;      // the nearest point a + t (b - a)
+    uint64_t inside;     // lanes whose pixel is inside the triangle
+    uint64_t e1, e2;     // lanes whose nearest edge is 1, 2 (else 0); the first minimum wins (grad.rs:236-242)
+    __device__ float sd() const { return in_mask(inside) ? dist : -dist; }  // positive inside
 };
 
 // The reference compares square-rooted distances (grad.rs:236-242): an earlier
@@ -632,7 +650,10 @@ __device__ inline bool same_sqrt(float a, float b) {
     return sqrtf(a) == sqrtf(b);
 }
 
-template <bool QUICK>
+// NEAREST: with the nearest edge's t, point and masks (the backward pass);
+// without, the distance and the side only, which a tie of edges leaves as they
+// are (the forward pass: no tie check).
+template <bool QUICK, bool NEAREST>
 __device__ inline Geo geometry(const Rec& r, Pix p) {
     float apx[3], apy[3];
     for (int j = 0; j < 3; j++) {
@@ -641,13 +662,8 @@ __device__ inline Geo geometry(const Rec& r, Pix p) {
     }
     float c[3];
     for (int j = 0; j < 3; j++) c[j] = r.f(R_E + 2 * j) * apy[j] - r.f(R_E + 2 * j + 1) * apx[j];
-    bool inside = (c[0] >= 0.0f && c[1] >= 0.0f && c[2] >= 0.0f) ||
-                  (c[0] <= 0.0f && c[1] <= 0.0f && c[2] <= 0.0f);
-    Geo g;
-    float best = INFINITY;
-    float d2v[3], tv[3];
-    g.edge = 0;
-    g.t = 0.0f;
+    Geo g{};
+    float d2v[3], tv[3], qx[3], qy[3];  // per edge: squared distance, t, t (b - a)
     for (int j = 0; j < 3; j++) {
         float ex = r.f(R_E + 2 * j), ey = r.f(R_E + 2 * j + 1);
         float dot = apx[j] * ex + apy[j] * ey;
@@ -667,37 +683,70 @@ __device__ inline Geo geometry(const Rec& r, Pix p) {
             float len2 = r.f(R_LEN2 + j);
             t = (len2 <= 1e-20f) ? 0.0f : rust_clamp(dot / len2, 0.0f, 1.0f);
         }
-        float dx = apx[j] - t * ex;
-        float dy = apy[j] - t * ey;
-        float d2 = dx * dx + dy * dy;
-        d2v[j] = d2;
         tv[j] = t;
-        if (d2 < best) {  // strict: the first minimum wins, NaN never does
-            best = d2;
-            g.edge = j;
-            g.t = t;
+        qx[j] = t * ex;
+        qy[j] = t * ey;
+        float dx = apx[j] - qx[j];
+        float dy = apy[j] - qy[j];
+        d2v[j] = dx * dx + dy * dy;
+    }
+    float best;
+    if (QUICK) {
+        // Finite coordinates of at most 1e4 (F_FAST): no NaN among the d2, and
+        // an area far above the cross products' rounding, so min and max of
+        // three decide the signs.
+        const float cmin = fminf(fminf(c[0], c[1]), c[2]), cmax = fmaxf(fmaxf(c[0], c[1]), c[2]);
+        g.inside = lane_mask(cmin >= 0.0f) | lane_mask(cmax <= 0.0f);
+        best = fminf(fminf(d2v[0], d2v[1]), d2v[2]);
+        if (NEAREST) {
+            g.e1 = lane_mask(d2v[0] != best);
+            g.e2 = g.e1 & lane_mask(d2v[1] != best);
+            g.e1 &= ~g.e2;
+        }
+    } else {
+        g.inside = (lane_mask(c[0] >= 0.0f) & lane_mask(c[1] >= 0.0f) & lane_mask(c[2] >= 0.0f)) |
+                   (lane_mask(c[0] <= 0.0f) & lane_mask(c[1] <= 0.0f) & lane_mask(c[2] <= 0.0f));
+        // strict: the first minimum wins, NaN never does (all NaN: edge 0, t 0)
+        best = INFINITY;
+        int edge = 0;
+        bool none = true;
+        for (int j = 0; j < 3; j++)
+            if (d2v[j] < best) {
+                best = d2v[j];
+                edge = j;
+                none = false;
+            }
+        if (NEAREST) {
+            g.e1 = lane_mask(edge == 1);
+            g.e2 = lane_mask(edge == 2);
+            if (none) {
+                tv[0] = 0.0f;
+                qx[0] = 0.0f * r.f(R_E);
+                qy[0] = 0.0f * r.f(R_E + 1);
+            }
         }
     }
-    // Near ties are rare; the wave takes the square roots at every lane when
-    // any lane has one (a wave-uniform branch, so no divergent control flow
-    // for the compiler to thread path flags through), and the others keep
-    // their edge. Edge 0 wins over edge 1, as the first minimum.
-    const float near = best * 1.0000005f;
-    const bool tie0 = g.edge > 0 && d2v[0] <= near, tie1 = g.edge > 1 && d2v[1] <= near;
-    if (__builtin_amdgcn_ballot_w64(tie0 || tie1) != 0) {
-        const bool eq0 = same_sqrt(d2v[0], best), eq1 = same_sqrt(d2v[1], best);
-        const bool s0 = tie0 && eq0, s1 = !s0 && tie1 && eq1;
-        g.t = s0 ? tv[0] : (s1 ? tv[1] : g.t);
-        g.edge = s0 ? 0 : (s1 ? 1 : g.edge);
-    }
-    const int ed = g.edge;
-    g.ax = pick3_lane(r, ed, R_V + 0, R_V + 2, R_V + 4);
-    g.ay = pick3_lane(r, ed, R_V + 1, R_V + 3, R_V + 5);
-    g.ex = pick3_lane(r, ed, R_E + 0, R_E + 2, R_E + 4);
-    g.ey = pick3_lane(r, ed, R_E + 1, R_E + 3, R_E + 5);
     // sqrt is monotone, so sqrt(min d2) == min sqrt(d2) (raster.rs:97-99).
     g.dist = QUICK ? __builtin_amdgcn_sqrtf(best) : sqrtf(best);
-    g.sd = inside ? g.dist : -g.dist;
+    if (NEAREST) {
+        // Near ties are rare; the wave takes the square roots at every lane when
+        // any lane has one (a wave-uniform branch, so no divergent control flow
+        // for the compiler to thread path flags through), and the others keep
+        // their edge. Edge 0 wins over edge 1, as the first minimum.
+        const float near = best * 1.0000005f;
+        const uint64_t tie0 = lane_mask(d2v[0] <= near) & (g.e1 | g.e2), tie1 = lane_mask(d2v[1] <= near) & g.e2;
+        if ((tie0 | tie1) != 0) {
+            const uint64_t s0 = tie0 & lane_mask(same_sqrt(d2v[0], best));
+            const uint64_t s1 = tie1 & ~s0 & lane_mask(same_sqrt(d2v[1], best));
+            g.e1 = (g.e1 & ~s0) | s1;
+            g.e2 &= ~(s0 | s1);
+        }
+        const bool e1 = in_mask(g.e1), e2 = in_mask(g.e2);
+        auto pick = [&](float f0, float f1, float f2) { return e2 ? f2 : (e1 ? f1 : f0); };
+        g.t = pick(tv[0], tv[1], tv[2]);
+        g.cpx = pick(r.f(R_V + 0) + qx[0], r.f(R_V + 2) + qx[1], r.f(R_V + 4) + qx[2]);
+        g.cpy = pick(r.f(R_V + 1) + qy[0], r.f(R_V + 3) + qy[1], r.f(R_V + 5) + qy[2]);
+    }
     return g;
 }
 
@@ -746,8 +795,8 @@ __device__ inline void load_entry(const float* __restrict__ rec, uint32_t off, u
 }
 
 // The edge's fields come from its block of the record (load_entry).
-__device__ inline Geo geometry1(const Rec& r, const f8v& eb, Pix p, uint32_t plan) {
-    const int j = (int)(plan & 3u);
+__device__ inline Geo geometry1(const f8v& eb, Pix p, uint32_t plan) {
+    static_assert(PLAN_INNER == 4, "geometry1 reads the plan's bits");
     const float ax = eb[0], ay = eb[1], ex = eb[2], ey = eb[3], len2 = eb[4], rl = eb[5];
     const float apx = p.px - ax, apy = p.py - ay;
     const float c = ex * apy - ey * apx;
@@ -756,55 +805,52 @@ __device__ inline Geo geometry1(const Rec& r, const f8v& eb, Pix p, uint32_t pla
     const float res = fmaf(-q0, len2, dot);
     Geo g;
     g.t = __builtin_amdgcn_fmed3f(fmaf(res, rl, q0), 0.0f, 1.0f);
-    const float dx = apx - g.t * ex;
-    const float dy = apy - g.t * ey;
+    const float qx = g.t * ex, qy = g.t * ey;
+    const float dx = apx - qx;
+    const float dy = apy - qy;
     g.dist = __builtin_amdgcn_sqrtf(dx * dx + dy * dy);
     // c <= 0 is -c >= 0, also for c = +-0
     const float cs = c * eb[6];  // the orientation flag as an exact factor of +-1
-    const bool inside = (plan & PLAN_INNER) && cs >= 0.0f;
-    g.sd = inside ? g.dist : -g.dist;
-    g.edge = j;
-    g.ax = ax;
-    g.ay = ay;
-    g.ex = ex;
-    g.ey = ey;
+    g.inside = lane_mask(cs >= 0.0f) & all_lanes_if(plan, 2);  // PLAN_INNER
+    g.e1 = all_lanes_if(plan, 0);  // the plan's edge is 0, 1 or 2
+    g.e2 = all_lanes_if(plan, 1);
+    g.cpx = ax + qx;
+    g.cpy = ay + qy;
     return g;
 }
 
 // Exact-path coverage of one pair. The branches on the triangle's F_FAST flag
 // and on the plan are wave-uniform; the empty volatile asm keeps the compiler
 // from if-converting them, which would evaluate every variant every time.
-template <bool FAST>
-__device__ inline void exact_cov(const Rec& r, const f8v& eb, Pix p, uint32_t code, float rsig, float sig, Geo& g,
+template <bool FAST, bool NEAREST>
+__device__ inline void exact_cov(const Rec& r, const f8v& eb, Pix p, uint32_t code, const Soft& so, Geo& g,
                                  float& cov) {
     // single-edge plans are given to F_FAST triangles only (build_list)
     if (FAST && (code & ENT_SINGLE)) {
-        g = geometry1(r, eb, p, (code >> 2) & 7u);
-        cov = sigmoid_f<true>(g.sd * rsig);
+        g = geometry1(eb, p, (code >> 2) & 7u);
     } else if (FAST && (r.i(R_FLAGS) & F_FAST)) {
         asm volatile("");
-        g = geometry<true>(r, p);
-        cov = sigmoid_f<true>(g.sd * rsig);
+        g = geometry<true, NEAREST>(r, p);
     } else {
         asm volatile("");
-        g = geometry<false>(r, p);
-        cov = sigmoid_f<FAST>(FAST ? g.sd * rsig : g.sd / sig);
+        g = geometry<false, NEAREST>(r, p);
     }
+    cov = coverage_of<FAST>(g.sd(), so);
 }
 
-// The exact coverage at the lanes of `bandm` (`band`: this lane's bit), 1.0f
+// The exact coverage at the lanes of `bandm`, 1.0f
 // at the others. Every lane evaluates it, under a wave-uniform branch on
 // `bandm`, and the others discard theirs: a divergent branch would cost the
 // same vector issue (masked lanes issue alike) plus the exec-mask saves and
 // restores, and makes the compiler carry flags through the branches around it.
-template <bool FAST>
-__device__ inline void band_cov(const Rec& r, const f8v& eb, Pix p, uint32_t code, uint64_t bandm, bool band,
-                                float rsig, float sig, Geo& g, float& cov) {
+template <bool FAST, bool NEAREST>
+__device__ inline void band_cov(const Rec& r, const f8v& eb, Pix p, uint32_t code, uint64_t bandm, const Soft& so,
+                                Geo& g, float& cov) {
     cov = 1.0f;
     if (bandm != 0) {
         float c;
-        exact_cov<FAST>(r, eb, p, code, rsig, sig, g, c);
-        cov = band ? c : 1.0f;
+        exact_cov<FAST, NEAREST>(r, eb, p, code, so, g, c);
+        cov = in_mask(bandm) ? c : 1.0f;
     }
 }
 
@@ -818,11 +864,6 @@ template <int ctrl>
 __device__ inline float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, false));
 }
-
-// The wave's lanes for which `c` holds (inactive lanes 0). HIP's __ballot widens
-// the condition to an integer and compares it again, two vector instructions
-// more per call than the builtin, which takes the compare's lane mask as is.
-__device__ inline uint64_t lane_mask(bool c) { return __builtin_amdgcn_ballot_w64(c); }
 
 // Wave-uniform copies of values every lane holds (loaded from one address).
 // The builtin returns int: widen through uint32_t, never by sign extension.
@@ -1061,13 +1102,14 @@ classify:
 // Per-pixel weight of one triangle: returns the mask of the lanes where the
 // pair contributes (not outside the box, not classified far outside, and
 // w > MIN_WEIGHT). `bandm` holds the lanes where the exact path ran with a
-// coverage below 1.0f, and there `g` holds its geometry. The tests are
+// coverage below 1.0f, and there `g` holds its geometry (NEAREST: see `geometry`).
+// The tests are
 // predicates rather than branches; only the exact path is a (divergent)
 // branch, so the wave runs it once for the lanes that need it.
-template <bool FAST>
+template <bool FAST, bool NEAREST>
 __device__ inline uint64_t pair_weight(const Rec& r, const f8v& eb, uint32_t ent, int x, int y,
                                        Pix p, uint64_t validm, float& w, float& cov, uint64_t& bandm, Geo& g,
-                                       float rsig, float sig) {
+                                       const Soft& so) {
     const float alpha = r.f(R_A);
     cov = 1.0f;
     // The lane sets are wave masks (`validm`: the lanes whose pixel is in the
@@ -1090,8 +1132,8 @@ __device__ inline uint64_t pair_weight(const Rec& r, const f8v& eb, uint32_t ent
         // pixel (more than 17 sigma + slack inside every edge line) gets
         // exp(-x) < 2^-24 and coverage exactly 1.0f, as classified; a far one
         // (beyond `far`) a weight below MIN_WEIGHT, skipped as classified.
-        g = geometry1(r, eb, p, (ent >> 2) & 7u);
-        cov = sigmoid_f<true>(g.sd * rsig);
+        g = geometry1(eb, p, (ent >> 2) & 7u);
+        cov = coverage_of<true>(g.sd(), so);
         w = alpha * cov;
         bandm = actm & lane_mask(cov != 1.0f);
         return actm & lane_mask(!(w <= MIN_WEIGHT));
@@ -1102,10 +1144,10 @@ __device__ inline uint64_t pair_weight(const Rec& r, const f8v& eb, uint32_t ent
         // edge: a pixel that the edge-line distances would class deep gets
         // coverage exactly 1.0f, a far one a weight below MIN_WEIGHT.
         asm volatile("");
-        g = geometry<true>(r, p);
-        cov = sigmoid_f<true>(g.sd * rsig);
+        g = geometry<true, NEAREST>(r, p);
+        cov = coverage_of<true>(g.sd(), so);
     } else {
-        band_cov<FAST>(r, eb, p, ent, bandm, __builtin_amdgcn_inverse_ballot_w64(bandm), rsig, sig, g, cov);
+        band_cov<FAST, NEAREST>(r, eb, p, ent, bandm, so, g, cov);
     }
     w = alpha * cov;
     // `bandm` hands the backward pass the lanes whose coverage it must evaluate:
@@ -1297,7 +1339,7 @@ __device__ inline TileGeo tile_geo_split(int W, int H, int gx, int gy, const int
 // segment of fused_seg_kernel).
 template <int MODE, bool FAST, bool CKPT, bool MERGE = false, bool ROWS = false>
 __device__ __forceinline__ void forward_sweep(const RasterArgs& a, const float* __restrict__ rec, const TileGeo& tg,
-                                              uint64_t validm, float rsig, float sig, uint32_t* lw,
+                                              uint64_t validm, const Soft& so, uint32_t* lw,
                                               float (&col)[3], Trans& tot, int& n2, int& rec_chunks,
                                               int kbeg = 0, int kend = -1, int ent_off = 0) {
     const int T = a.T, lane = tg.lane;
@@ -1351,7 +1393,7 @@ __device__ __forceinline__ void forward_sweep(const RasterArgs& a, const float* 
                 uint64_t bandm;
                 Geo g;
                 const uint64_t onm =
-                    pair_weight<FAST>(r, eb, ent, tg.x, tg.y, tg.p, validm, w, cov, bandm, g, rsig, sig);
+                    pair_weight<FAST, false>(r, eb, ent, tg.x, tg.y, tg.p, validm, w, cov, bandm, g, so);
                 const bool on = __builtin_amdgcn_inverse_ballot_w64(onm);
                 // MODE_RECORD draws what a render draws but hands over what the
                 // taped forward keeps (F_TAPE); in the other modes the two agree.
@@ -1428,8 +1470,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(8)))
     const TileGeo tg = tile_geo(W, H, a.perm_fwd, a.B);
     const uint64_t validm = lane_mask(tg.valid);  // lanes whose pixel is in the image
     const int lane = tg.lane, wave = tg.wave, b = tg.b;
-    const float sig = fmaxf(a.sigma, 1e-8f);
-    const float rsig = a.rsig;
+    const Soft so = {fmaxf(a.sigma, 1e-8f), a.rsig, a.nl2};
     const float* __restrict__ rec = records + (size_t)b * T * REC;
 
     float col[3];
@@ -1438,7 +1479,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(8)))
     col[2] = a.bg[b * 3 + 2];
     Trans tot = {1.0f, 0, 0};
     int n2, rec_chunks;
-    forward_sweep<MODE, FAST, CKPT>(a, rec, tg, validm, rsig, sig, list[wave], col, tot, n2, rec_chunks);
+    forward_sweep<MODE, FAST, CKPT>(a, rec, tg, validm, so, list[wave], col, tot, n2, rec_chunks);
     const int cap2 = a.cap2;
 
     if (MODE == MODE_RENDER || MODE == MODE_RECORD || (MODE == MODE_LOSS && a.out_img)) {
@@ -1491,15 +1532,15 @@ struct Back {
 // The backward of one triangle at this lane's pixel (grad.rs:148-181) into the
 // lane's partial gradient `a`, zero where the lane does not contribute. The
 // chain is predicated rather than branched: in the backward every entry has
-// contributing lanes, so a branch would never skip. `any_band` (wave-uniform)
-// skips the vertex terms when no lane took the exact path.
+// contributing lanes, so a branch would never skip. The vertex terms are skipped
+// when no lane took the exact path (`bandm`: those that did).
 // PLAIN: no pixel of the wave met a zero factor or a rescaling in the forward
 // pass (its totals have z == e == 0). The prefixes of a pixel's product are at
 // least its total, so none of them needs either, and the transmittance is a
 // plain product: trans_mul and trans_suffix then give these same values.
 template <bool PLAIN>
-__device__ inline void grad_pixel(const Rec& r, bool on, bool band, bool any_band, float w, float cov,
-                                  const Geo& g, Pix p, float rsig, Back& st, float (&a)[NP]) {
+__device__ inline void grad_pixel(const Rec& r, bool on, uint64_t bandm, float w, float cov, const Geo& g, Pix p,
+                                  float rsig, Back& st, float (&a)[NP]) {
     const float omw = 1.0f - w;
     // d_canvas as the reference holds it at layer k: g0 prod_{j>k} (1 - w_j)
     float tk;
@@ -1522,33 +1563,36 @@ __device__ inline void grad_pixel(const Rec& r, bool on, bool band, bool any_ban
     const float d_w = tk * sw;
     a[9] = (r.i(R_FLAGS) & F_ACTIVE) ? d_w * cov : 0.0f;
     for (int j = 0; j < 6; j++) a[j] = 0.0f;
-    if (!any_band) return;
+    if (bandm == 0) return;
     const float d_cov = d_w * r.f(R_A);
     // grad.rs:252-268: vertex terms, zero exactly on the boundary.
     // Every lane evaluates them (no divergent branch: the wave runs this block
     // only for entries with band lanes, where the masked lanes would issue
-    // alike) and the lanes off the band or on the boundary take zeros.
-    const bool vt = band && g.dist >= 1e-9f;
+    // alike); the lanes off the band or on the boundary take zeros, through the
+    // two factors of every term (the chain may be no number there, and so may
+    // the reciprocal of a zero distance).
+    const bool vt = in_mask(bandm & lane_mask(g.dist >= 1e-9f));
     // u = (pt - cp) / dist with cp = a + t (b - a), rounded as
     // grad.rs:256-259 does: for a pixel within ~1e-7 of an edge the
     // direction is set by these roundings, and the reference's gradient
     // inherits them.
-    float inv = __builtin_amdgcn_rcpf(g.dist);
-    float cpx = g.ax + g.t * g.ex, cpy = g.ay + g.t * g.ey;
-    float ux = (p.px - cpx) * inv, uy = (p.py - cpy) * inv;
+    const float inv = vt ? __builtin_amdgcn_rcpf(g.dist) : 0.0f;
+    const float ux = (p.px - g.cpx) * inv, uy = (p.py - g.cpy) * inv;
     float chain = d_cov * cov * (1.0f - cov) * rsig;
-    chain = g.sd > 0.0f ? chain : -chain;
-    float A = -(1.0f - g.t) * chain;  // onto the edge's first vertex
-    float Bc = -g.t * chain;           // onto its second vertex
-    float s0 = g.edge == 0 ? A : (g.edge == 2 ? Bc : 0.0f);
-    float s1 = g.edge == 1 ? A : (g.edge == 0 ? Bc : 0.0f);
-    float s2 = g.edge == 2 ? A : (g.edge == 1 ? Bc : 0.0f);
-    a[0] = vt ? s0 * ux : 0.0f;
-    a[1] = vt ? s0 * uy : 0.0f;
-    a[2] = vt ? s1 * ux : 0.0f;
-    a[3] = vt ? s1 * uy : 0.0f;
-    a[4] = vt ? s2 * ux : 0.0f;
-    a[5] = vt ? s2 * uy : 0.0f;
+    chain = in_mask(g.inside) ? chain : -chain;  // inside is sd > 0 at the lanes that count: dist >= 1e-9
+    chain = vt ? chain : 0.0f;
+    const float A = -(1.0f - g.t) * chain;  // onto the edge's first vertex
+    const float Bc = -g.t * chain;           // onto its second vertex
+    const bool e1 = in_mask(g.e1), e2 = in_mask(g.e2);
+    const float s0 = e2 ? Bc : (e1 ? 0.0f : A);
+    const float s1 = e2 ? 0.0f : (e1 ? A : Bc);
+    const float s2 = e2 ? A : (e1 ? Bc : 0.0f);
+    a[0] = s0 * ux;
+    a[1] = s0 * uy;
+    a[2] = s1 * ux;
+    a[3] = s1 * uy;
+    a[4] = s2 * ux;
+    a[5] = s2 * uy;
 }
 
 // Wave sum of the lanes' partial gradients of one triangle, added to its row
@@ -1593,7 +1637,7 @@ __device__ inline void reduce_entry(const float (&a)[NP], lds_float* tw, lds_flo
 template <int MODE, bool FAST, bool REBUILD, bool DET>
 __device__ __forceinline__ void backward_sweep(const RasterArgs& a, const float* __restrict__ rec,
                                                const TileEnt* __restrict__ ents, const TileGeo& tg,
-                                               uint64_t validm, float rsig, float sig, Back& st, int i_begin,
+                                               uint64_t validm, const Soft& so, Back& st, int i_begin,
                                                int i_end, int rec_chunks, bool plain, uint32_t* lw, float* acc,
                                                float* trans) {
     constexpr int ROWS = DET ? WAVES : 1;  // accumulator row sets
@@ -1620,16 +1664,15 @@ __device__ __forceinline__ void backward_sweep(const RasterArgs& a, const float*
             if (k >= k1) break;
             nx = ent_at(te, min(i2 + 1, cap2 - 1));
             const bool on = __builtin_amdgcn_inverse_ballot_w64(cur.on);
-            const bool band = __builtin_amdgcn_inverse_ballot_w64(cur.band);
             Rec r;
             f8v eb;
             load_entry<FAST, true>(rec, rec_off((uint32_t)k), cur.k, r, eb);
             float cov;
             Geo g;
-            band_cov<FAST>(r, eb, tg.p, cur.k, cur.band, band, rsig, sig, g, cov);
+            band_cov<FAST, true>(r, eb, tg.p, cur.k, cur.band, so, g, cov);
             const float w = r.f(R_A) * cov;
             float part[NP];
-            grad_pixel<PLAIN>(r, on, band, cur.band != 0, w, cov, g, tg.p, rsig, st, part);
+            grad_pixel<PLAIN>(r, on, cur.band, w, cov, g, tg.p, so.rsig, st, part);
             // the recorded byte offset of the triangle's row (the product
             // (k - k0) * NP would become a 64-bit multiply-add on the vector unit)
             reduce_entry(part, tw, (lds_float*)((lds_char*)accw + cur.row), lane);
@@ -1675,14 +1718,12 @@ __device__ __forceinline__ void backward_sweep(const RasterArgs& a, const float*
                 uint64_t bandm;
                 Geo g;
                 const uint64_t onm =
-                    pair_weight<FAST>(r, eb, ent, tg.x, tg.y, tg.p, validm, w, cov, bandm, g, rsig, sig);
+                    pair_weight<FAST, true>(r, eb, ent, tg.x, tg.y, tg.p, validm, w, cov, bandm, g, so);
                 if (onm == 0) continue;
                 bandm &= onm;
-                const bool any_band = bandm != 0;
                 const bool on = __builtin_amdgcn_inverse_ballot_w64(onm);
-                const bool band = __builtin_amdgcn_inverse_ballot_w64(bandm);
                 float part[NP];
-                grad_pixel<false>(r, on, band, any_band, w, cov, g, tg.p, rsig, st, part);
+                grad_pixel<false>(r, on, bandm, w, cov, g, tg.p, so.rsig, st, part);
                 reduce_entry(part, tw, (lds_float*)accw + kl * NP, lane);
             }
         }
@@ -1786,8 +1827,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(REBU
                              : tile_geo(W, H, a.perm_bwd, a.B);
     const uint64_t validm = lane_mask(tg.valid);  // lanes whose pixel is in the image
     const int lane = tg.lane, wave = tg.wave, b = tg.b;
-    const float sig = fmaxf(a.sigma, 1e-8f);
-    const float rsig = a.rsig;
+    const Soft so = {fmaxf(a.sigma, 1e-8f), a.rsig, a.nl2};
     const float* __restrict__ rec = records + (size_t)b * T * REC;
 
     const int n2r = (int)uniform_u32((uint32_t)a.tl_n[2 * tg.tile]);
@@ -1832,7 +1872,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(REBU
         st.pre = {1.0f, 0, 0};
     }
     // no lane of the tile met a zero factor or a rescaling in the forward pass
-    backward_sweep<MODE, FAST, REBUILD, DET>(a, rec, ents, tg, validm, rsig, sig, st, i_begin, i_end, rec_chunks,
+    backward_sweep<MODE, FAST, REBUILD, DET>(a, rec, ents, tg, validm, so, st, i_begin, i_end, rec_chunks,
                                              !irregular, list[wave], &acc[0][0], &trans[0][0]);
     // The per-item loss (canvas.rs:45-58) from the forward kernel's per-block
     // sums, by the scene's first block, in a fixed order.
@@ -1872,8 +1912,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(DET 
     const TileGeo tg = tile_geo(W, H, a.perm_bwd, a.B);
     const uint64_t validm = lane_mask(tg.valid);  // lanes whose pixel is in the image
     const int lane = tg.lane, wave = tg.wave, b = tg.b;
-    const float sig = fmaxf(a.sigma, 1e-8f);
-    const float rsig = a.rsig;
+    const Soft so = {fmaxf(a.sigma, 1e-8f), a.rsig, a.nl2};
     const float* __restrict__ rec = records + (size_t)b * T * REC;
 
     Back st;
@@ -1881,7 +1920,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(DET 
     for (int ch = 0; ch < 3; ch++) col[ch] = st.col[ch] = a.bg[b * 3 + ch];
     Trans tot = {1.0f, 0, 0};
     int n2, rec_chunks;
-    forward_sweep<MODE, FAST, false>(a, rec, tg, validm, rsig, sig, list[wave], col, tot, n2, rec_chunks);
+    forward_sweep<MODE, FAST, false>(a, rec, tg, validm, so, list[wave], col, tot, n2, rec_chunks);
     if (MODE == MODE_LOSS && a.out_img && tg.valid)
         for (int ch = 0; ch < 3; ch++) a.out_img[img_index(a, tg.pix, b, ch)] = col[ch];
     for (int ch = 0; ch < 3; ch++) st.g0[ch] = 0.0f;
@@ -1918,7 +1957,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(DET 
     st.tot = tot;
     st.pre = {1.0f, 0, 0};
     const bool irregular = lane_mask(tot.z != 0 || tot.e != 0) != 0;
-    backward_sweep<MODE, FAST, false, DET>(a, rec, ents, tg, validm, rsig, sig, st, 0, n2, rec_chunks, !irregular,
+    backward_sweep<MODE, FAST, false, DET>(a, rec, ents, tg, validm, so, st, 0, n2, rec_chunks, !irregular,
                                            list[wave], acc, &trans[0][0]);
 }
 
@@ -2009,8 +2048,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void fu
     const TileGeo tg = tile_geo_wave(W, H, a.gx, a.gy, a.perm_bwd, a.B, a.perm_tiles != 0, a.tdiv_m);
     const uint64_t validm = lane_mask(tg.valid);  // lanes whose pixel is in the image
     const int lane = tg.lane, b = tg.b;
-    const float sig = fmaxf(a.sigma, 1e-8f);
-    const float rsig = a.rsig;
+    const Soft so = {fmaxf(a.sigma, 1e-8f), a.rsig, a.nl2};
     const float* __restrict__ rec = records + (size_t)b * T * REC;
 
     Back st;
@@ -2019,7 +2057,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void fu
     Trans tot = {1.0f, 0, 0};
     int n2, rec_chunks;
     // merged chunks: the sweep below reads each entry's triangle index
-    forward_sweep<MODE, FAST, false, true, ROWS>(a, rec, tg, validm, rsig, sig, list, col, tot, n2, rec_chunks);
+    forward_sweep<MODE, FAST, false, true, ROWS>(a, rec, tg, validm, so, list, col, tot, n2, rec_chunks);
     if (MODE == MODE_LOSS && a.out_img && tg.valid)
         for (int ch = 0; ch < 3; ch++) a.out_img[img_index(a, tg.pix, b, ch)] = col[ch];
     for (int ch = 0; ch < 3; ch++) st.g0[ch] = 0.0f;
@@ -2073,16 +2111,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void fu
             off += (uint32_t)sizeof(TileEnt);
             nx = *reinterpret_cast<const TileEnt*>(reinterpret_cast<const char*>(te) + off);
             const bool on = __builtin_amdgcn_inverse_ballot_w64(cur.on);
-            const bool band = __builtin_amdgcn_inverse_ballot_w64(cur.band);
             Rec r;
             f8v eb;
             load_entry<FAST, true>(rec, rec_off((uint32_t)k), cur.k, r, eb);
             float cov;
             Geo g;
-            band_cov<FAST>(r, eb, tg.p, cur.k, cur.band, band, rsig, sig, g, cov);
+            band_cov<FAST, true>(r, eb, tg.p, cur.k, cur.band, so, g, cov);
             const float w = r.f(R_A) * cov;
             float part[NP];
-            grad_pixel<PLAIN>(r, on, band, cur.band != 0, w, cov, g, tg.p, rsig, st, part);
+            grad_pixel<PLAIN>(r, on, cur.band, w, cov, g, tg.p, so.rsig, st, part);
             if (cur.band != 0)
                 reduce_entry_global(part, tw, grads + (size_t)k * NP, lane);
             else
@@ -2161,8 +2198,7 @@ __global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const f
     const TileGeo tg = tile_geo_wave(W, H, a.gx, a.gy, a.perm_bwd, a.B, a.perm_tiles != 0);
     const uint64_t validm = lane_mask(tg.valid);  // lanes whose pixel is in the image
     const int lane = tg.lane, b = tg.b;
-    const float sig = fmaxf(a.sigma, 1e-8f);
-    const float rsig = a.rsig;
+    const Soft so = {fmaxf(a.sigma, 1e-8f), a.rsig, a.nl2};
     const float* __restrict__ rec = records + (size_t)b * T * REC;
     const int k0 = (int)(((long long)s * T) / S), k1 = (int)(((long long)(s + 1) * T) / S);
     const int capS = a.cap2 / S;     // entry slots per segment in the tile's region
@@ -2192,7 +2228,7 @@ __global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const f
                 uint64_t bandm;
                 Geo g;
                 const uint64_t onm =
-                    pair_weight<FAST>(r, eb, ent, tg.x, tg.y, tg.p, validm, w, cov, bandm, g, rsig, sig);
+                    pair_weight<FAST, false>(r, eb, ent, tg.x, tg.y, tg.p, validm, w, cov, bandm, g, so);
                 if (onm == 0) continue;  // wave-uniform
                 SegEnt& e = sent[s * lcap + n2];
                 e.w[lane] = w;
@@ -2298,16 +2334,15 @@ __global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const f
             const int k = (int)(cur.k >> 8);
             nx = ent_at(tr, min(i2 + 1, capS - 1));
             const bool on = __builtin_amdgcn_inverse_ballot_w64(cur.on);
-            const bool band = __builtin_amdgcn_inverse_ballot_w64(cur.band);
             Rec r;
             f8v eb;
             load_entry<FAST, true>(rec, rec_off((uint32_t)k), cur.k, r, eb);
             float cov;
             Geo g;
-            band_cov<FAST>(r, eb, tg.p, cur.k, cur.band, band, rsig, sig, g, cov);
+            band_cov<FAST, true>(r, eb, tg.p, cur.k, cur.band, so, g, cov);
             const float w = r.f(R_A) * cov;
             float part[NP];
-            grad_pixel<PLAIN>(r, on, band, cur.band != 0, w, cov, g, tg.p, rsig, st, part);
+            grad_pixel<PLAIN>(r, on, cur.band, w, cov, g, tg.p, so.rsig, st, part);
             if (DET)
                 reduce_entry(part, tw, accs + (k - k0) * NP, lane);
             else if (cur.band != 0)
