@@ -1978,8 +1978,13 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(DET 
 // loads the slots with device-scope atomic loads, which see the tiles'
 // device-scope atomic stores from any XCD. The wait is bounded: a scene whose
 // slots are still pending after TAIL_SPIN polls gets a NaN loss.
-constexpr int TAIL_U = 4;           // blocks per lane held in registers (scenes of up to 256 blocks)
-constexpr int TAIL_SPIN = 1 << 22;  // polls, each at least one round trip to memory
+// The slots are taken 64 TAIL_U blocks at a time, all their loads in flight at
+// once, each chunk waited for before the next: when the last tile stores, the
+// earlier chunks are summed. Polling every slot of a large scene before summing
+// any (its loads one block after another) took ~13 us at 512x512 (B=1, T = 128
+// medium triangles: 36.1 -> 22.9 us per call).
+constexpr int TAIL_U = 4;           // blocks per lane and chunk (scenes of up to 256 blocks: one chunk)
+constexpr int TAIL_SPIN = 1 << 22;  // polls in all, each at least one round trip to memory
 __device__ inline double tail_load(const double* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1988,42 +1993,36 @@ __device__ inline bool tail_pending(double v) { return (uint64_t)__double_as_lon
 __device__ inline void loss_tail(const RasterArgs& a, int b) {
     const int lane = threadIdx.x & 63, nblk = a.gx * a.gy;
     const double* pl = a.partial_loss + (size_t)b * nblk * WAVES;
-    const bool held = nblk <= 64 * TAIL_U;
-    double v[TAIL_U][WAVES];
-    bool ok = false;
-    for (int spin = 0; spin < TAIL_SPIN; spin++) {
-        bool pending = false;
-        if (held) {
-            for (int u = 0; u < TAIL_U; u++) {
-                const int r = lane + 64 * u;
-                for (int q = 0; q < WAVES; q++) {
-                    v[u][q] = r < nblk ? tail_load(pl + (size_t)r * WAVES + q) : 0.0;
-                    pending = pending || (r < nblk && tail_pending(v[u][q]));
-                }
-            }
-        } else {
-            for (int r = lane; r < nblk; r += 64)
-                for (int q = 0; q < WAVES; q++)
-                    pending = pending || tail_pending(tail_load(pl + (size_t)r * WAVES + q));
-        }
-        if (lane_mask(pending) == 0) {
-            ok = true;
-            break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-    }
     double l = 0.0;
-    if (held) {
+    bool ok = true;
+    int spin = 0;
+    for (int r0 = lane; __builtin_amdgcn_readfirstlane(r0) < nblk && ok; r0 += 64 * TAIL_U) {
+        double v[TAIL_U][WAVES];
+        for (;;) {
+            bool pending = false;
+#pragma unroll
+            for (int u = 0; u < TAIL_U; u++) {
+                const int r = min(r0 + 64 * u, nblk - 1);  // past the end: the last block's, not added
+#pragma unroll
+                for (int q = 0; q < WAVES; q++) v[u][q] = tail_load(pl + (size_t)r * WAVES + q);
+            }
+#pragma unroll
+            for (int u = 0; u < TAIL_U; u++)
+#pragma unroll
+                for (int q = 0; q < WAVES; q++) pending = pending || tail_pending(v[u][q]);
+            if (lane_mask(pending) == 0) break;
+            if (++spin >= TAIL_SPIN) {
+                ok = false;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(2);
+        }
+#pragma unroll
         for (int u = 0; u < TAIL_U; u++) {
             double lb = v[u][0];
+#pragma unroll
             for (int q = 1; q < WAVES; q++) lb += v[u][q];
-            l = lane + 64 * u < nblk ? l + lb : l;
-        }
-    } else {
-        for (int r = lane; r < nblk; r += 64) {
-            double lb = tail_load(pl + (size_t)r * WAVES);
-            for (int q = 1; q < WAVES; q++) lb += tail_load(pl + (size_t)r * WAVES + q);
-            l += lb;
+            l = r0 + 64 * u < nblk ? l + lb : l;
         }
     }
     l = wave_sum_f64(l);

@@ -1,0 +1,34 @@
+"""The fused kernels' loss tail over scenes of more than one chunk of 256 blocks:
+its losses are the fixed-order mode's bits (both add the tiles' partials four to
+a block, then blocks lane, lane + 64, ... per lane, then the lanes)."""
+
+import numpy as np
+import pytest
+
+from diffrast import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from diffrast import _lib
+
+    c = _lib.Context()
+    yield c
+    c.close()
+
+
+# 256, 272, 512, 561 and 1071 blocks a scene
+@pytest.mark.parametrize("H,W", [(256, 256), (257, 250), (512, 248), (513, 260), (1000, 270)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("B", [1, 2])
+def test_tail_chunks(ctx, B, H, W):
+    T, sigma = 24, 0.004
+    params = synth.batch("random", B, T, 2200)
+    bgs = synth.uniforms(2207, B * 3).reshape(B, 3).astype(np.float32)
+    targets = np.stack([synth.blob_target(2200 + b, H, W) for b in range(B)])
+    print(f"tail chunks B={B} {H}x{W}", flush=True)
+    tail = ctx.fused_loss_backward(params, targets, sigma, bgs)[0]
+    fixed = ctx.fused_loss_backward(params, targets, sigma, bgs, deterministic=True)[0]
+    assert np.array_equal(tail, fixed)
