@@ -59,16 +59,9 @@ enum : int { SETUP_RENDER = 0, SETUP_TAPE = 1, SETUP_RECORD = 2 };
 // reclassifies its remaining chunks there.
 constexpr int CAP2_MIN = 128;
 
-// fused_seg_kernel: waves per tile, and the most triangles per scene (its LDS
-// holds a 288-byte record per triangle of the scene, 45 KB at 160). Eight
-// waves measured faster than four (B=1 64x64 T=32: 18.0 -> 15.3 us; the
-// 176x176 T=150 fit: 26.4 -> 23.4 us per iteration).
-constexpr int SEG_WAVES = 8;
-constexpr int SEG_MAX_T = 160;
-// Its entry region per tile: SEG_WAVES segments of whole 64-byte lines (8
-// entries) of more than T / SEG_WAVES entries each, so that cap2 > T, as the
-// fused paths require.
-__host__ __device__ constexpr int seg_cap2(int T) { return SEG_WAVES * (((T + SEG_WAVES - 1) / SEG_WAVES + 8) & ~7); }
+// fused_seg_kernel: the most triangles per scene (its LDS holds 20 bytes per
+// triangle, and the waves' lists while it makes the tile's).
+constexpr int SEG_MAX_T = 1024;
 // A loss slot not yet written (RasterArgs::loss_tail): a signalling NaN with
 // the lowest mantissa bit set. Arithmetic only returns quiet NaNs, and NaNs
 // that reach the loss from float inputs have their low 29 mantissa bits clear,
@@ -139,8 +132,8 @@ struct RasterArgs {
     int2* pze;             // ntiles*64 zero and rescaling counts (irregular tiles)
     TileEnt* tl_ent;       // ntiles*cap2 recorded entries
     int cap2;              // entries recorded per tile
-    // fused_seg_kernel's waves per tile (SEG_WAVES), or 0: the fused path
-    // takes the other kernels. cap2 is then SEG_WAVES x a multiple of 8, and
+    // fused_seg_kernel's waves per tile (2, 4 or 8), or 0: the fused path
+    // takes the other kernels. It records no entries (tl_ent is unused), and
     // with DRH_DETERMINISTIC the partial rows and loss partials are per tile.
     int segw;
     int* tl_n;             // ntiles*2: entries recorded, chunks fully recorded | TN_IRREGULAR

@@ -1751,8 +1751,10 @@ __device__ __forceinline__ void backward_sweep(const RasterArgs& a, const float*
 }
 
 // reduce_entry's wave sum, added by lane 4p straight into parameter p of the
-// triangle's gradient row `grow` in global memory (one float atomic each).
-__device__ inline void reduce_entry_global(const float (&a)[NP], lds_float* tw, float* grow, int lane) {
+// triangle's gradient row `grow` in global memory (one float atomic each), or
+// STORE: stored there.
+template <bool STORE>
+__device__ inline void reduce_entry_global_all(const float (&a)[NP], lds_float* tw, float* grow, int lane) {
     for (int q = 0; q < NP; q++) tw[q * TP + lane] = a[q];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -1766,19 +1768,24 @@ __device__ inline void reduce_entry_global(const float (&a)[NP], lds_float* tw, 
                 (((x2.x + x2.y) + (x2.z + x2.w)) + ((x3.x + x3.y) + (x3.z + x3.w)));
     sum += dpp<DPP_XOR1>(sum);
     sum += dpp<DPP_XOR2>(sum);
-    if (g == 0 && lane < 4 * NP && sum != 0.0f) unsafeAtomicAdd(grow + prm, sum);
+    if (STORE) {
+        if (g == 0 && lane < 4 * NP) grow[prm] = sum;
+    } else {
+        if (g == 0 && lane < 4 * NP && sum != 0.0f) unsafeAtomicAdd(grow + prm, sum);
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// reduce_entry_global for an entry with no band lane, whose vertex terms are
+// reduce_entry_global_all for an entry with no band lane, whose vertex terms are
 // all zero (grad_pixel): only parameters 6-9 are summed. Lane 16p + g sums
 // pixels 4g..4g+3 of parameter 6 + p (one 16-byte read, three adds), the row
 // of sixteen partials is combined across its lanes (two quad steps, the
 // half-row and the row mirror) and lane 16p adds the total. About half of the
 // entries of B=16 256x256 T=128 have no band lane: -1.0 us of ~88.
 constexpr int DPP_ROW_MIRROR = 0x140, DPP_ROW_HALF_MIRROR = 0x141;
+template <bool STORE>
 __device__ inline void reduce_entry_global_cw(const float (&a)[NP], lds_float* tw, float* grow, int lane) {
     for (int q = 0; q < 4; q++) tw[q * TP + lane] = a[6 + q];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1793,10 +1800,23 @@ __device__ inline void reduce_entry_global_cw(const float (&a)[NP], lds_float* t
     sum += dpp<DPP_XOR2>(sum);
     sum += dpp<DPP_ROW_HALF_MIRROR>(sum);
     sum += dpp<DPP_ROW_MIRROR>(sum);
-    if (g == 0 && sum != 0.0f) unsafeAtomicAdd(grow + 6 + prm, sum);
+    if (STORE) {
+        if (g == 0) grow[6 + prm] = sum;
+    } else {
+        if (g == 0 && sum != 0.0f) unsafeAtomicAdd(grow + 6 + prm, sum);
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// An entry's wave sums into its gradient row. `band`: it has band lanes.
+template <bool STORE>
+__device__ inline void reduce_entry_global(const float (&a)[NP], lds_float* tw, float* grow, int lane, bool band) {
+    if (band)
+        reduce_entry_global_all<STORE>(a, tw, grow, lane);
+    else
+        reduce_entry_global_cw<STORE>(a, tw, grow, lane);
 }
 
 // Backward: the reverse-mode sweep (grad.rs:135-182) over the entries the
@@ -2119,10 +2139,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void fu
             const float w = r.f(R_A) * cov;
             float part[NP];
             grad_pixel<PLAIN>(r, on, cur.band, w, cov, g, tg.p, so.rsig, st, part);
-            if (cur.band != 0)
-                reduce_entry_global(part, tw, grads + (size_t)k * NP, lane);
-            else
-                reduce_entry_global_cw(part, tw, grads + (size_t)k * NP, lane);
+            reduce_entry_global<false>(part, tw, grads + (size_t)k * NP, lane, cur.band != 0);
         }
     };
     if (plain)
@@ -2131,237 +2148,278 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void fu
         sweep(std::false_type{});
 }
 
-// Grids of few tiles (a single scene of a few hundred 8x8 tiles, the fit):
-// one tile per workgroup of S waves. Where the one-wave kernel runs about one
-// wave per SIMD and is bound by the chain of dependent waits per entry of its
-// tile (scalar record loads, LDS round trips), this one splits the tile's
-// triangles over the waves, wave s taking [s T / S, (s + 1) T / S):
-//  A. each wave lists its triangles and evaluates their weights at the tile's
-//     pixels (pair_weight: the exact path, the classification), records its
-//     entries for the backward, and leaves each entry's weights, colour and
-//     contributing lanes in LDS;
-//  B. every wave composites all the tile's entries from LDS in scene order
-//     (raster.rs:37-68), exactly as the one-wave kernel's forward sweep does,
-//     so the image, the transmittance and the loss are the same bits; a wave
-//     keeps the canvas and the transmittance at the start of its segment;
-//  C. each wave sweeps its own entries backward from that state, as the
-//     one-wave kernel sweeps all of them.
-// The tile's entry region (cap2 = S x capS entries) holds segment s's entries
-// at s capS. DET: each wave sums its entries' gradients into LDS rows of its
-// segment's triangles and the tile writes its partial rows (B x tiles x T x
-// NP) for reduce_partials / fit_step; otherwise each entry's wave sum goes to
-// the gradients as float atomics. The loss partial is per tile either way,
-// summed four to a 16x16 block first, as sum_losses sums the one-wave
-// kernel's.
+// Grids of few tiles: one tile per workgroup of S waves. Where the one-wave
+// kernel runs a few waves per SIMD it is bound by the chain of dependent waits
+// per entry of its tile (scalar record loads, LDS round trips, the latency of
+// its own instructions), and by its heaviest tiles; this one splits a tile's
+// entries over the waves:
+//  L. each wave lists the triangles of its share of [0, T) that can touch the
+//     tile (build_list); the lists go one after another into the tile's list of
+//     N entries, in scene order;
+//  A. the waves evaluate the entries' weights at the tile's pixels
+//     (pair_weight: the exact path, the classification), a block of entries at
+//     a time, shared evenly; weights, contributing lanes and band lanes go to
+//     LDS;
+//  B. wave 0 composites the block's entries in scene order (raster.rs:37-68),
+//     exactly as the one-wave kernel's forward sweep does, so the image, the
+//     transmittance and the loss are the same bits, while the other waves
+//     evaluate the next block (two block buffers); at entry s N / S it leaves the
+//     canvas and the transmittance for wave s, and at the end dL/dpixel and the
+//     totals;
+//  C. each wave sweeps its S-th of the N entries backward from that state, as
+//     the one-wave kernel sweeps all of them.
+// A wave's entries (list word, contributing and band lanes) are held one per
+// lane and read with v_readlane: no entry goes through memory. DET: a (tile,
+// triangle) pair is one wave's, which stores its sum in the tile's partial rows
+// (B x tiles x T x NP, cleared at the start) for reduce_partials / fit_step;
+// otherwise each entry's wave sum goes to the gradients as float atomics. The
+// loss partial is per tile either way, summed four to a 16x16 block first, as
+// sum_losses sums the one-wave kernel's.
 //
-// Dynamic LDS: phases A and B hold SEG_WAVES x seg_tris(T) SegEnt records;
-// phase C reuses the same area for the waves' transposition areas (and DET
-// accumulator rows).
-struct SegEnt {
-    float w[64];       // weight at each lane's pixel
-    float c[3];        // colour
-    uint32_t on[2];    // lanes it contributes at (low, high word)
-    uint32_t pad[3];
-};
-static_assert(sizeof(SegEnt) == 288 && sizeof(SegEnt) % 16 == 0, "SegEnt keeps 16-byte alignment");
-
-// Triangles per segment (at most), the pitch of the segments' SegEnt records
-// in LDS; phase C's LDS bytes; and the workgroup's dynamic LDS.
-__host__ __device__ constexpr int seg_tris(int T) { return (T + SEG_WAVES - 1) / SEG_WAVES; }
-__host__ __device__ constexpr size_t seg_lds_c(bool det, int T) {
-    return (size_t)SEG_WAVES * NP * TP * sizeof(float) +
-           (det ? (size_t)SEG_WAVES * seg_tris(T) * NP * sizeof(float) : 0);
+// LDS (dynamic, seg_lds_bytes): the entries' words and lanes (20 bytes each, at
+// most T) and one area that holds the waves' lists, then the block buffers, the
+// S handed-over states and the totals, then phase C's transposition areas. Small
+// blocks keep it small (S = 2: 8.7 KB and 20 bytes a triangle): a grid of 4096
+// tiles of two waves is one round of a device with 24 of them on a CU.
+//
+// An earlier form gave each of eight waves an eighth of the triangles for all
+// three phases, with every wave compositing all entries: its LDS held every
+// triangle's weights (288 bytes, so at most 160 triangles), the waves' entries
+// were uneven, and the lists cost eight passes. B=1 256x256 T=128 large
+// triangles 34.8 -> 27.9 us; T=512, with the one-wave kernel before,
+// 171 -> 67; B=16 64x64 T=512 medium triangles sigma 0.01 129 -> 73; B=16
+// 128x128 T=128, with the two-kernel split before, 63.6 -> 48.3; 96 fit
+// iterations at 132x176 T=150 2862 -> 2680.
+__host__ __device__ constexpr int seg_block(int S) { return 4 * S; }  // entries per block buffer (one block of both for up to twice as many)
+constexpr int SEG_STATE = 6 * 64;
+__host__ __device__ constexpr int seg_tpad(int T) { return (T + 3) & ~3; }
+__host__ __device__ constexpr size_t seg_area_floats(int S) {
+    const size_t n = (size_t)2 * seg_block(S) * 64 + (size_t)(S + 1) * SEG_STATE;
+    return n > (size_t)S * NP * TP ? n : (size_t)S * NP * TP;
 }
-__host__ __device__ constexpr size_t seg_lds_bytes(bool det, int T) {
-    return (size_t)SEG_WAVES * seg_tris(T) * sizeof(SegEnt) > seg_lds_c(det, T)
-               ? (size_t)SEG_WAVES * seg_tris(T) * sizeof(SegEnt)
-               : seg_lds_c(det, T);
+__host__ __device__ constexpr size_t seg_lds_bytes(int S, int T) {
+    return (size_t)seg_tpad(T) * 20 + seg_area_floats(S) * sizeof(float);
 }
 
+__device__ inline uint32_t read_lane(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
+__device__ inline uint64_t read_lane64(uint32_t lo, uint32_t hi, int lane) {
+    return (uint64_t)read_lane(hi, lane) << 32 | read_lane(lo, lane);
+}
 template <int MODE, bool FAST, bool DET, int S>
-__global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const float* __restrict__ records,
-                                                          const TileEnt* __restrict__ ents) {
+__global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const float* __restrict__ records) {
     static_assert(MODE == MODE_LOSS || MODE == MODE_GRAD_IN, "gradient modes only");
-    static_assert(S == SEG_WAVES, "seg_lds_bytes sizes the LDS for SEG_WAVES waves");
-    __shared__ uint32_t list[S][CH];
-    __shared__ int nent[S];
+    static_assert(SEG_MAX_T + 64 * S <= (int)seg_area_floats(S), "the waves' lists fit the area");
+    constexpr int SEG_BLOCK = seg_block(S);
+    static_assert(2 * SEG_BLOCK <= 64, "a block's entries are held one per lane");
+    __shared__ int count[S];
     extern __shared__ __attribute__((aligned(16))) float seg_lds[];
-    SegEnt* const sent = reinterpret_cast<SegEnt*>(seg_lds);
     if (a.halt && *a.halt >= 0) return;
     if (MODE == MODE_LOSS && !DET && a.loss_tail && (int)blockIdx.x >= (int)gridDim.x - a.B) {
         if (threadIdx.x < 64) loss_tail(a, (int)blockIdx.x - ((int)gridDim.x - a.B));
         return;
     }
-    const int W = a.W, H = a.H, T = a.T;
-    const int s = (int)uniform_u32(threadIdx.x >> 6);  // this wave's segment
+    const int W = a.W, H = a.H, T = a.T, tpad = seg_tpad(T);
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    u4v* const lanes = reinterpret_cast<u4v*>(seg_lds);             // tpad: contributing lanes, band lanes
+    uint32_t* const codes = reinterpret_cast<uint32_t*>(lanes + tpad);  // tpad: (k << 8) | kind, plan
+    float* const area = reinterpret_cast<float*>(codes + tpad);     // see above
+    float* const fin = area + (seg_area_floats(S) - SEG_STATE);     // 6 x 64
+    float* const state = fin - S * SEG_STATE;                       // S x 6 x 64
+    const int s = (int)uniform_u32(threadIdx.x >> 6);  // this wave
     const TileGeo tg = tile_geo_wave(W, H, a.gx, a.gy, a.perm_bwd, a.B, a.perm_tiles != 0);
     const uint64_t validm = lane_mask(tg.valid);  // lanes whose pixel is in the image
     const int lane = tg.lane, b = tg.b;
     const Soft so = {fmaxf(a.sigma, 1e-8f), a.rsig, a.nl2};
     const float* __restrict__ rec = records + (size_t)b * T * REC;
-    const int k0 = (int)(((long long)s * T) / S), k1 = (int)(((long long)(s + 1) * T) / S);
-    const int capS = a.cap2 / S;     // entry slots per segment in the tile's region
-    const int lcap = seg_tris(T);    // SegEnt slots per segment in LDS (>= k1 - k0)
-    // wave-uniform: the entry stores and loads address from a scalar base
-    TileEnt* const te = a.tl_ent + (size_t)uniform_u32((uint32_t)tg.tile) * a.cap2 + s * capS;
+    if (DET) {
+        // rows of triangles that do not touch the tile stay zero
+        float* prow = a.partials + (size_t)tg.tile * T * NP;
+        for (int j = threadIdx.x; j < T * NP; j += S * 64) prow[j] = 0.0f;
+    }
+    // wave 0 takes the pixels' targets (or the incoming gradients) on the way
+    float in[3] = {0.0f, 0.0f, 0.0f};
+    if (s == 0 && tg.valid)
+        for (int ch = 0; ch < 3; ch++) in[ch] = (MODE == MODE_LOSS ? a.target : a.grad_in)[img_index(a, tg.pix, b, ch)];
 
-    // A. the segment's entries and their weights
-    int n2 = 0;
-    for (int kb = k0; kb < k1;) {
-        int kend;
-        const int count = tg.live ? build_list<true>(rec, kb, k1, tg.tx0, tg.ty0, tg.tx1, tg.ty1, tg.cx0, tg.cy0,
-                                                     tg.cx1, tg.cy1, list[s], lane, F_LIVE, &kend)
-                                  : 0;
-        kb = tg.live ? kend : k1;
-        // the list one half at a time, one entry per lane (as forward_sweep)
-        for (int h = 0; h < count; h += 64) {
-            const uint32_t held = list[s][min(h + lane, CH - 1)];
-            const int nh = (int)uniform_u32((uint32_t)min(count - h, 64));
-            for (int i = 0; i < nh; i++) {
-                const uint32_t ent = (uint32_t)__builtin_amdgcn_readlane((int)held, i);
-                const int k = (int)(ent >> 8);  // merged lists hold the triangle index
+    // L. the tile's list. Shares of whole passes of 64 triangles (a pass costs a
+    // wave the same with fewer): with few triangles the last waves list none.
+    const int share = 64 * ((T + 64 * S - 1) / (64 * S));
+    {
+        uint32_t* const own = reinterpret_cast<uint32_t*>(area) + s * share;
+        const int k1 = min(T, (s + 1) * share);
+        int n = 0;
+        for (int k = s * share; tg.live && k < k1;) {
+            int kend;
+            n += build_list<true>(rec, k, k1, tg.tx0, tg.ty0, tg.tx1, tg.ty1, tg.cx0, tg.cy0, tg.cx1, tg.cy1, own + n,
+                                  lane, F_LIVE, &kend);
+            k = kend;
+        }
+        if (lane == 0) count[s] = n;
+    }
+    __syncthreads();
+    int N = 0, first = 0;  // entries of the tile, and before this wave's
+    for (int q = 0; q < S; q++) {
+        first = q == s ? N : first;
+        N += (int)uniform_u32((uint32_t)count[q]);
+    }
+    first = (int)uniform_u32((uint32_t)first);
+    {
+        const uint32_t* const own = reinterpret_cast<const uint32_t*>(area) + s * share;
+        const int n = (int)uniform_u32((uint32_t)count[s]);
+        for (int i = lane; i < n; i += 64) codes[first + i] = own[i];
+    }
+    __syncthreads();
+
+    // A and B, a block of entries at a time
+    const int step = N <= 2 * SEG_BLOCK ? 2 * SEG_BLOCK : SEG_BLOCK;
+    float col[3];
+    for (int ch = 0; ch < 3; ch++) col[ch] = a.bg[b * 3 + ch];
+    Trans tot = {1.0f, 0, 0};
+    int q = 0, at = 0;  // wave 0: the next state to leave, and the entry it is due before
+    for (int b0 = 0, buf = 0; b0 < N; b0 += step, buf ^= SEG_BLOCK) {
+        const int n = min(step, N - b0);
+        float* const wb = area + buf * 64;
+        {
+            // this wave's entries [i0, i1) of the block
+            const int i0 = b0 + (n * s) / S, m = b0 + (n * (s + 1)) / S - i0;
+            const uint32_t held = codes[min(i0 + lane, N - 1)];
+            for (int i = 0; i < m; i++) {
+                const uint32_t ent = read_lane(held, i);
                 Rec r;
                 f8v eb;
-                load_entry<FAST, true>(rec, rec_off((uint32_t)k), ent, r, eb);
+                load_entry<FAST, true>(rec, rec_off(ent >> 8), ent, r, eb);
                 float w = 0.0f, cov;
                 uint64_t bandm;
                 Geo g;
                 const uint64_t onm =
                     pair_weight<FAST, false>(r, eb, ent, tg.x, tg.y, tg.p, validm, w, cov, bandm, g, so);
-                if (onm == 0) continue;  // wave-uniform
-                SegEnt& e = sent[s * lcap + n2];
-                e.w[lane] = w;
-                if (lane == 0) {
-                    e.c[0] = r.f(R_C);
-                    e.c[1] = r.f(R_C + 1);
-                    e.c[2] = r.f(R_C + 2);
-                    e.on[0] = (uint32_t)onm;
-                    e.on[1] = (uint32_t)(onm >> 32);
-                    TileEnt t;
-                    t.k = ent;
-                    t.row = 0;
-                    t.on = onm;
-                    t.band = onm & bandm;
-                    te[n2] = t;
+                bandm &= onm;
+                wb[(i0 - b0 + i) * 64 + lane] = w;
+                if (lane == 0)
+                    lanes[i0 + i] = u4v{(uint32_t)onm, (uint32_t)(onm >> 32), (uint32_t)bandm, (uint32_t)(bandm >> 32)};
+            }
+        }
+        __syncthreads();
+        if (s == 0) {
+            const int ie = b0 + min(lane, n - 1);
+            const float* const c = rec_at(rec, rec_off(codes[ie] >> 8)) + R_C;
+            const uint32_t c0 = __float_as_uint(c[0]), c1 = __float_as_uint(c[1]), c2 = __float_as_uint(c[2]);
+            const u4v on4 = lanes[ie];
+            float w = wb[lane];
+            for (int i = 0; i < n; i++) {
+                while (q < S && at == b0 + i) {  // the state before entry q N / S
+                    float* const st = state + q * SEG_STATE + lane;
+                    st[0] = col[0];
+                    st[64] = col[1];
+                    st[128] = col[2];
+                    st[192] = tot.q;
+                    st[256] = __int_as_float(tot.z);
+                    st[320] = __int_as_float(tot.e);
+                    q++;
+                    at = (int)(((long long)q * N) / S);
                 }
-                n2++;
+                const bool on = in_mask(read_lane64(on4.x, on4.y, i));
+                const float cc[3] = {__uint_as_float(read_lane(c0, i)), __uint_as_float(read_lane(c1, i)),
+                                     __uint_as_float(read_lane(c2, i))};
+                const float wn = wb[min(i + 1, n - 1) * 64 + lane];  // the next entry's, on the way
+                // forward_sweep's arithmetic
+                const float omw = 1.0f - w;
+                for (int ch = 0; ch < 3; ch++) {
+                    const float o = fmaf(w, cc[ch] - col[ch], col[ch]);
+                    col[ch] = on ? o : col[ch];
+                }
+                const float f = on ? omw : 1.0f;
+                const float qn = tot.q * f;
+                if (lane_mask(!(qn >= 5.421010862427522e-20f)) == 0)
+                    tot.q = qn;
+                else
+                    trans_mul(tot, f);
+                w = wn;
             }
         }
     }
-    if (lane == 0) nent[s] = n2;
-    // The entries were recorded with vector stores and are read back below with
-    // scalar loads: the stores are complete (in L2, which the scalar cache reads
-    // from) before any of those loads issue (the regions are whole cache lines).
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-
-    // B. the tile's composite in scene order, forward_sweep's arithmetic
     Back st;
-    float col[3];
-    Trans tot = {1.0f, 0, 0};
-    for (int ch = 0; ch < 3; ch++) col[ch] = a.bg[b * 3 + ch];
-    for (int q = 0; q < S; q++) {
-        if (q == s) {
-            for (int ch = 0; ch < 3; ch++) st.col[ch] = col[ch];
-            st.pre = tot;
-        }
-        const int n = nent[q];
-        for (int i = 0; i < n; i++) {
-            const SegEnt& e = sent[q * lcap + i];
-            const float w = e.w[lane];
-            const bool on = ((lane < 32 ? e.on[0] >> lane : e.on[1] >> (lane - 32)) & 1u) != 0;
-            const float omw = 1.0f - w;
-            for (int ch = 0; ch < 3; ch++) {
-                const float o = fmaf(w, e.c[ch] - col[ch], col[ch]);
-                col[ch] = on ? o : col[ch];
+    if (s == 0) {
+        float g0[3] = {0.0f, 0.0f, 0.0f};
+        double l = 0.0;
+        if (tg.valid) {
+            if (MODE == MODE_LOSS) {
+                if (a.out_img)
+                    for (int ch = 0; ch < 3; ch++) a.out_img[img_index(a, tg.pix, b, ch)] = col[ch];
+                // the loss (canvas.rs:45-58) and dL/dpixel (grad.rs:111-114) as forward_kernel forms them
+                const float scale = a.lscale;
+                for (int ch = 0; ch < 3; ch++) {
+                    const float d = col[ch] - in[ch];
+                    l += (double)d * (double)d;
+                    g0[ch] = scale * (col[ch] - in[ch]);
+                }
+            } else {
+                for (int ch = 0; ch < 3; ch++) g0[ch] = in[ch];
             }
-            const float f = on ? omw : 1.0f;
-            const float qn = tot.q * f;
-            if (lane_mask(!(qn >= 5.421010862427522e-20f)) == 0)
-                tot.q = qn;
-            else
-                trans_mul(tot, f);
         }
-    }
-    st.tot = tot;
-    if (MODE == MODE_LOSS && a.out_img && tg.valid && s == 0)
-        for (int ch = 0; ch < 3; ch++) a.out_img[img_index(a, tg.pix, b, ch)] = col[ch];
-    for (int ch = 0; ch < 3; ch++) st.g0[ch] = 0.0f;
-    double l = 0.0;
-    if (tg.valid) {
+        float* const f = fin + lane;
+        f[0] = g0[0];
+        f[64] = g0[1];
+        f[128] = g0[2];
+        f[192] = tot.q;
+        f[256] = __int_as_float(tot.z);
+        f[320] = __int_as_float(tot.e);
         if (MODE == MODE_LOSS) {
-            // the loss (canvas.rs:45-58) and dL/dpixel (grad.rs:111-114) as forward_kernel forms them
-            const float scale = a.lscale;
-            for (int ch = 0; ch < 3; ch++) {
-                float t = a.target[img_index(a, tg.pix, b, ch)];
-                float d = col[ch] - t;
-                l += (double)d * (double)d;
-                st.g0[ch] = scale * (col[ch] - t);
+            l = wave_sum_f64(l);
+            if (lane == 0) {
+                if (!DET && a.loss_tail)
+                    __hip_atomic_store(&a.partial_loss[tg.tile], l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else
+                    a.partial_loss[tg.tile] = l;
             }
-        } else {
-            for (int ch = 0; ch < 3; ch++) st.g0[ch] = a.grad_in[img_index(a, tg.pix, b, ch)];
         }
     }
-    if (MODE == MODE_LOSS && s == 0) {
-        l = wave_sum_f64(l);
-        if (lane == 0) {
-            if (!DET && a.loss_tail)
-                __hip_atomic_store(&a.partial_loss[tg.tile], l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            else
-                a.partial_loss[tg.tile] = l;
-        }
+    // the cleared partial rows are in place before any wave's sums go over them
+    if (DET) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // phase C reuses the block buffers
+    {
+        const float* const f = fin + lane;
+        for (int ch = 0; ch < 3; ch++) st.g0[ch] = f[64 * ch];
+        st.tot = {f[192], __float_as_int(f[256]), __float_as_int(f[320])};
+        const float* const c = state + s * SEG_STATE + lane;
+        for (int ch = 0; ch < 3; ch++) st.col[ch] = c[64 * ch];
+        st.pre = {c[192], __float_as_int(c[256]), __float_as_int(c[320])};
     }
-    const bool plain = lane_mask(tot.z != 0 || tot.e != 0) == 0;  // the same in every wave
-    __syncthreads();  // phase C reuses the SegEnt area
+    __syncthreads();  // the transposition areas go over the states
+    const bool plain = lane_mask(st.tot.z != 0 || st.tot.e != 0) == 0;  // the same in every wave
 
-    // C. this segment's entries backward
-    lds_float* const tw = (lds_float*)(seg_lds + s * (NP * TP));
-    lds_float* const accs = (lds_float*)(seg_lds + S * (NP * TP) + s * (lcap * NP));
-    if (DET) {
-        for (int j = lane; j < lcap * NP; j += 64) accs[j] = 0.0f;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    }
-    const TileEnt* __restrict__ tr = te;
-    float* const grads = DET ? nullptr : a.grads + (size_t)b * T * NP;
+    // C. this wave's entries backward
+    lds_float* const tw = (lds_float*)(area + s * (NP * TP));
+    float* const grads = DET ? a.partials + (size_t)tg.tile * T * NP : a.grads + (size_t)b * T * NP;
+    const int e0 = (int)(((long long)s * N) / S), e1 = (int)(((long long)(s + 1) * N) / S);
     auto sweep = [&](auto plain_c) {
         constexpr bool PLAIN = decltype(plain_c)::value;
-        TileEnt nx = tr[0];
-        for (int i2 = 0; i2 < n2; i2++) {
-            const TileEnt cur = nx;
-            const int k = (int)(cur.k >> 8);
-            nx = ent_at(tr, min(i2 + 1, capS - 1));
-            const bool on = __builtin_amdgcn_inverse_ballot_w64(cur.on);
-            Rec r;
-            f8v eb;
-            load_entry<FAST, true>(rec, rec_off((uint32_t)k), cur.k, r, eb);
-            float cov;
-            Geo g;
-            band_cov<FAST, true>(r, eb, tg.p, cur.k, cur.band, so, g, cov);
-            const float w = r.f(R_A) * cov;
-            float part[NP];
-            grad_pixel<PLAIN>(r, on, cur.band, w, cov, g, tg.p, so.rsig, st, part);
-            if (DET)
-                reduce_entry(part, tw, accs + (k - k0) * NP, lane);
-            else if (cur.band != 0)
-                reduce_entry_global(part, tw, grads + (size_t)k * NP, lane);
-            else
-                reduce_entry_global_cw(part, tw, grads + (size_t)k * NP, lane);
+        for (int h = e0; h < e1; h += 64) {
+            const int ie = min(h + lane, e1 - 1), nh = min(e1 - h, 64);
+            const uint32_t held = codes[ie];
+            const u4v lm = lanes[ie];
+            for (int i = 0; i < nh; i++) {
+                const uint64_t onm = read_lane64(lm.x, lm.y, i);
+                if (onm == 0) continue;  // wave-uniform
+                const uint64_t bandm = read_lane64(lm.z, lm.w, i);
+                const uint32_t ent = read_lane(held, i), k = ent >> 8;
+                Rec r;
+                f8v eb;
+                load_entry<FAST, true>(rec, rec_off(k), ent, r, eb);
+                float cov;
+                Geo g;
+                band_cov<FAST, true>(r, eb, tg.p, ent, bandm, so, g, cov);
+                const float w = r.f(R_A) * cov;
+                float part[NP];
+                grad_pixel<PLAIN>(r, in_mask(onm), bandm, w, cov, g, tg.p, so.rsig, st, part);
+                reduce_entry_global<DET>(part, tw, grads + (size_t)k * NP, lane, bandm != 0);
+            }
         }
     };
     if (plain)
         sweep(std::true_type{});
     else
         sweep(std::false_type{});
-    if (DET) {
-        // the tile's partial rows of this segment's triangles
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        float* prow = a.partials + ((size_t)tg.tile * T + k0) * NP;
-        for (int j = lane; j < (k1 - k0) * NP; j += 64) prow[j] = accs[j];
-    }
 }
 
 // Lane `lane`'s share of a scene's block loss sums: blocks lane, lane + 64, ...
@@ -2757,22 +2815,35 @@ static void launch_fused_d(bool fast, const RasterArgs& a, dim3 grid, hipStream_
         launch_k((fused_kernel<MODE, false, DET>), grid, dim3(WAVES * 64), 0, s, a, a.rec, a.tl_ent);
 }
 
+template <int MODE, int S>
+static void launch_seg_s(bool fast, const RasterArgs& a, dim3 grid, hipStream_t s) {
+    // with the loss tail (not in the fixed-order mode), B more workgroups after the tiles
+    const dim3 tiles(grid.x * grid.y * grid.z * WAVES +
+                     (MODE == MODE_LOSS && !a.deterministic && a.loss_tail ? a.B : 0)),
+        threads(S * 64);
+    const size_t lds = seg_lds_bytes(S, a.T);
+    if (a.deterministic && fast)
+        launch_k((fused_seg_kernel<MODE, true, true, S>), tiles, threads, lds, s, a, a.rec);
+    else if (a.deterministic)
+        launch_k((fused_seg_kernel<MODE, false, true, S>), tiles, threads, lds, s, a, a.rec);
+    else if (fast)
+        launch_k((fused_seg_kernel<MODE, true, false, S>), tiles, threads, lds, s, a, a.rec);
+    else
+        launch_k((fused_seg_kernel<MODE, false, false, S>), tiles, threads, lds, s, a, a.rec);
+}
+
 template <int MODE>
 static void launch_fused_m(bool fast, const RasterArgs& a, dim3 grid, hipStream_t s) {
-    if (a.segw) {
-        // with the loss tail (not in the fixed-order mode), B more workgroups after the tiles
-        const dim3 tiles(grid.x * grid.y * grid.z * WAVES +
-                         (MODE == MODE_LOSS && !a.deterministic && a.loss_tail ? a.B : 0)),
-            threads(SEG_WAVES * 64);
-        const size_t lds = seg_lds_bytes(a.deterministic != 0, a.T);
-        if (a.deterministic && fast)
-            launch_k((fused_seg_kernel<MODE, true, true, SEG_WAVES>), tiles, threads, lds, s, a, a.rec, a.tl_ent);
-        else if (a.deterministic)
-            launch_k((fused_seg_kernel<MODE, false, true, SEG_WAVES>), tiles, threads, lds, s, a, a.rec, a.tl_ent);
-        else if (fast)
-            launch_k((fused_seg_kernel<MODE, true, false, SEG_WAVES>), tiles, threads, lds, s, a, a.rec, a.tl_ent);
-        else
-            launch_k((fused_seg_kernel<MODE, false, false, SEG_WAVES>), tiles, threads, lds, s, a, a.rec, a.tl_ent);
+    if (a.segw == 8) {
+        launch_seg_s<MODE, 8>(fast, a, grid, s);
+        return;
+    }
+    if (a.segw == 4) {
+        launch_seg_s<MODE, 4>(fast, a, grid, s);
+        return;
+    }
+    if (a.segw == 2) {
+        launch_seg_s<MODE, 2>(fast, a, grid, s);
         return;
     }
     if (a.deterministic) {
@@ -2801,10 +2872,9 @@ static void launch_fused_m(bool fast, const RasterArgs& a, dim3 grid, hipStream_
 
 hipError_t launch_fused(int mode, bool fast, const RasterArgs& a, hipStream_t s) {
     if ((size_t)a.B * a.H * a.W == 0) return hipSuccess;
-    if ((mode != MODE_LOSS && mode != MODE_GRAD_IN) || a.cap2 < a.T || a.cap2 % 8 != 0 || a.nseg > 1)
-        return hipErrorInvalidValue;
-    if (a.segw && (a.segw != SEG_WAVES || a.T > SEG_MAX_T || a.cap2 % (8 * SEG_WAVES) != 0 ||
-                   a.cap2 / SEG_WAVES < (a.T + SEG_WAVES - 1) / SEG_WAVES))
+    if ((mode != MODE_LOSS && mode != MODE_GRAD_IN) || a.nseg > 1) return hipErrorInvalidValue;
+    // fused_seg_kernel keeps its entries in LDS; the others record them in regions of cap2
+    if (a.segw ? (a.segw != 2 && a.segw != 4 && a.segw != 8) || a.T > SEG_MAX_T : a.cap2 < a.T || a.cap2 % 8 != 0)
         return hipErrorInvalidValue;
     const dim3 grid = raster_grid(a.B, a.W, a.H);
     if (mode == MODE_LOSS)

@@ -226,12 +226,12 @@ bool use_order(const drh_ctx* ctx, int B, int gx, int gy);
 // Device buffers of one raster call besides its inputs and outputs.
 struct RasterBufs {
     float* rec = nullptr;           // B*T*REC
-    float* partials = nullptr;      // B*nblk*T*NP (deterministic gradient modes)
+    float* partials = nullptr;      // B*nblk*T*NP (deterministic gradient modes; per tile with segw)
     double* ploss = nullptr;        // B*nblk (gradient modes)
     float* pq = nullptr;            // B*H*W (gradient modes)
     float* pg0 = nullptr;           // B*H*W*3 (MODE_LOSS)
     int2* pze = nullptr;            // ntiles*64 (gradient modes)
-    drh::TileEnt* tent = nullptr;   // ntiles*cap2 (gradient modes)
+    drh::TileEnt* tent = nullptr;   // ntiles*cap2 (gradient modes without segw)
     int* tn = nullptr;              // ntiles*2 (gradient modes)
     int* order = nullptr;           // B*nblk, or null: launch order
     int cap2 = 0;
@@ -244,16 +244,32 @@ struct RasterBufs {
     int segw = 0;                   // fused_seg_kernel's waves per tile (RasterArgs::segw), or 0
 };
 
-// fused_seg_kernel takes the gradient calls (fused, outside the split backward)
-// whose grids hold at most SEG_MAX_TILES 8x8 tiles, two per SIMD of the
-// device: there the one-wave kernel runs about one wave per SIMD, bound by
-// each tile's chain of dependent waits, and splitting a tile's triangles over
-// SEG_WAVES waves shortens that chain. From SEG_MIN_T triangles (a couple per
-// wave) up to drh::SEG_MAX_T. DRH_NO_SEGMENTS=1 in the environment keeps the
-// other fused kernels (for comparing the paths).
-constexpr size_t SEG_MAX_TILES = 2048;
-constexpr int SEG_MIN_T = 2 * drh::SEG_WAVES;
-bool use_segments(int mode, size_t ntiles, int T);
+// fused_seg_kernel's waves per tile for a gradient call (fused) of `ntiles` 8x8
+// tiles, 0: the other kernels. Up to about a tile per SIMD a wave per tile is
+// bound by each tile's chain of dependent waits, and splitting a tile's entries
+// over waves shortens it: eight waves up to 3 tiles per CU, four up to 8 (10 for
+// a batch), two below 24, where a batch otherwise splits its heaviest blocks'
+// backward (SPLIT_*); from there on the one-wave kernel fills the device and its
+// tiles' fixed costs are less. Measured on 256 CUs, us per call, T = 128 large
+// triangles (uniform) / medium ones (random, sigma 0.01) / the same with sigma
+// 0.0015:
+//   tiles           other kernels        8 waves              4 waves              2 waves
+//    676 B=1      59 /  33 /  20      27 /  22 /  21      32 /  21 /  21      45 /  26 /  21
+//   1024 B=1      57 /  31 /  21      28 /  24 /  20      32 /  21 /  20      45 /  25 /  20
+//   2048 B=8      60 /  39 /  28      47 /  36 /  29      35 /  28 /  21      51 /  28 /  20
+//   4096 B=16     64 /  42 /  29      78 /  62 /  47      53 /  43 /  31      49 /  37 /  25
+//   5120 B=5      64 /  49 /  31      88 /  72 /  55      57 /  47 /  34      49 /  38 /  26
+//   6144 B=6      67 /  37 /  25     102 /  83 /  63      65 /  54 /  38      56 /  43 /  28
+//   4096 B=1      71 /  42 /  23      76 /  64 /  51      62 /  46 /  28      64 /  43 /  23
+// Past SEG2_MAX_T triangles two waves' LDS (20 bytes a triangle) leaves few
+// workgroups a CU: four there (B=4 256x256 T=800: 333 / 169 / 88 with the other
+// kernels, 203 / 144 / 68 with four waves, 247 / 176 / 75 with two). In the
+// fixed-order mode the tiles' partial rows grow with them: none past 8 tiles per
+// CU. From SEG_MIN_T triangles (a couple per wave) up to drh::SEG_MAX_T.
+// DRH_NO_SEGMENTS=1 in the environment keeps the other kernels (for comparing).
+constexpr size_t SEG8_MAX_TILES = 768, SEG4_MAX_TILES = 2048, SEG4_MAX_TILES_BATCH = 2560, SEG2_END_TILES = 6144;
+constexpr int SEG_MIN_T = 16, SEG2_MAX_T = 512;
+int segment_waves(int mode, int B, size_t ntiles, int T, bool det);
 
 // The one-wave fused kernel's lists scan the triangles of their tile row
 // (OrderArgs::rows) from this many triangles on. Below it a tile's box tests

@@ -304,20 +304,21 @@ bool use_order(const drh_ctx* ctx, int B, int gx, int gy) {
 
 bool fused_gradients(int mode, int nseg, int cap2, int T) {
     // cap2 > T: the one-wave kernel's backward loop reads the slot after a
-    // tile's last entry (at most T of them); the segmented kernel's regions
-    // are sized alike
+    // tile's last entry (at most T of them)
     if ((mode != drh::MODE_LOSS && mode != drh::MODE_GRAD_IN) || nseg > 1 || cap2 <= T || cap2 % 8 != 0)
         return false;
     const char* e = std::getenv("DRH_UNFUSED");
     return !(e && e[0] == '1');
 }
 
-bool use_segments(int mode, size_t ntiles, int T) {
-    if ((mode != drh::MODE_LOSS && mode != drh::MODE_GRAD_IN) || T < SEG_MIN_T || T > drh::SEG_MAX_T ||
-        ntiles > SEG_MAX_TILES)
-        return false;
+int segment_waves(int mode, int B, size_t ntiles, int T, bool det) {
+    if ((mode != drh::MODE_LOSS && mode != drh::MODE_GRAD_IN) || T < SEG_MIN_T || T > drh::SEG_MAX_T) return 0;
     const char* e = std::getenv("DRH_NO_SEGMENTS");
-    return !(e && e[0] == '1');
+    if (e && e[0] == '1') return 0;
+    if (ntiles <= SEG8_MAX_TILES) return 8;
+    if (ntiles <= (B > 1 && !det ? SEG4_MAX_TILES_BATCH : SEG4_MAX_TILES)) return 4;
+    if (B > 1 && !det && ntiles < SEG2_END_TILES) return T <= SEG2_MAX_T ? 2 : 4;
+    return 0;
 }
 
 int run_raster_bufs(drh_ctx* ctx, int mode, const float* params, const float* bgs, const float* img_in, int B,
@@ -432,9 +433,10 @@ int run_raster(drh_ctx* ctx, int mode, const float* params, const float* bgs, co
     // the records: the fit's own (FitTail::rec), else pooled
     int rc = tail && tail->rec ? DRH_OK : rec.acquire(ctx, K_REC, (size_t)B * T * drh::REC * sizeof(float), s);
     if (rc) return rc;
+    if (fused_gradients(mode, 1, bufs.cap2, T)) bufs.segw = segment_waves(mode, B, ntiles, T, det);
     const bool ordered =
         use_order(ctx, B, (int)grid.x, (int)grid.y) && (mode != drh::MODE_RENDER || T <= FWD_ORDER_MAX_T);
-    if (ordered) {
+    if (ordered && !bufs.segw) {
         const int nseg = mode == drh::MODE_RENDER ? 1 : backward_segments(T, bufs.cap2, det, (size_t)B * nblk, ctx->cus);
         if (nseg > 1) {
             const size_t words = ntiles * (size_t)(nseg - 1) * drh::CKPT_WORDS * 64;
@@ -446,11 +448,6 @@ int run_raster(drh_ctx* ctx, int mode, const float* params, const float* bgs, co
         }
     }
     bufs.fused = fused_gradients(mode, bufs.nseg, bufs.cap2, T);
-    if (bufs.fused && use_segments(mode, ntiles, T)) {
-        // each wave's region whole 64-byte lines
-        bufs.segw = drh::SEG_WAVES;
-        bufs.cap2 = drh::seg_cap2(T);
-    }
     if (ordered) {
         // the one-wave fused kernel takes an order of tiles where its cells fit
         bufs.order_tiles = bufs.fused && !det &&
@@ -471,7 +468,7 @@ int run_raster(drh_ctx* ctx, int mode, const float* params, const float* bgs, co
         const size_t prows = (size_t)B * nblk * (bufs.segw ? drh::WAVES : 1);  // per block, or per tile
         if (det && (rc = partials.acquire(ctx, K_PARTIALS, prows * T * NP * sizeof(float), s))) return rc;
         if ((rc = ploss.acquire(ctx, K_PLOSS, (size_t)B * nblk * drh::WAVES * sizeof(double), s))) return rc;  // per tile
-        if ((rc = tent.acquire(ctx, K_TILE_ENT, ntiles * bufs.cap2 * sizeof(drh::TileEnt), s))) return rc;
+        if (!bufs.segw && (rc = tent.acquire(ctx, K_TILE_ENT, ntiles * bufs.cap2 * sizeof(drh::TileEnt), s))) return rc;
         // the hand-over between the two kernels (the fused kernel keeps it in registers)
         if (!bufs.fused) {
             if ((rc = pq.acquire(ctx, K_PIXSTATE, (size_t)B * H * W * sizeof(float), s))) return rc;

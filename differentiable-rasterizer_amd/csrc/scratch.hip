@@ -64,8 +64,9 @@ struct ScratchLayout {
     bool ordered = false;
 };
 
-ScratchLayout scratch_layout(const drh_ctx* ctx, int B, int T, int H, int W, bool det) {
+ScratchLayout scratch_layout(const drh_ctx* ctx, int B, int T, int H, int W, bool det, int segw) {
     ScratchLayout L;
+    L.segw = segw;
     const dim3 grid = drh::raster_grid(B, W, H);
     const size_t nblk = (size_t)grid.x * grid.y, ntiles = (size_t)B * nblk * drh::WAVES;
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
@@ -85,23 +86,29 @@ ScratchLayout scratch_layout(const drh_ctx* ctx, int B, int T, int H, int W, boo
     L.ordered = use_order(ctx, B, (int)grid.x, (int)grid.y);
     L.order = off;
     if (L.ordered) off = up(off + (size_t)B * nblk * sizeof(int));
-    // the call takes fused_seg_kernel where drh_fused_loss_backward would
-    const int seg_cap2 = drh::seg_cap2((int)T);
-    L.segw = use_segments(drh::MODE_LOSS, ntiles, T) && fused_gradients(drh::MODE_LOSS, 1, seg_cap2, T)
-                 ? drh::SEG_WAVES
-                 : 0;
     L.partials = off;
     if (det) off = up(off + (size_t)B * nblk * (L.segw ? drh::WAVES : 1) * T * NP * sizeof(float));
     L.tent = off;
     const size_t left = SCRATCH_BYTES > off ? SCRATCH_BYTES - off : 0;
-    // whole 64-byte lines per tile and one slot past T entries, as the fused kernel needs
-    L.cap2 = tile_entries(ntiles, (T + 8) & ~7, left, 1);
-    if (L.segw && (size_t)seg_cap2 * ntiles * sizeof(drh::TileEnt) <= left)
-        L.cap2 = seg_cap2;
-    else
-        L.segw = 0;
+    // fused_seg_kernel records no entries; else whole 64-byte lines per tile and one slot past T entries, as the
+    // fused kernel needs
+    if (!L.segw) L.cap2 = tile_entries(ntiles, (T + 8) & ~7, left, 1);
     L.total = up(off + ntiles * (size_t)L.cap2 * sizeof(drh::TileEnt));
     return L;
+}
+
+// fused_seg_kernel where drh_fused_loss_backward takes it and its partial rows
+// fit (with DRH_DETERMINISTIC they are per tile), else the other kernels.
+ScratchLayout scratch_layout(const drh_ctx* ctx, int B, int T, int H, int W, bool det) {
+    const dim3 grid = drh::raster_grid(B, W, H);
+    const int segw = fused_gradients(drh::MODE_LOSS, 1, (T + 8) & ~7, T)
+                         ? segment_waves(drh::MODE_LOSS, B, (size_t)B * grid.x * grid.y * drh::WAVES, T, det)
+                         : 0;
+    if (segw) {
+        const ScratchLayout L = scratch_layout(ctx, B, T, H, W, det, segw);
+        if (L.total <= SCRATCH_BYTES) return L;
+    }
+    return scratch_layout(ctx, B, T, H, W, det, 0);
 }
 
 }  // namespace
@@ -168,8 +175,8 @@ int drh_fused_loss_backward_noalloc(drh_ctx* ctx, const float* params, const flo
     bufs.partials = det ? reinterpret_cast<float*>(base + L.partials) : nullptr;
     bufs.tent = reinterpret_cast<drh::TileEnt*>(base + L.tent);
     bufs.cap2 = L.cap2;
-    bufs.fused = fused_gradients(drh::MODE_LOSS, bufs.nseg, bufs.cap2, (int)T);
-    bufs.segw = bufs.fused ? L.segw : 0;
+    bufs.segw = L.segw;
+    bufs.fused = L.segw || fused_gradients(drh::MODE_LOSS, bufs.nseg, bufs.cap2, (int)T);
     // Nothing in the scratch array needs to start at zero: every buffer is
     // written by this call's kernels before it is read (the gradients are the
     // caller's output and setup_records clears them).
