@@ -99,18 +99,30 @@ struct OrderArgs {
     int* perm;
     int gx, gy;
     int shift = 4;
-    // Optional (the tile order, gy ceil(T / 32) <= ORD_ROW_WORDS): the live
-    // triangles whose cull box meets each cell row, in index order:
-    // rows[(b gy + y) T + i] for i < row_n[b gy + y].
-    int* rows = nullptr;
-    int* row_n = nullptr;
     // Scalings of the reach estimate, set by launch_setup from W, H and shift:
     // 1/H, a cell's height 2^shift / H, W / 2^shift, and the offsets of the
     // cell-index bounds (0.5 - 2^shift) / 2^shift and -0.5 / 2^shift.
     float r_h = 0, cell_h = 0, w_cells = 0, c0_off = 0, c1_off = 0;
 };
 constexpr int ORD_MAX_CELLS = 8192;
-constexpr int ORD_ROW_WORDS = 2048;  // LDS bit-mask words of the row lists (one bit per triangle and row)
+
+// The tile rows' lists, made by setup_records (rows null: none): the live
+// triangles whose cull box meets 8x8-tile row y of scene b, in index order:
+// rows[(b gy + y) T + i] for i < n[b gy + y], gy tile rows per scene. An entry
+// holds what a tile's box test needs: x = triangle << 3 | ROW_* and y = the first
+// and last tile column of the box, c0 | c1 << 16.
+enum : int {
+    ROW_IN = 1,     // the row's pixels lie inside the box
+    ROW_LEFT = 2,   // column c0 only partly
+    ROW_RIGHT = 4,  // column c1 only partly
+};
+struct RowArgs {
+    int2* rows = nullptr;
+    int* n = nullptr;
+    int gy = 0;
+    int parts = 0;  // workgroups per scene that make them, set by launch_setup
+};
+constexpr int ROWS_MAX_W = 65535 * TILE;  // tile columns fit 16 bits
 
 struct RasterArgs {
     int B, T, H, W;
@@ -154,9 +166,9 @@ struct RasterArgs {
     // ceil(2^32 / (2 gx)), set by the one-wave fused kernel's launch: an ordered
     // tile's row in its scene's tile grid by one multiply-high instead of a division
     uint32_t tdiv_m;
-    // OrderArgs::rows / row_n of 8x8-tile rows (row_gy per scene), or null:
-    // the one-wave fused kernel's lists then scan every triangle
-    const int* rows;
+    // RowArgs::rows / n of 8x8-tile rows (row_gy per scene), or null: the lists of
+    // the one-wave fused kernel and of renders then scan every triangle
+    const int2* rows;
     const int* row_n;
     int row_gy;
     const int* halt;       // null, or a flag: every block returns at entry once it is >= 0
@@ -260,7 +272,7 @@ hipError_t launch_setup(const float* params, int B, int T, int W, int H, float s
                         float* rec, float* zero_grads, hipStream_t s, const float* bg_src = nullptr,
                         float* bg_dst = nullptr, const OrderArgs& o = OrderArgs{}, const int* halt = nullptr,
                         RecordHead* head = nullptr, const RecordHead& head_val = RecordHead{},
-                        double* pending = nullptr, int npending = 0);
+                        double* pending = nullptr, int npending = 0, const RowArgs& rows = RowArgs{});
 // n floats set to zero by a kernel (no memset node, so callers may capture it).
 hipError_t launch_zero(float* p, size_t n, hipStream_t s);
 hipError_t launch_forward(int mode, bool fast, const RasterArgs& a, hipStream_t s);

@@ -61,6 +61,19 @@ static void launch_k(F kernel, const dim3& grid, const dim3& block, size_t lds, 
 
 constexpr float MIN_WEIGHT = 1e-6f;  // raster.rs:31-34
 
+// The wave's lanes for which `c` holds (inactive lanes 0). HIP's __ballot widens
+// the condition to an integer and compares it again, two vector instructions
+// more per call than the builtin, which takes the compare's lane mask as is.
+__device__ inline uint64_t lane_mask(bool c) { return __builtin_amdgcn_ballot_w64(c); }
+__device__ inline bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// Wave-uniform copies of values every lane holds (loaded from one address).
+// The builtin returns int: widen through uint32_t, never by sign extension.
+__device__ inline uint32_t uniform_u32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ inline uint64_t uniform_u64(uint64_t v) {
+    return ((uint64_t)uniform_u32((uint32_t)(v >> 32)) << 32) | (uint64_t)uniform_u32((uint32_t)v);
+}
+
 // ---------------------------------------------------------------- records
 
 __device__ inline float rust_clamp(float x, float lo, float hi) {
@@ -81,6 +94,32 @@ __device__ inline int upper_bound_px(float hi, float pad, int n) {
     return (c >= (float)n) ? n : (int)c + 1;
 }
 
+// The padded integer box of a triangle with vertices v (raster.rs:144-168),
+// empty unless every coordinate is finite.
+struct PixBox {
+    int x0, y0, x1, y1;  // half-open
+    __device__ bool any() const { return x0 < x1 && y0 < y1; }
+};
+__device__ inline PixBox pix_box(const float (&v)[6], int W, int H, float sigma) {
+    PixBox b = {0, 0, 0, 0};
+    bool finite = true;
+    for (int j = 0; j < 6; j++) finite = finite && isfinite(v[j]);
+    if (finite) {
+        const float pad = 6.0f * sigma;  // raster.rs:26-28
+        b.x0 = lower_bound_px(fminf(fminf(v[0], v[2]), v[4]), pad, W);
+        b.y0 = lower_bound_px(fminf(fminf(v[1], v[3]), v[5]), pad, H);
+        b.x1 = upper_bound_px(fmaxf(fmaxf(v[0], v[2]), v[4]), pad, W);
+        b.y1 = upper_bound_px(fmaxf(fmaxf(v[1], v[3]), v[5]), pad, H);
+    }
+    return b;
+}
+// A triangle of clamped opacity alpha in a setup mode (SETUP_*): render
+// (raster.rs:48-51) rejects `alpha <= 0`, which lets NaN through; the taped
+// forward (grad.rs:61-62) keeps only `alpha > 0`.
+__device__ inline bool drawn(float alpha, int setup_mode) {
+    return setup_mode == SETUP_TAPE ? alpha > 0.0f : !(alpha <= 0.0f);
+}
+
 // A triangle's cull box in order cells (inclusive; x0 > x1 when empty).
 struct BlockBox {
     int x0, y0, x1, y1;
@@ -90,20 +129,10 @@ struct BlockBox {
 // pixels, for the block-order estimate (a taped forward's liveness: alpha > 0).
 __device__ inline BlockBox block_box(const float* __restrict__ p, int W, int H, float sigma, int shift) {
     float v[6];
-    bool finite = true;
-    for (int j = 0; j < 6; j++) {
-        v[j] = p[j];
-        finite = finite && isfinite(v[j]);
-    }
-    BlockBox bb = {1, 1, 0, 0};
-    if (!finite || !(p[9] > 0.0f)) return bb;
-    const float pad = 6.0f * sigma;
-    const int bx0 = lower_bound_px(fminf(fminf(v[0], v[2]), v[4]), pad, W);
-    const int by0 = lower_bound_px(fminf(fminf(v[1], v[3]), v[5]), pad, H);
-    const int bx1 = upper_bound_px(fmaxf(fmaxf(v[0], v[2]), v[4]), pad, W);
-    const int by1 = upper_bound_px(fmaxf(fmaxf(v[1], v[3]), v[5]), pad, H);
-    if (bx0 < bx1 && by0 < by1) bb = {bx0 >> shift, by0 >> shift, (bx1 - 1) >> shift, (by1 - 1) >> shift};
-    return bb;
+    for (int j = 0; j < 6; j++) v[j] = p[j];
+    const PixBox b = pix_box(v, W, H, sigma);
+    if (!b.any() || !(p[9] > 0.0f)) return BlockBox{1, 1, 0, 0};
+    return BlockBox{b.x0 >> shift, b.y0 >> shift, (b.x1 - 1) >> shift, (b.y1 - 1) >> shift};
 }
 
 // The order estimate of one triangle: which cells it can reach. Its cull box
@@ -171,24 +200,18 @@ constexpr int REACH_PAIR_ROWS = 8;  // cell rows of a box from which reach_rows 
 // cull box alone also counts the cells between a thin or slanted triangle's
 // edges and its box, which are often most of them. r is taken by value: its
 // fields stay in registers over the rows.
-// With `rowmask` it also sets the triangle's bit k in the masks of every row of
-// its cull box (words 32-bit words per row). Without (no row lists: fewer than
-// 256 triangles, which are large), a triangle whose box spans REACH_PAIR_ROWS
-// or more cell rows takes them in pairs, each pair's run that of the two rows'
-// joint band, added to both: half the walk, which is the order workgroup's
-// longest phase for such triangles.
-template <bool MASKS>
-__device__ inline void reach_rows(const Reach r, const OrderArgs& o, int j, int m, int* cells, int pitch,
-                                  uint32_t* rowmask, int words, int k) {
+// A triangle whose box spans REACH_PAIR_ROWS or more cell rows takes them in
+// pairs, each pair's run that of the two rows' joint band, added to both: half
+// the walk, which is the order workgroup's longest phase for such triangles.
+__device__ inline void reach_rows(const Reach r, const OrderArgs& o, int j, int m, int* cells, int pitch) {
     const float cs = (float)(1 << o.shift), rH = o.r_h, cell_h = o.cell_h, wc = o.w_cells;
     const float band = (cs - 1.0f) * rH + 2.0f * r.far, y_first = 0.5f * rH - r.far;
     const float c0_off = o.c0_off, c1_off = o.c1_off;
     auto short_x = [&](float y) { return y <= r.ym ? fmaf(y - r.yt, r.s_tm, r.xt) : fmaf(y - r.ym, r.s_mb, r.xm); };
     const int x0 = r.x0(), x1 = r.x1(), y1 = r.y1();
-    const int rows = !MASKS && y1 - r.y0() + 1 >= REACH_PAIR_ROWS ? 2 : 1;
+    const int rows = y1 - r.y0() + 1 >= REACH_PAIR_ROWS ? 2 : 1;
     const float bandr = band + (float)(rows - 1) * cell_h;
     for (int y = r.y0() + rows * j; y <= y1; y += rows * m) {
-        if (MASKS) atomicOr(&rowmask[y * words + (k >> 5)], 1u << (k & 31));
         const float ya = fmaf((float)y, cell_h, y_first);
         const float ca = fmaxf(ya, r.yt), cb = fminf(ya + bandr, r.yb);
         if (!(ca <= cb)) continue;
@@ -205,7 +228,7 @@ __device__ inline void reach_rows(const Reach r, const OrderArgs& o, int j, int 
         if (c0 > c1) continue;
         atomicAdd(&cells[y * pitch + c0], 1);
         atomicAdd(&cells[y * pitch + c1 + 1], -1);
-        if (!MASKS && rows == 2 && y + 1 <= y1) {
+        if (rows == 2 && y + 1 <= y1) {
             atomicAdd(&cells[(y + 1) * pitch + c0], 1);
             atomicAdd(&cells[(y + 1) * pitch + c1 + 1], -1);
         }
@@ -223,23 +246,9 @@ __device__ inline void setup_from(const float* __restrict__ p, size_t i, int W, 
 
     bool finite = true;
     for (int j = 0; j < 6; j++) finite = finite && isfinite(v[j]);
-    int bx0 = 0, by0 = 0, bx1 = 0, by1 = 0;
-    if (finite) {
-        float pad = 6.0f * sigma;  // raster.rs:26-28
-        float lo_x = fminf(fminf(fminf(INFINITY, v[0]), v[2]), v[4]);
-        float hi_x = fmaxf(fmaxf(fmaxf(-INFINITY, v[0]), v[2]), v[4]);
-        float lo_y = fminf(fminf(fminf(INFINITY, v[1]), v[3]), v[5]);
-        float hi_y = fmaxf(fmaxf(fmaxf(-INFINITY, v[1]), v[3]), v[5]);
-        bx0 = lower_bound_px(lo_x, pad, W);
-        by0 = lower_bound_px(lo_y, pad, H);
-        bx1 = upper_bound_px(hi_x, pad, W);
-        by1 = upper_bound_px(hi_y, pad, H);
-    }
-    bool box_ok = finite && bx0 < bx1 && by0 < by1;
-    // render (raster.rs:48-51) rejects `alpha <= 0`, which lets NaN through;
-    // the taped forward (grad.rs:61-62) keeps only `alpha > 0`.
-    const bool taped = box_ok && alpha > 0.0f;
-    bool live = setup_mode == SETUP_TAPE ? taped : box_ok && !(alpha <= 0.0f);
+    const PixBox box = pix_box(v, W, H, sigma);
+    const bool taped = box.any() && drawn(alpha, SETUP_TAPE);
+    const bool live = box.any() && drawn(alpha, setup_mode);
 
     // Edges in the reference's order: (v0,v1), (v1,v2), (v2,v0); e = b - a.
     float e[6];
@@ -281,10 +290,10 @@ __device__ inline void setup_from(const float* __restrict__ p, size_t i, int W, 
     for (int j = 0; j < 3; j++) r[R_C + j] = p[6 + j];
     r[R_A] = alpha;
     int* ri = reinterpret_cast<int*>(r);
-    ri[R_BOX + 0] = live ? bx0 : 0;
-    ri[R_BOX + 1] = live ? by0 : 0;
-    ri[R_BOX + 2] = live ? bx1 : 0;
-    ri[R_BOX + 3] = live ? by1 : 0;
+    ri[R_BOX + 0] = live ? box.x0 : 0;
+    ri[R_BOX + 1] = live ? box.y0 : 0;
+    ri[R_BOX + 2] = live ? box.x1 : 0;
+    ri[R_BOX + 3] = live ? box.y1 : 0;
     bool active = p[9] > 0.0f && p[9] < 1.0f;  // grad.rs:145
     ri[R_FLAGS] = (live ? F_LIVE : 0) | (active ? F_ACTIVE : 0) | (fast && live ? F_FAST : 0) |
                   (area2 >= 0.0f ? F_CCW : 0) | (taped ? F_TAPE : 0);
@@ -355,16 +364,6 @@ constexpr int SETUP_THREADS = 1024, ORD_BUCKETS = 1024, ORD_REACH = 512, SETUP_R
 static_assert(ORD_BUCKETS == 16 * 64 && SETUP_THREADS % 64 == 0 && ORD_REACH <= SETUP_THREADS,
               "order workgroup shape: 16 buckets per lane of one wave");
 
-// Inclusive prefix sum within each row of 16 lanes (every lane active): DPP
-// row shifts (lanes with no source read the `old` operand, 0).
-__device__ inline int row_scan_incl(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);  // row_shr:2
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);  // row_shr:4
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);  // row_shr:8
-    return v;
-}
-
 // Inclusive prefix sum over the wave's lanes (every lane active).
 // DPP row shifts within each row of 16 lanes (lanes with no source read the
 // `old` operand, 0), then the last lane of rows 0 and 2 broadcast into rows 1
@@ -428,19 +427,91 @@ __device__ inline void order_scene(const OrderArgs& o, int* cells, int* hist, in
     }
 }
 
-// Workgroup (b, y): the records of scene b's triangles [x per, x per + per)
-// (and every nx per after, nx the records workgroups per scene), per the
-// records per workgroup and x = y. With o.perm (then the workgroup
-// size is SETUP_THREADS and per SETUP_REC_PER), workgroup (b, 0) makes the
-// scene's block order from the triangles' boxes, computed again from the
-// parameters, concurrently with the records of workgroups (b, x + 1). The
-// order workgroups, the longest, come first in the grid, so that they are
-// dispatched before any records.
+// The triangles of scene b whose cull box meets 8x8-tile row y, in index order,
+// by a team of up to ROW_TEAM waves of the workgroup (the other teams take other
+// rows): each wave tests up to ROW_PASSES passes of 64 triangles, from the
+// parameters (so that the rows are listed beside the records, not after them),
+// all its loads in flight at once, and compacts them by ballots behind the waves
+// before it. counts: the workgroup's, an int per wave. Every thread of the
+// workgroup enters (y may be past the last row). An earlier form set a bit per
+// triangle and row in LDS in the order workgroup, which it made the setup's
+// longest, and only beside an order.
+constexpr int ROW_TEAM = 4, ROW_PASSES = 4;
+__device__ inline void list_row(const float* __restrict__ params, int b, int y, int team, int T, int W, int H,
+                                float sigma, int setup_mode, const RowArgs& ra, int* counts) {
+    const int lane = threadIdx.x & 63, wave = (int)uniform_u32(threadIdx.x >> 6), w = wave % team;
+    const int ty0 = y * TILE, ty1 = min(ty0 + TILE, H);
+    const bool row = y < ra.gy;
+    int2* const out = ra.rows + ((size_t)b * ra.gy + (row ? y : 0)) * T;
+    const float* const p = params + (size_t)b * T * NP;
+    int n = 0;
+    for (int k0 = 0; k0 < T; k0 += 64 * ROW_PASSES * team) {
+        const int per = min((T - k0 + 64 * team - 1) / (64 * team), ROW_PASSES);  // passes of each wave
+        const int kw = k0 + w * per * 64 + lane;
+        float v[ROW_PASSES][6], al[ROW_PASSES];
+#pragma unroll
+        for (int u = 0; u < ROW_PASSES; u++) {
+            if (u >= per) break;
+            const float* const q = p + (size_t)min(kw + 64 * u, T - 1) * NP;
+            for (int j = 0; j < 6; j++) v[u][j] = q[j];
+            al[u] = q[9];
+        }
+        PixBox x[ROW_PASSES];
+        uint64_t m[ROW_PASSES];
+        int cnt = 0;
+#pragma unroll
+        for (int u = 0; u < ROW_PASSES; u++) {
+            m[u] = 0;
+            if (u >= per) break;
+            x[u] = pix_box(v[u], W, H, sigma);
+            m[u] = lane_mask(row && kw + 64 * u < T && x[u].any() &&
+                             drawn(rust_clamp(al[u], 0.0f, 1.0f), setup_mode) && x[u].y0 < ty1 && ty0 < x[u].y1);
+            cnt += (int)__popcll(m[u]);
+        }
+        int pos = n;
+        if (team > 1) {
+            if (lane == 0) counts[wave] = cnt;
+            __syncthreads();
+            for (int q = 0; q < team; q++) {
+                const int c = counts[wave - w + q];
+                pos += q < w ? c : 0;
+                n += c;
+            }
+            __syncthreads();  // before the next chunk's counts
+        } else {
+            n += cnt;
+        }
+#pragma unroll
+        for (int u = 0; u < ROW_PASSES; u++) {
+            if (u >= per) break;
+            if (in_mask(m[u])) {
+                const int c0 = x[u].x0 >> 3, c1 = (x[u].x1 - 1) >> 3;
+                int2 e;
+                e.x = (kw + 64 * u) << 3 | (x[u].x1 < min((c1 + 1) * TILE, W) ? ROW_RIGHT : 0) |
+                      (x[u].x0 > c0 * TILE ? ROW_LEFT : 0) | (x[u].y0 <= ty0 && ty1 <= x[u].y1 ? ROW_IN : 0);
+                e.y = (int)((uint32_t)c1 << 16 | (uint32_t)c0);
+                out[pos + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m[u] >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m[u], 0))] = e;
+            }
+            pos += (int)__popcll(m[u]);
+        }
+    }
+    if (row && w == 0 && lane == 0) ra.n[(size_t)b * ra.gy + y] = n;
+}
+
+// Workgroup (b, y), parts of scene b in this order:
+//  with o.perm (then of SETUP_THREADS threads), one that makes the scene's block
+//    order from the triangles' boxes, computed again from the parameters, first,
+//    so that the order workgroups, the longest, are dispatched before the rest;
+//  with ra.rows, ra.parts that list its tile rows, a team of waves each;
+//  the rest the records of triangles [x per, x per + per) (and every nx per
+//    after, nx the records workgroups per scene), per = SETUP_REC_PER beside an
+//    order or rows, else the workgroup's threads.
 __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __restrict__ params, int T, int W,
                                                                int H, float sigma, int setup_mode,
                                                                float* __restrict__ rec, float* __restrict__ zero_grads,
                                                                const float* __restrict__ bg_src,
-                                                               float* __restrict__ bg_dst, OrderArgs o,
+                                                               float* __restrict__ bg_dst, OrderArgs o, RowArgs ra,
                                                                const int* __restrict__ halt,
                                                                RecordHead* __restrict__ head, RecordHead head_val,
                                                                double* __restrict__ pending, int npending) {
@@ -448,7 +519,7 @@ __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __re
     __shared__ __attribute__((aligned(16))) int hist[ORD_BUCKETS];
     if (halt && *halt >= 0) return;
     const int b = blockIdx.x, part = blockIdx.y, pitch = o.gx + 1;
-    const int per = o.perm ? SETUP_REC_PER : (int)blockDim.x;  // records per workgroup
+    const int per = min((int)blockDim.x, SETUP_REC_PER);  // records per workgroup
     if (head && b == 0 && part == 0 && threadIdx.x == 0) *head = head_val;
     // A record kept for a later backward holds its own copy of the backgrounds.
     if (bg_dst && part == 0 && threadIdx.x < 3) bg_dst[b * 3 + threadIdx.x] = bg_src[b * 3 + threadIdx.x];
@@ -460,10 +531,18 @@ __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __re
              i += (int)(gridDim.y * blockDim.x))
             pending[(size_t)b * npending + i] = __longlong_as_double((long long)LOSS_PENDING);
     if (!o.perm || part > 0) {
+        int x = part - (o.perm ? 1 : 0);
+        if (x < ra.parts) {
+            const int waves = (int)blockDim.x / 64, team = min(waves, ROW_TEAM), teams = waves / team;
+            for (int y0 = x * teams; y0 < ra.gy; y0 += ra.parts * teams)
+                list_row(params, b, y0 + (int)(threadIdx.x >> 6) / team, team, T, W, H, sigma, setup_mode, ra, hist);
+            return;
+        }
+        x -= ra.parts;
         // grid rows are capped at 65535: a records workgroup strides over the rest
-        const int nparts = (int)gridDim.y - (o.perm ? 1 : 0);
+        const int nparts = (int)gridDim.y - (o.perm ? 1 : 0) - ra.parts;
         if ((int)threadIdx.x < per)
-            for (int k = (o.perm ? part - 1 : part) * per + (int)threadIdx.x; k < T; k += nparts * per)
+            for (int k = x * per + (int)threadIdx.x; k < T; k += nparts * per)
                 setup_one(params, (size_t)b * T + k, W, H, sigma, setup_mode, rec, zero_grads);
         return;
     }
@@ -473,11 +552,6 @@ __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __re
     // are loaded before the work that precedes its Reach (the first batch's
     // before the cells are cleared).
     __shared__ Reach reach[ORD_REACH];
-    __shared__ uint32_t rowmask_s[ORD_ROW_WORDS];
-    const int words = (T + 31) / 32;
-    uint32_t* const rowmask = o.rows && o.gy * words <= ORD_ROW_WORDS ? rowmask_s : nullptr;
-    if (rowmask)
-        for (int c = threadIdx.x; c < o.gy * words; c += SETUP_THREADS) rowmask[c] = 0u;
     float pk[NP];
     auto load_batch = [&](int k0) {
         const int k = k0 + (int)threadIdx.x;
@@ -494,50 +568,11 @@ __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __re
         __syncthreads();
         // a power of two, so that the thread's triangle and row are a shift and a mask
         const int lg = 31 - __clz(min(SETUP_THREADS / nt, 16)), m = 1 << lg;
-        for (int w = threadIdx.x; w < nt * m; w += SETUP_THREADS) {
-            if (rowmask)
-                reach_rows<true>(reach[w >> lg], o, w & (m - 1), m, cells, pitch, rowmask, words, k0 + (w >> lg));
-            else
-                reach_rows<false>(reach[w >> lg], o, w & (m - 1), m, cells, pitch, nullptr, 0, 0);
-        }
+        for (int w = threadIdx.x; w < nt * m; w += SETUP_THREADS)
+            reach_rows(reach[w >> lg], o, w & (m - 1), m, cells, pitch);
         __syncthreads();
     }
     order_scene(o, cells, hist, b, T);
-    if (!rowmask) return;
-    // Each row's set bits in index order: a scan of the words' bit counts
-    // places each word's indices. Up to 16 words (512 triangles) a row takes
-    // one 16-lane row of a wave (four rows per wave, DPP row scans), so that
-    // every row is expanded in one pass instead of one row after another.
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (words <= 16) {
-        const int sub = lane >> 4, wl = lane & 15;
-        for (int y0 = 4 * wave; y0 < o.gy; y0 += 4 * (SETUP_THREADS / 64)) {
-            const int y = y0 + sub;
-            uint32_t bits = y < o.gy && wl < words ? rowmask[y * words + wl] : 0u;
-            const int cnt = __popc(bits), incl = row_scan_incl(cnt);
-            const int total = __shfl(incl, lane | 15, 64);
-            if (y < o.gy) {
-                int* out = o.rows + ((size_t)b * o.gy + y) * T;
-                int pos = incl - cnt;
-                for (; bits; bits &= bits - 1) out[pos++] = 32 * wl + __ffs((int)bits) - 1;
-                if (wl == 0) o.row_n[(size_t)b * o.gy + y] = total;
-            }
-        }
-        return;
-    }
-    for (int y = wave; y < o.gy; y += SETUP_THREADS / 64) {
-        int* out = o.rows + ((size_t)b * o.gy + y) * T;
-        int carry = 0;
-        for (int w0 = 0; w0 < words; w0 += 64) {
-            const int w = w0 + lane;
-            uint32_t bits = w < words ? rowmask[y * words + w] : 0u;
-            const int cnt = __popc(bits), incl = wave_scan_incl(cnt, lane);
-            int pos = carry + incl - cnt;
-            for (; bits; bits &= bits - 1) out[pos++] = 32 * w + __ffs((int)bits) - 1;
-            carry += __shfl(incl, 63, 64);
-        }
-        if (lane == 0) o.row_n[(size_t)b * o.gy + y] = carry;
-    }
 }
 
 // ---------------------------------------------------------------- per-pair math
@@ -575,12 +610,6 @@ __device__ inline TileEnt ent_at(const TileEnt* __restrict__ te, int i) {
 struct Pix {
     float px, py;
 };
-
-// The wave's lanes for which `c` holds (inactive lanes 0). HIP's __ballot widens
-// the condition to an integer and compares it again, two vector instructions
-// more per call than the builtin, which takes the compare's lane mask as is.
-__device__ inline uint64_t lane_mask(bool c) { return __builtin_amdgcn_ballot_w64(c); }
-__device__ inline bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
 // All lanes where bit `bit` of the wave-uniform v is set, else none.
 __device__ inline uint64_t all_lanes_if(uint32_t v, int bit) {
@@ -865,13 +894,6 @@ __device__ inline float dpp(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, false));
 }
 
-// Wave-uniform copies of values every lane holds (loaded from one address).
-// The builtin returns int: widen through uint32_t, never by sign extension.
-__device__ inline uint32_t uniform_u32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-__device__ inline uint64_t uniform_u64(uint64_t v) {
-    return ((uint64_t)uniform_u32((uint32_t)(v >> 32)) << 32) | (uint64_t)uniform_u32((uint32_t)v);
-}
-
 // A pointer into LDS: 32-bit addresses (a generic pointer is 64-bit).
 typedef __attribute__((address_space(3))) float lds_float;
 
@@ -942,43 +964,59 @@ enum : uint32_t { CLS_PARTIAL = 1, CLS_FULL = 2 };
 // front (one round trip instead of one per branch level; the other callers
 // keep the lazy loads, whose registers their occupancy needs).
 //
-// With `ilist` (merged lists only) [k0, k1) are positions in ilist, a list of
-// triangle indices in order.
-template <bool MERGE = false>
+// ROWS (merged lists only): [k0, k1) are positions in `rows`, the list of the
+// tile row's live triangles (RowArgs), in order. The box test then needs neither
+// their records nor the row: a coalesced 8-byte load per triangle instead of a
+// cache line of its record.
+template <bool MERGE = false, bool ROWS = false>
 __device__ inline int build_list(const float* __restrict__ rec, int k0, int k1, int tx0, int ty0,
                                  int tx1, int ty1, float cx0, float cy0, float cx1, float cy1,
                                  uint32_t* list, int lane, int live, int* kend = nullptr,
-                                 const int* __restrict__ ilist = nullptr) {
+                                 const int2* __restrict__ rows = nullptr) {
     static_assert(CH >= 128, "a merged list holds two passes of candidates");
+    static_assert(MERGE || !ROWS, "row lists are merged lists");
     static_assert(R_FLAGS == R_BOX + 4, "the box tests read x0 y0 x1 y1 flags as five consecutive ints");
     const int kbase = MERGE ? 0 : k0;
     int nc = 0;
     if (MERGE) *kend = k1;
     for (int base2 = k0; base2 < k1; base2 += 128) {
         int bf[2][5];  // x0 y0 x1 y1 flags of the triangle k of each pass
-        int kk[2];     // its index
+        int2 re[2];    // ROWS: its entry
         for (int h = 0; h < 2; h++) {
             // Lanes past the chunk read its last record (in bounds) and are
             // masked out.
             const int pos = min(base2 + 64 * h + lane, k1 - 1);
-            kk[h] = ilist ? ilist[pos] : pos;
-            const int* ri = reinterpret_cast<const int*>(rec + (size_t)kk[h] * REC);
-            for (int f = 0; f < 5; f++) bf[h][f] = ri[R_BOX + f];
+            if (ROWS) {
+                re[h] = rows[pos];
+            } else {
+                const int* ri = reinterpret_cast<const int*>(rec + (size_t)pos * REC);
+                for (int f = 0; f < 5; f++) bf[h][f] = ri[R_BOX + f];
+            }
         }
         for (int h = 0; h < 2; h++) {
         const int base = base2 + 64 * h, k = base + lane;
         if (base >= k1) break;
-        const int bx0 = bf[h][0], by0 = bf[h][1], bx1 = bf[h][2], by1 = bf[h][3], flags = bf[h][4];
+        uint64_t mask, inm;
+        int index;
         // the tests are single-compare lane masks, ANDed as scalars
-        const uint64_t mask = lane_mask(k < k1) & lane_mask((flags & live) != 0) & lane_mask(tx0 < bx1) &
-                              lane_mask(bx0 < tx1) & lane_mask(ty0 < by1) & lane_mask(by0 < ty1);
-        const bool cand = __builtin_amdgcn_inverse_ballot_w64(mask);
-        const bool in_box = __builtin_amdgcn_inverse_ballot_w64(lane_mask(bx0 <= tx0) & lane_mask(tx1 <= bx1) &
-                                                                lane_mask(by0 <= ty0) & lane_mask(ty1 <= by1));
+        if (ROWS) {
+            const uint32_t c0 = (uint32_t)re[h].y & 0xFFFFu, c1 = (uint32_t)re[h].y >> 16, tc = (uint32_t)tx0 >> 3;
+            index = re[h].x >> 3;
+            mask = lane_mask(k < k1) & lane_mask(c0 <= tc) & lane_mask(tc <= c1);
+            inm = lane_mask((re[h].x & ROW_IN) != 0) & (lane_mask(c0 < tc) | lane_mask((re[h].x & ROW_LEFT) == 0)) &
+                  (lane_mask(tc < c1) | lane_mask((re[h].x & ROW_RIGHT) == 0));
+        } else {
+            const int bx0 = bf[h][0], by0 = bf[h][1], bx1 = bf[h][2], by1 = bf[h][3], flags = bf[h][4];
+            index = k;
+            mask = lane_mask(k < k1) & lane_mask((flags & live) != 0) & lane_mask(tx0 < bx1) & lane_mask(bx0 < tx1) &
+                   lane_mask(ty0 < by1) & lane_mask(by0 < ty1);
+            inm = lane_mask(bx0 <= tx0) & lane_mask(tx1 <= bx1) & lane_mask(by0 <= ty0) & lane_mask(ty1 <= by1);
+        }
+        const bool cand = in_mask(mask), in_box = in_mask(inm);
         if (cand) {
             const int pos = nc + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-            list[pos] = ((uint32_t)(kk[h] - kbase) << 1) | (in_box ? 1u : 0u);
+            list[pos] = ((uint32_t)(index - kbase) << 1) | (in_box ? 1u : 0u);
         }
         nc += (int)__popcll(mask);
         if (MERGE && nc > 64) {
@@ -1316,6 +1354,13 @@ __device__ inline TileGeo tile_geo_split(int W, int H, int gx, int gy, const int
     return tile_at(W, H, gx, gy, b, local % gx, local / gx, rank, seg, rank < K ? S : 1);
 }
 
+// The list of the tile's row (RowArgs) and its length.
+__device__ inline const int2* tile_row(const RasterArgs& a, const TileGeo& tg, int& n) {
+    const size_t row = (size_t)tg.b * a.row_gy + (tg.ty0 >> 3);
+    n = (int)uniform_u32((uint32_t)a.row_n[row]);
+    return a.rows + row * a.T;
+}
+
 // Forward: composite in scene order (raster.rs:37-68). In the gradient modes it
 // also keeps each pixel's total transmittance and records, per tile, the
 // entries that contribute at any of its pixels with their lane masks (on,
@@ -1334,21 +1379,17 @@ __device__ inline TileGeo tile_geo_split(int W, int H, int gx, int gy, const int
 // split backward's checkpoints too. lw: the wave's LDS list. MERGE: lists of
 // merged chunks (build_list), for a caller that takes every triangle index from
 // the recorded entries; rec_chunks is then meaningless.
-// [kbeg, kend) (merged lists without ROWS only; default all of them): the
-// triangles swept, and ent_off: where in the tile's region the entries go (a
-// segment of fused_seg_kernel).
 template <int MODE, bool FAST, bool CKPT, bool MERGE = false, bool ROWS = false>
 __device__ __forceinline__ void forward_sweep(const RasterArgs& a, const float* __restrict__ rec, const TileGeo& tg,
                                               uint64_t validm, const Soft& so, uint32_t* lw,
-                                              float (&col)[3], Trans& tot, int& n2, int& rec_chunks,
-                                              int kbeg = 0, int kend = -1, int ent_off = 0) {
+                                              float (&col)[3], Trans& tot, int& n2, int& rec_chunks) {
     const int T = a.T, lane = tg.lane;
     const int n_chunks = (T + CH - 1) / CH;
     n2 = 0;                 // contributing entries seen (recorded while n2 < cap2)
     rec_chunks = n_chunks;  // chunks whose contributing entries are all recorded
     const int cap2 = a.cap2;
     // wave-uniform: the entry stores address from a scalar base
-    TileEnt* te = a.tl_ent + (size_t)uniform_u32((uint32_t)tg.tile) * cap2 + ent_off;
+    TileEnt* te = a.tl_ent + (size_t)uniform_u32((uint32_t)tg.tile) * cap2;
     const TileEnt* const te0 = te;
     // Split backward: before recorded entry (c + 1) seg_m the pixel state goes to
     // checkpoint c of this tile, the start of the backward's segment c + 1 (of
@@ -1360,21 +1401,16 @@ __device__ __forceinline__ void forward_sweep(const RasterArgs& a, const float* 
     float* ckw = nck > 0 ? a.ckpt + (size_t)uniform_u32((uint32_t)tg.tile) * nck * (CKPT_WORDS * 64) : nullptr;
 
     static_assert(!(MERGE && CKPT), "checkpoints count entries per chunk");
-    static_assert(MERGE || !ROWS, "row lists are merged lists");
     // ROWS: merged lists over the tile row's triangles, which setup_records listed
-    const int* ilist = nullptr;
-    int nlist = kend < 0 ? T : kend;
-    if (ROWS) {
-        const size_t row = (size_t)tg.b * a.row_gy + (tg.ty0 >> 3);
-        ilist = a.rows + row * T;
-        nlist = a.row_n[row];
-    }
-    int k1 = MERGE ? kbeg : 0;
+    const int2* rows = nullptr;
+    int nlist = T;
+    if (ROWS && tg.live) rows = tile_row(a, tg, nlist);
+    int k1 = 0;
     for (int c = 0; MERGE ? k1 < nlist : c < n_chunks; c++) {
         const int k0 = MERGE ? k1 : c * CH;
         k1 = MERGE ? nlist : min(T, k0 + CH);
-        int count = tg.live ? build_list<MERGE>(rec, k0, k1, tg.tx0, tg.ty0, tg.tx1, tg.ty1, tg.cx0, tg.cy0,
-                                                tg.cx1, tg.cy1, lw, lane, F_LIVE, &k1, ilist)
+        int count = tg.live ? build_list<MERGE, ROWS>(rec, k0, k1, tg.tx0, tg.ty0, tg.tx1, tg.ty1, tg.cx0, tg.cy0,
+                                                      tg.cx1, tg.cy1, lw, lane, F_LIVE, &k1, rows)
                             : 0;
         const int kbase = MERGE ? 0 : k0;
         // the list one half (64 entries) at a time, one entry per lane: each
@@ -1461,8 +1497,10 @@ __device__ __forceinline__ void forward_sweep(const RasterArgs& a, const float* 
     if (MERGE) n2 = (int)(te - te0);
 }
 
-template <int MODE, bool FAST, bool CKPT>
+// ROWS (renders, which record no entries): merged lists over the tile rows' lists.
+template <int MODE, bool FAST, bool CKPT, bool ROWS>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(8))) void forward_kernel(RasterArgs a, const float* __restrict__ records) {
+    static_assert(!ROWS || MODE == MODE_RENDER, "merged lists hold no accumulator rows");
     __shared__ uint32_t list[WAVES][CH];
     __shared__ double loss[WAVES];
     if (a.halt && *a.halt >= 0) return;
@@ -1479,7 +1517,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(8)))
     col[2] = a.bg[b * 3 + 2];
     Trans tot = {1.0f, 0, 0};
     int n2, rec_chunks;
-    forward_sweep<MODE, FAST, CKPT>(a, rec, tg, validm, so, list[wave], col, tot, n2, rec_chunks);
+    forward_sweep<MODE, FAST, CKPT, ROWS, ROWS>(a, rec, tg, validm, so, list[wave], col, tot, n2, rec_chunks);
     const int cap2 = a.cap2;
 
     if (MODE == MODE_RENDER || MODE == MODE_RECORD || (MODE == MODE_LOSS && a.out_img)) {
@@ -2727,14 +2765,19 @@ hipError_t launch_fit_step(const float* partials, const double* partial_loss, in
 hipError_t launch_setup(const float* params, int B, int T, int W, int H, float sigma, int setup_mode,
                         float* rec, float* zero_grads, hipStream_t s, const float* bg_src, float* bg_dst,
                         const OrderArgs& o, const int* halt, RecordHead* head, const RecordHead& head_val,
-                        double* pending, int npending) {
+                        double* pending, int npending, const RowArgs& rows) {
     if (B == 0 || (T == 0 && !bg_dst && !o.perm && !head && !pending)) return hipSuccess;
     if (o.perm && (o.gy + 1) * (o.gx + 1) > ORD_MAX_CELLS) return hipErrorInvalidValue;
-    // without an order, small workgroups spread the triangles over more CUs;
-    // with one, a last workgroup per scene makes it
-    const int n = o.perm ? SETUP_THREADS : 64;
-    const int per = o.perm ? SETUP_REC_PER : n;  // records per workgroup (setup_records' `per`)
-    const int gx = min((T + per - 1) / per, 65534) + (o.perm || T == 0 ? 1 : 0);
+    if (rows.rows && (T == 0 || W > ROWS_MAX_W)) return hipErrorInvalidValue;
+    // without an order, small workgroups spread the triangles over more CUs (a
+    // whole team per row where one wave would take several rounds of passes: B=1
+    // 512x512 T=1024 setup 9.4 -> 5.3 us); with one, a workgroup per scene makes it
+    const int n = o.perm ? SETUP_THREADS : (rows.rows && T > 64 * ROW_PASSES ? 64 * ROW_TEAM : 64);
+    const int per = min(n, SETUP_REC_PER);  // records per workgroup (setup_records' `per`)
+    RowArgs ra = rows;
+    const int teams = n / 64 / min(n / 64, ROW_TEAM);  // rows a workgroup lists at a time
+    ra.parts = rows.rows ? min((rows.gy + teams - 1) / teams, 16384) : 0;
+    const int gx = min((T + per - 1) / per, 65534 - ra.parts) + ra.parts + (o.perm || T == 0 ? 1 : 0);
     OrderArgs oa = o;
     const float cs = (float)(1 << o.shift);
     oa.r_h = 1.0f / (float)H;
@@ -2743,7 +2786,7 @@ hipError_t launch_setup(const float* params, int B, int T, int W, int H, float s
     oa.c0_off = (0.5f - cs) / cs;
     oa.c1_off = -0.5f / cs;
     launch_k(setup_records, dim3(B, gx), dim3(n), 0, s, params, T, W, H, sigma, setup_mode, rec,
-                       zero_grads, bg_src, bg_dst, oa, halt, head, head_val, pending, npending);
+                       zero_grads, bg_src, bg_dst, oa, ra, halt, head, head_val, pending, npending);
     return hipGetLastError();
 }
 
@@ -2758,9 +2801,9 @@ dim3 raster_grid(int B, int W, int H) {
     return dim3((W + 2 * TILE - 1) / (2 * TILE), (H + 2 * TILE - 1) / (2 * TILE), B);
 }
 
-template <int MODE, bool FAST, bool CKPT = false>
+template <int MODE, bool FAST, bool CKPT = false, bool ROWS = false>
 static hipError_t launch_forward_t(const RasterArgs& a, hipStream_t s) {
-    launch_k((forward_kernel<MODE, FAST, CKPT>), raster_grid(a.B, a.W, a.H), dim3(WAVES * 64), 0, s, a,
+    launch_k((forward_kernel<MODE, FAST, CKPT, ROWS>), raster_grid(a.B, a.W, a.H), dim3(WAVES * 64), 0, s, a,
                        a.rec);
     return hipGetLastError();
 }
@@ -2771,6 +2814,9 @@ static hipError_t launch_forward_c(const RasterArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_forward(int mode, bool fast, const RasterArgs& a, hipStream_t s) {
+    if (mode == MODE_RENDER && a.rows)
+        return fast ? launch_forward_t<MODE_RENDER, true, false, true>(a, s)
+                    : launch_forward_t<MODE_RENDER, false, false, true>(a, s);
     if (mode == MODE_RENDER)
         return fast ? launch_forward_t<MODE_RENDER, true>(a, s) : launch_forward_t<MODE_RENDER, false>(a, s);
     if (mode == MODE_LOSS)

@@ -239,7 +239,7 @@ struct RasterBufs {
     int nseg = 1, seg_m = 0, nsplit = 0;  // its segments, entries per segment, split blocks per scene
     bool fused = false;             // one fused kernel (fused_gradients); pq, pg0, pze, tn unused
     bool order_tiles = false;       // `order` ranks 8x8 tiles (one-wave fused kernel only), not blocks
-    int* rows = nullptr;            // with order_tiles: B*2gy*T triangle indices per 8x8-tile row, or null
+    int2* rows = nullptr;           // B*2gy*T entries of the tile rows' lists (RowArgs), or null
     int* row_n = nullptr;           // B*2gy counts
     int segw = 0;                   // fused_seg_kernel's waves per tile (RasterArgs::segw), or 0
 };
@@ -271,12 +271,18 @@ constexpr size_t SEG8_MAX_TILES = 768, SEG4_MAX_TILES = 2048, SEG4_MAX_TILES_BAT
 constexpr int SEG_MIN_T = 16, SEG2_MAX_T = 512;
 int segment_waves(int mode, int B, size_t ntiles, int T, bool det);
 
-// The one-wave fused kernel's lists scan the triangles of their tile row
-// (OrderArgs::rows) from this many triangles on. Below it a tile's box tests
-// are at most a few passes of 64 and making the row lists costs setup_records
-// more than it saves (measured at T = 128: +3.3 us of setup, the fused kernel
-// unchanged; at T = 512 with small triangles the fused kernel 35.7 -> 31.7 us).
-constexpr int ROW_LISTS_MIN_T = 256;
+// From these many triangles on the one-wave fused kernel's and renders' lists scan
+// the triangles of their tile row (RowArgs), which setup_records lists beside the
+// records: a tile's box tests then read a few coalesced words instead of every
+// triangle's record. us per call without and with, large (uniform) / medium
+// (random, sigma 0.004) / small triangles: fused B=16 256x256 T=64 54.9 / 34.7 /
+// 25.3 -> 51.4 / 34.5 / 24.8, T=512 308 / 127 / 62.6 -> 301 / 123 / 50.1; renders
+// B=1 512x512 T=1024 107 / 48.8 / 29.3 -> 111 / 39.5 / 22.7, 1024x1024 T=150 41.1
+// / 30.6 / 20.9 -> 36.9 / 25.4 / 20.7, T=64 unchanged. The segmented kernel's
+// waves share the scan, and waiting for a row first cost it up to 10%: it scans
+// every triangle.
+constexpr int ROW_LISTS_MIN_T_FUSED = 64, ROW_LISTS_MIN_T_RENDER = 128;
+constexpr size_t ROW_LISTS_BUDGET = 256ull << 20;  // bytes
 
 // Split of the backward's sweep over a tile's recorded entries. A tile's sweep
 // is sequential, and the tiles with the longest lists sit together (a block's

@@ -333,8 +333,9 @@ int run_raster_bufs(drh_ctx* ctx, int mode, const float* params, const float* bg
     const int nrows = bufs.segw ? nblk * drh::WAVES : nblk;
     drh::OrderArgs ord{};
     if (bufs.order)
-        ord = bufs.order_tiles ? drh::OrderArgs{bufs.order, 2 * (int)grid.x, 2 * (int)grid.y, 3, bufs.rows, bufs.row_n}
+        ord = bufs.order_tiles ? drh::OrderArgs{bufs.order, 2 * (int)grid.x, 2 * (int)grid.y, 3}
                                : drh::OrderArgs{bufs.order, (int)grid.x, (int)grid.y, 4};
+    const drh::RowArgs rows{bufs.rows, bufs.row_n, bufs.rows ? 2 * (int)grid.y : 0};
     // the fused kernels sum the losses themselves outside the fixed-order mode
     // (RasterArgs::loss_tail): setup_records marks the loss slots pending
     const bool loss_tail = bufs.fused && !det && mode == drh::MODE_LOSS && !(tail && tail->rec_ready);
@@ -344,7 +345,7 @@ int run_raster_bufs(drh_ctx* ctx, int mode, const float* params, const float* bg
                                   mode == drh::MODE_RENDER ? drh::SETUP_RENDER : drh::SETUP_TAPE, bufs.rec,
                                   mode != drh::MODE_RENDER && !det ? out_grads : nullptr, s, nullptr, nullptr,
                                   ord, halt, nullptr, drh::RecordHead{}, loss_tail ? bufs.ploss : nullptr,
-                                  nblk * drh::WAVES),
+                                  nblk * drh::WAVES, rows),
                 "setup_records launch");
     }
     drh::RasterArgs a{};
@@ -371,8 +372,8 @@ int run_raster_bufs(drh_ctx* ctx, int mode, const float* params, const float* bg
     a.perm_fwd = T <= FWD_ORDER_MAX_T ? ord.perm : nullptr;
     a.perm_bwd = ord.perm;
     a.perm_tiles = bufs.order_tiles ? 1 : 0;
-    a.rows = bufs.order_tiles ? bufs.rows : nullptr;
-    a.row_n = bufs.order_tiles ? bufs.row_n : nullptr;
+    a.rows = bufs.rows;
+    a.row_n = bufs.row_n;
     a.row_gy = 2 * (int)grid.y;
     a.halt = halt;
     a.nseg = bufs.ckpt && ord.perm ? bufs.nseg : 1;
@@ -455,14 +456,15 @@ int run_raster(drh_ctx* ctx, int mode, const float* params, const float* bgs, co
         const size_t cells = (size_t)B * nblk * (bufs.order_tiles ? drh::WAVES : 1);
         if ((rc = order.acquire(ctx, K_ORDER, cells * sizeof(int), s))) return rc;
         bufs.order = order.get<int>();
-        // the tile rows' triangle lists, where their bit masks fit setup_records' LDS
-        const size_t trows = (size_t)B * 2 * grid.y;
-        if (bufs.order_tiles && !bufs.segw && T >= ROW_LISTS_MIN_T &&
-            (size_t)2 * grid.y * ((T + 31) / 32) <= (size_t)drh::ORD_ROW_WORDS) {
-            if ((rc = rows.acquire(ctx, K_ROWS, (trows * T + trows) * sizeof(int), s))) return rc;
-            bufs.rows = rows.get<int>();
-            bufs.row_n = bufs.rows + trows * T;
-        }
+    }
+    // the tile rows' lists, where the call's kernel reads them
+    const size_t trows = (size_t)B * 2 * grid.y;
+    const int rows_min_t = mode == drh::MODE_RENDER ? ROW_LISTS_MIN_T_RENDER : ROW_LISTS_MIN_T_FUSED;
+    if ((mode == drh::MODE_RENDER || (bufs.fused && !bufs.segw && !det)) && T >= rows_min_t && W <= drh::ROWS_MAX_W &&
+        trows * T * sizeof(int2) <= ROW_LISTS_BUDGET) {
+        if ((rc = rows.acquire(ctx, K_ROWS, trows * T * sizeof(int2) + trows * sizeof(int), s))) return rc;
+        bufs.rows = rows.get<int2>();
+        bufs.row_n = reinterpret_cast<int*>(bufs.rows + trows * T);
     }
     if (mode != drh::MODE_RENDER) {
         const size_t prows = (size_t)B * nblk * (bufs.segw ? drh::WAVES : 1);  // per block, or per tile
