@@ -297,7 +297,16 @@ hipError_t launch_reduce(const float* partials, const double* partial_loss, int 
 struct SrgbTable {
     float v[256];
 };
-hipError_t launch_encode_srgb(const float* in, int64_t n, uint8_t* out, const SrgbTable& thresholds, hipStream_t s);
+// The encoding's tables: the thresholds, and per run of floats with the same
+// exponent and first seven mantissa bits, from SRGB_FIRST (2^-13, below t_1) up to
+// 1.0f, the byte of the run's first float, four to a word.
+constexpr int SRGB_SHIFT = 16, SRGB_FIRST = 0x3900, SRGB_RUNS = 0x3F80 - SRGB_FIRST + 4;
+static_assert(SRGB_RUNS % 4 == 0, "whole words");
+struct SrgbEncode {
+    SrgbTable t;
+    uint32_t base[SRGB_RUNS / 4];
+};
+hipError_t launch_encode_srgb(const float* in, int64_t n, uint8_t* out, const SrgbEncode& tab, hipStream_t s);
 hipError_t launch_decode_srgb(const uint8_t* in, int64_t n, float* out, const SrgbTable& values, hipStream_t s);
 
 hipError_t launch_adam(float* params, const float* grads, float* m, float* v, const float* lr, int n,

@@ -2703,25 +2703,50 @@ __global__ __launch_bounds__(256) void zero_floats(float* __restrict__ p, size_t
 
 // ---------------------------------------------------------------- sRGB bytes
 
-// canvas.rs:100-105 encode_srgb, one value per thread: the byte is the number
-// of thresholds t_1 < ... < t_255 at or below v (t_k the smallest linear value
-// the reference encodes to k), found by an 8-step binary search in LDS. The
-// reference's encoding is monotonic in v on [0, 1] (checked over every float
-// there) and constant outside it after its clamp, so the count is its byte;
-// NaN compares false everywhere and gives 0, as its saturating cast does.
+// canvas.rs:100-105 encode_srgb: the byte is the number of thresholds t_1 < ... <
+// t_255 at or below v (t_k the smallest linear value the reference encodes to k).
+// The reference's encoding is monotonic in v on [0, 1] (checked over every float
+// there) and constant outside it after its clamp, so the count is its byte; NaN
+// gives 0, as its saturating cast does. The value's exponent and first seven
+// mantissa bits index a table of the count at the start of that run of floats,
+// and no run holds more than one threshold (neighbouring ones are at least 1.5
+// runs apart, just above 1/2, and t_1 = 1.52e-4 lies above the first run), so one
+// more compare gives the count: two LDS reads a value, where a binary search
+// among the thresholds took eight, and four values a load instead of one. 3.1
+// million values 8.0 -> 5.1 us (3.3 at the rate of a large copy), 50 million a
+// call 91 -> 37 us.
+__device__ inline uint32_t encode_value(float v, const float* t, const uint8_t* base) {
+    v = v > 0.0f ? v : 0.0f;  // NaN: 0
+    v = v < 1.0f ? v : 1.0f;
+    const int i = max((int)(__float_as_uint(v) >> SRGB_SHIFT) - SRGB_FIRST, 0);  // v <= 1: below SRGB_RUNS
+    const uint32_t b = base[i];
+    return b + (t[b + 1] <= v ? 1u : 0u);
+}
+// VEC: four values per load and store (`in` 16-byte, `out` 4-byte aligned).
+template <bool VEC>
 __global__ __launch_bounds__(256) void encode_srgb_kernel(const float* __restrict__ in, int64_t n,
-                                                          uint8_t* __restrict__ out, SrgbTable thr) {
-    __shared__ float t[256];
-    t[threadIdx.x] = thr.v[threadIdx.x];
+                                                          uint8_t* __restrict__ out, SrgbEncode tab) {
+    __shared__ float t[257];
+    __shared__ uint32_t base4[SRGB_RUNS / 4];
+    t[threadIdx.x] = tab.t.v[threadIdx.x];
+    if (threadIdx.x == 0) t[256] = INFINITY;
+    for (int i = threadIdx.x; i < SRGB_RUNS / 4; i += 256) base4[i] = tab.base[i];
     __syncthreads();
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const float v = in[i];
-        int b = 0;
-#pragma unroll
-        for (int step = 128; step >= 1; step >>= 1) b += (t[b + step] <= v) ? step : 0;
-        out[i] = (uint8_t)b;
+    const uint8_t* const base = reinterpret_cast<const uint8_t*>(base4);
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int64_t done = 0;
+    if (VEC) {
+        const int64_t n4 = n / 4;
+        const float4* const in4 = reinterpret_cast<const float4*>(in);
+        uint32_t* const out4 = reinterpret_cast<uint32_t*>(out);
+        for (int64_t i = first; i < n4; i += stride) {
+            const float4 v = in4[i];
+            out4[i] = encode_value(v.x, t, base) | encode_value(v.y, t, base) << 8 | encode_value(v.z, t, base) << 16 |
+                      encode_value(v.w, t, base) << 24;
+        }
+        done = 4 * n4;
     }
+    for (int64_t i = done + first; i < n; i += stride) out[i] = (uint8_t)encode_value(in[i], t, base);
 }
 
 // canvas.rs:108-115 decode_srgb: a lookup in the table of all 256 values.
@@ -2740,9 +2765,16 @@ static dim3 stream_grid(int64_t n) {
     return dim3((unsigned)(blocks < 8192 ? (blocks > 0 ? blocks : 1) : 8192));
 }
 
-hipError_t launch_encode_srgb(const float* in, int64_t n, uint8_t* out, const SrgbTable& thresholds, hipStream_t s) {
+hipError_t launch_encode_srgb(const float* in, int64_t n, uint8_t* out, const SrgbEncode& tab, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    launch_k(encode_srgb_kernel, stream_grid(n), dim3(256), 0, s, in, n, out, thresholds);
+    // a workgroup's table costs it about what 2000 values do: fewer, longer ones
+    const bool vec = (uintptr_t)in % 16 == 0 && (uintptr_t)out % 4 == 0;
+    const int64_t want = (vec ? n / 4 : n) / (256 * 2) + 1;
+    const dim3 grid((unsigned)(want < 2048 ? want : 2048));
+    if (vec)
+        launch_k(encode_srgb_kernel<true>, grid, dim3(256), 0, s, in, n, out, tab);
+    else
+        launch_k(encode_srgb_kernel<false>, grid, dim3(256), 0, s, in, n, out, tab);
     return hipGetLastError();
 }
 

@@ -629,7 +629,8 @@ float float_of_bits(uint32_t b) {
 }
 
 struct SrgbTables {
-    drh::SrgbTable thresholds, values;
+    drh::SrgbEncode encode;
+    drh::SrgbTable values;
 };
 
 // Entry k of the thresholds: the smallest float in [0, 1] that encodes to k or
@@ -639,7 +640,8 @@ const SrgbTables& srgb_tables() {
     static SrgbTables t;
     static std::once_flag once;
     std::call_once(once, [] {
-        t.thresholds.v[0] = 0.0f;
+        drh::SrgbTable& th = t.encode.t;
+        th.v[0] = 0.0f;
         for (int k = 1; k < 256; k++) {
             uint32_t lo = 0, hi = 0x3F800000u;  // encode(0) = 0 < k <= encode(1) = 255
             while (lo + 1 < hi) {
@@ -649,7 +651,14 @@ const SrgbTables& srgb_tables() {
                 else
                     lo = mid;
             }
-            t.thresholds.v[k] = float_of_bits(hi);
+            th.v[k] = float_of_bits(hi);
+        }
+        // the bytes at the starts of the runs
+        int k = 0;
+        for (int r = 0; r < drh::SRGB_RUNS; r++) {
+            const float start = float_of_bits((uint32_t)(drh::SRGB_FIRST + r) << drh::SRGB_SHIFT);
+            while (k < 255 && th.v[k + 1] <= start) k++;
+            t.encode.base[r / 4] |= (uint32_t)k << (8 * (r % 4));
         }
         for (int b = 0; b < 256; b++) t.values.v[b] = decode_srgb_host((uint8_t)b);
     });
@@ -1044,7 +1053,7 @@ int drh_encode_srgb(drh_ctx* ctx, const float* values, int64_t n, uint8_t* out, 
         if ((rc = ob.acquire(ctx, K_SRGB_U8, (size_t)n, s))) return rc;
         dout = ob.get<uint8_t>();
     }
-    HIP_TRY(drh::launch_encode_srgb(in.dev, n, dout, srgb_tables().thresholds, s), "encode_srgb launch");
+    HIP_TRY(drh::launch_encode_srgb(in.dev, n, dout, srgb_tables().encode, s), "encode_srgb launch");
     if (host) {
         hipError_t e = hipMemcpyAsync(out, dout, (size_t)n, hipMemcpyDeviceToHost, s);
         if (e != hipSuccess) return fail(DRH_ERR_READBACK, std::string("hipMemcpyAsync D2H: ") + hipGetErrorString(e));
