@@ -109,11 +109,10 @@ int launch_iteration(drh_fitter* f, int64_t i) {
 
 // Reads the device state (and, when `loss` is given, the last loss) back.
 int read_state(drh_fitter* f, float* loss = nullptr) {
-    HIP_TRY(hipMemcpyAsync(&f->last, f->st + (f->launched & 1), sizeof f->last, hipMemcpyDeviceToHost, f->s),
-            "read fit state");
-    if (loss) HIP_TRY(hipMemcpyAsync(loss, f->loss, sizeof(float), hipMemcpyDeviceToHost, f->s), "read loss");
-    int rc = wait_stream(f->s);
-    if (rc) return rc;
+    HostStage hs(f->ctx, f->s, sizeof f->last + sizeof(float) + HOST_PAD);
+    int rc = hs.out(&f->last, f->st + (f->launched & 1), sizeof f->last);
+    if (!rc && loss) rc = hs.out(loss, f->loss, sizeof(float));
+    if (rc || (rc = hs.finish())) return rc;
     if (f->last.stop >= 0) {
         f->stopped = true;
         f->stop_reason = f->last.stop;
@@ -124,13 +123,33 @@ int read_state(drh_fitter* f, float* loss = nullptr) {
     return DRH_OK;
 }
 
-int copy_out(drh_fitter* f, float* dst, const float* src, size_t n, uint32_t flags) {
+// n device floats to the caller's array, host memory through hs (which the
+// caller finishes).
+int copy_out(drh_fitter* f, float* dst, const float* src, size_t n, uint32_t flags, HostStage& hs) {
     if (n == 0) return DRH_OK;
     if (!dst) return fail(DRH_ERR_INVALID_ARG, "output pointer is NULL");
-    const hipMemcpyKind k = (flags & DRH_HOST_PTRS) ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
-    hipError_t e = hipMemcpyAsync(dst, src, n * sizeof(float), k, f->s);
+    if (flags & DRH_HOST_PTRS) return hs.out(dst, src, n * sizeof(float));
+    hipError_t e = hipMemcpyAsync(dst, src, n * sizeof(float), hipMemcpyDeviceToDevice, f->s);
     if (e != hipSuccess) return fail(DRH_ERR_READBACK, std::string("hipMemcpyAsync: ") + hipGetErrorString(e));
-    return finish(flags, f->s);
+    return DRH_OK;
+}
+
+size_t host_bytes(uint32_t flags, size_t floats) {
+    return (flags & DRH_HOST_PTRS) ? floats * sizeof(float) + HOST_PAD : 0;
+}
+
+int copy_out(drh_fitter* f, float* dst, const float* src, size_t n, uint32_t flags) {
+    HostStage hs(f->ctx, f->s, host_bytes(flags, n));
+    int rc = copy_out(f, dst, src, n, flags, hs);
+    return rc || n == 0 ? rc : finish(flags, f->s, hs);
+}
+
+void fill_report(const drh_fitter* f, drh_fit_report* report) {
+    // Fitter::into_report (fit.rs:326-334): stop_reason.unwrap_or(Completed)
+    report->n_losses = f->last.n_losses;
+    report->best_iter = f->last.best_iter;
+    report->best_loss = f->last.best_loss;
+    report->stop_reason = f->stopped ? f->stop_reason : DRH_STOP_COMPLETED;
 }
 
 }  // namespace
@@ -208,20 +227,21 @@ int drh_fitter_create(drh_ctx* ctx, const float* target, int64_t H, int64_t W, c
     }
     const drh::FitState st0{INFINITY, 0, 0, 0, -1};
     const FitDevState dev0{{st0, st0}, -1};
-    const hipMemcpyKind in = host ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-    auto copy = [&](void* dst, const void* src, size_t bytes, hipMemcpyKind k) {
-        return hipMemcpyAsync(dst, src, bytes, k, f->s);
+    HostStage hs(ctx, f->s, (host ? (2 * n + npix3 + 3) * sizeof(float) : 0) + n * sizeof(float) + sizeof dev0 + HOST_PAD);
+    auto copy = [&](void* dst, const void* src, size_t bytes) -> int {
+        if (host) return hs.in(dst, src, bytes);
+        HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, f->s), "fitter set-up copies");
+        return DRH_OK;
     };
-    hipError_t e = copy(f->params, init_params, n * sizeof(float), in);
-    if (e == hipSuccess) e = copy(f->best, init_params, n * sizeof(float), in);
-    if (e == hipSuccess) e = copy(f->target, target, npix3 * sizeof(float), in);
-    if (e == hipSuccess) e = copy(f->bg, background, 3 * sizeof(float), in);
-    if (e == hipSuccess) e = copy(f->lr, lr.data(), n * sizeof(float), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = copy(f->state.get<FitDevState>(), &dev0, sizeof dev0, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return bail(hip_fail(e, "fitter set-up copies"));
-    if ((e = drh::launch_zero(f->m, 2 * n, f->s)) != hipSuccess) return bail(hip_fail(e, "zero moments"));
-    // lr and dev0 are host stack memory: wait before they go
-    if ((rc = wait_stream(f->s))) return bail(rc);
+    if ((rc = copy(f->params, init_params, n * sizeof(float))) || (rc = copy(f->best, init_params, n * sizeof(float))) ||
+        (rc = copy(f->target, target, npix3 * sizeof(float))) || (rc = copy(f->bg, background, 3 * sizeof(float))) ||
+        (rc = hs.in(f->lr, lr.data(), n * sizeof(float))) ||
+        (rc = hs.in(f->state.get<FitDevState>(), &dev0, sizeof dev0)))
+        return bail(rc);
+    hipError_t e = drh::launch_zero(f->m, 2 * n, f->s);
+    if (e != hipSuccess) return bail(hip_fail(e, "zero moments"));
+    // the arrays may be host memory that goes when this returns
+    if ((rc = hs.finish())) return bail(rc);
     f->last = st0;
     *out = f;
     return DRH_OK;
@@ -317,14 +337,15 @@ int drh_fitter_render_current(drh_fitter* f, float* out_image, uint32_t flags) {
     if (!out_image) return fail(DRH_ERR_INVALID_ARG, "output pointer is NULL");
     DeviceGuard dg(f->ctx->device);
     // fit.rs:320-324: the current scene at its sharpest setting
+    HostStage hs(f->ctx, f->s, host_bytes(flags, (size_t)f->H * f->W * 3));
     Out img;
     int rc = stage_out(f->ctx, img, K_OUT_IMAGES, out_image, (size_t)f->H * f->W * 3, flags & DRH_HOST_PTRS, f->s);
     if (rc) return rc;
     if ((rc = run_raster(f->ctx, drh::MODE_RENDER, f->params, f->bg, nullptr, 1, f->T, f->H, f->W, f->cfg.sigma_end,
                          img.dev, nullptr, nullptr, f->math, f->s)))
         return rc;
-    if ((rc = copy_back(img, f->s))) return rc;
-    return finish(flags, f->s);
+    if ((rc = copy_back(img, hs))) return rc;
+    return finish(flags, f->s, hs);
 }
 
 int drh_fitter_report(drh_fitter* f, float* out_best_params, drh_fit_report* report, uint32_t flags) {
@@ -332,11 +353,7 @@ int drh_fitter_report(drh_fitter* f, float* out_best_params, drh_fit_report* rep
     DeviceGuard dg(f->ctx->device);
     int rc = copy_out(f, out_best_params, f->best, (size_t)f->T * NP, flags | DRH_SYNC);
     if (rc) return rc;
-    // Fitter::into_report (fit.rs:326-334): stop_reason.unwrap_or(Completed)
-    report->n_losses = f->last.n_losses;
-    report->best_iter = f->last.best_iter;
-    report->best_loss = f->last.best_loss;
-    report->stop_reason = f->stopped ? f->stop_reason : DRH_STOP_COMPLETED;
+    fill_report(f, report);
     return DRH_OK;
 }
 
@@ -349,12 +366,18 @@ int drh_fit(drh_ctx* ctx, const float* target, int64_t H, int64_t W, const float
     drh_fitter* f = nullptr;
     int rc = drh_fitter_create(ctx, target, H, W, background, init_params, T, cfg, stream, flags, &f);
     if (rc) return rc;
-    const uint32_t out_flags = flags & DRH_HOST_PTRS;
-    int64_t n = 0;
-    if (!(rc = drh_fitter_run(f, cfg->iters, nullptr)) &&
-        !(rc = drh_fitter_losses(f, out_losses, cfg->iters, &n, out_flags)) &&
-        !(rc = out_params ? drh_fitter_scene(f, out_params, out_flags) : DRH_OK))
-        rc = drh_fitter_report(f, out_best_params, report, out_flags);
+    const uint32_t out_flags = (flags & DRH_HOST_PTRS) | DRH_SYNC;
+    const size_t np = (size_t)T * NP;
+    if (!(rc = drh_fitter_run(f, cfg->iters, nullptr))) {
+        // everything that goes out, in one wait
+        DeviceGuard dg(ctx->device);
+        const size_t n = (size_t)f->last.n_losses;
+        HostStage hs(ctx, f->s, host_bytes(flags, n + 2 * np));
+        if (!(rc = copy_out(f, out_losses, f->losses, n, out_flags, hs)) &&
+            !(rc = out_params ? copy_out(f, out_params, f->params, np, out_flags, hs) : DRH_OK) &&
+            !(rc = copy_out(f, out_best_params, f->best, np, out_flags, hs)) && !(rc = finish(out_flags, f->s, hs)))
+            fill_report(f, report);
+    }
     drh_fitter_destroy(f);
     return rc;
 }

@@ -17,11 +17,11 @@
 // device sums in the same order without fusing (built with -ffp-contract=off).
 //
 // Memory traffic per pass is one read of its input rows per tap that covers
-// them and one write; this is a load-time helper (a few milliseconds for a
-// photograph), not part of the fit's hot path.
+// them and one write; this is a load-time helper, not part of the fit's hot path.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstdint>
@@ -128,13 +128,17 @@ extern "C" int drh_resize_lanczos3(drh_ctx* ctx, const uint8_t* src, int64_t H, 
     const size_t in_bytes = (size_t)(H * W * C), out_bytes = (size_t)(new_H * new_W * C);
     int rc;
 
+    // room for a host image both ways and the tables (at most 2 support + 2 weights an output index)
+    auto most = [](int64_t n, int64_t m) { return (size_t)m * (6 * ((size_t)std::max(n, m) / (size_t)m + 1) + 2); };
+    const size_t tables = (size_t)(new_H + new_W) * sizeof(Tap) + (most(H, new_H) + most(W, new_W)) * sizeof(float);
+    HostStage hs(ctx, s, (host ? in_bytes + out_bytes : 0) + tables + HOST_PAD);
     Lease in_l, out_l;
     const uint8_t* din = src;
     uint8_t* dout = dst;
     if (host) {
         if ((rc = in_l.acquire(ctx, K_SRGB_U8, in_bytes, s)) || (rc = out_l.acquire(ctx, K_RESIZE_U8, out_bytes, s)))
             return rc;
-        HIP_TRY(hipMemcpyAsync(in_l.get<uint8_t>(), src, in_bytes, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
+        if ((rc = hs.in(in_l.get<uint8_t>(), src, in_bytes))) return rc;
         din = in_l.get<uint8_t>();
         dout = out_l.get<uint8_t>();
     }
@@ -148,21 +152,20 @@ extern "C" int drh_resize_lanczos3(drh_ctx* ctx, const uint8_t* src, int64_t H, 
         build_taps(H, new_H, taps, weights);
         build_taps(W, new_W, taps, weights);
         const size_t tap_bytes = taps.size() * sizeof(Tap), w_bytes = weights.size() * sizeof(float);
-        const size_t tmp_bytes = (size_t)new_H * (size_t)(W * C) * sizeof(float);
         Lease tap_l, w_l, tmp_l;
-        if ((rc = tap_l.acquire(ctx, K_RESIZE_TAB, tap_bytes, s)) || (rc = w_l.acquire(ctx, K_RESIZE_TAB, w_bytes, s)) ||
-            (rc = tmp_l.acquire(ctx, K_RESIZE_TMP, tmp_bytes, s)))
+        if ((rc = tap_l.acquire(ctx, K_RESIZE_TAB, tap_bytes, s)) || (rc = w_l.acquire(ctx, K_RESIZE_TAB, w_bytes, s)))
             return rc;
         // Copied from host vectors: the stream is waited for below, before
         // they go out of scope.
-        HIP_TRY(hipMemcpyAsync(tap_l.get<Tap>(), taps.data(), tap_bytes, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
-        HIP_TRY(hipMemcpyAsync(w_l.get<float>(), weights.data(), w_bytes, hipMemcpyHostToDevice, s),
-                "hipMemcpyAsync H2D");
+        if ((rc = hs.in(tap_l.get<Tap>(), taps.data(), tap_bytes)) || (rc = hs.in(w_l.get<float>(), weights.data(), w_bytes)))
+            return rc;
         const Tap* dv = tap_l.get<Tap>();
         const Tap* dh = dv + new_H;
         const float* dw = w_l.get<float>();
         const int row_elems = (int)(W * C), out_elems = (int)(new_W * C);
         const unsigned gy = (unsigned)(new_H < RS_MAX_GRID_Y ? new_H : RS_MAX_GRID_Y);
+        const size_t tmp_bytes = (size_t)new_H * (size_t)(W * C) * sizeof(float);
+        if ((rc = tmp_l.acquire(ctx, K_RESIZE_TMP, tmp_bytes, s))) return rc;
         hipLaunchKernelGGL(resize_rows, dim3((unsigned)((row_elems + RS_THREADS - 1) / RS_THREADS), gy),
                            dim3(RS_THREADS), 0, s, din, row_elems, (int)new_H, dv, dw, tmp_l.get<float>());
         HIP_TRY(hipGetLastError(), "resize_rows launch");
@@ -170,11 +173,9 @@ extern "C" int drh_resize_lanczos3(drh_ctx* ctx, const uint8_t* src, int64_t H, 
                            dim3(RS_THREADS), 0, s, tmp_l.get<float>(), (int)W, (int)C, (int)new_W, (int)new_H, dh,
                            dw, dout);
         HIP_TRY(hipGetLastError(), "resize_cols launch");
-        if ((rc = wait_stream(s))) return rc;
+        if (host && (rc = hs.out(dst, dout, out_bytes))) return rc;
+        return hs.finish();
     }
-    if (host) {
-        hipError_t e = hipMemcpyAsync(dst, dout, out_bytes, hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) return fail(DRH_ERR_READBACK, std::string("hipMemcpyAsync D2H: ") + hipGetErrorString(e));
-    }
-    return finish(flags, s);
+    if (host && (rc = hs.out(dst, dout, out_bytes))) return rc;
+    return finish(flags, s, hs);
 }

@@ -76,6 +76,12 @@ struct PoolBuf {
     bool ev_recorded = false;      // `ev` marks the end of the last use
 };
 
+// Page-locked host memory that the calls with host arrays stage through.
+struct PinnedBuf {
+    char* ptr = nullptr;
+    size_t bytes = 0;
+};
+
 enum TimedKernel : int { TK_SETUP = 0, TK_RASTER, TK_REDUCE, TK_ADAM, TK_BACKWARD, TK_COUNT };
 struct TimedLaunch {
     int kernel;
@@ -104,6 +110,8 @@ struct drh_ctx {
     // so that drh_backward_recorded checks its arguments without reading the
     // device; a record made elsewhere has its head read from the device.
     std::unordered_map<const void*, drh::RecordHead> records;
+    std::vector<drh_rt::PinnedBuf> free_pinned;  // at most PINNED_KEEP bytes, freed by drh_clear_pool
+    size_t pinned_bytes = 0;
 };
 
 namespace drh_rt {
@@ -152,7 +160,46 @@ struct DeviceGuard {
 };
 
 // Host wait bounded like GpuRasterizer::POLL_TIMEOUT (crates/diffrast-gpu/src/lib.rs:229).
+// Polls without sleeping for WAIT_SPIN_US first: a sleep wakes ~100 us later at
+// best, which was longer than most of what is waited for.
+constexpr int WAIT_SPIN_US = 2000;
 int wait_stream(hipStream_t s);
+
+// The host arrays of one call, copied through one page-locked buffer: an
+// asynchronous copy each, where a copy from or to pageable memory blocks the host
+// for ~24 us however small. Arrays that do not fit the buffer (PINNED_MAX at
+// most) are copied as they are. in() may be followed by changes to the caller's
+// array at once; out()'s arrays hold their values once finish() has waited for
+// the stream. The buffer goes back to the context only when nothing queued uses
+// it: after finish(), or else after a wait in the destructor.
+constexpr size_t PINNED_MIN = 1ull << 20, PINNED_MAX = 16ull << 20, PINNED_KEEP = 64ull << 20;
+class HostStage {
+  public:
+    // bytes: of the arrays to come, all together (in and out); 0 where the arrays are device memory
+    HostStage(drh_ctx* ctx, hipStream_t s, size_t bytes);
+    ~HostStage();
+    HostStage(const HostStage&) = delete;
+    HostStage& operator=(const HostStage&) = delete;
+    int in(void* dev, const void* src, size_t bytes);
+    int out(void* dst, const void* dev, size_t bytes);
+    int finish();  // waits for the stream and fills out()'s arrays
+
+  private:
+    char* take(size_t bytes);
+    struct Back {
+        void* dst;
+        const char* src;
+        size_t bytes;
+    };
+    drh_ctx* ctx_;
+    hipStream_t s_;
+    PinnedBuf buf_;
+    size_t used_ = 0;
+    bool pending_ = false;
+    Back back_[4];
+    int nback_ = 0;
+};
+constexpr size_t HOST_PAD = 8 * 256;  // the arrays' alignment in a HostStage's buffer
 
 // Argument checks shared by the raster entry points, with the reference
 // binding's messages (crates/diffrast-py/src/lib.rs:162-195).
@@ -164,7 +211,8 @@ struct Staged {
     Lease lease;
     const float* dev = nullptr;
 };
-int stage_in(drh_ctx* ctx, Staged& st, uint64_t kind, const float* src, size_t n, bool host, hipStream_t s);
+int stage_in(drh_ctx* ctx, Staged& st, uint64_t kind, const float* src, size_t n, bool host, hipStream_t s,
+             HostStage& hs);
 
 // Device output: the caller's pointer, or a pooled buffer copied back by copy_back.
 struct Out {
@@ -174,10 +222,11 @@ struct Out {
     size_t n = 0;
 };
 int stage_out(drh_ctx* ctx, Out& o, uint64_t kind, float* dst, size_t n, bool host, hipStream_t s);
-int copy_back(Out& o, hipStream_t s);
+int copy_back(Out& o, HostStage& hs);
 
-// With host pointers, DRH_SYNC or DRH_PHASES: waits for the stream.
-int finish(uint32_t flags, hipStream_t s);
+// With host pointers, DRH_SYNC or DRH_PHASES: waits for the stream (and fills the
+// host arrays).
+int finish(uint32_t flags, hipStream_t s, HostStage& hs);
 
 // Host phases of one call under DRH_PHASES (drh_phases_read). lap() waits for
 // the stream and charges the time since the previous lap to `phase`; publish()

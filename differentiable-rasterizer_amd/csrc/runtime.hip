@@ -123,8 +123,7 @@ int wait_stream(hipStream_t s) {
         (void)hipEventDestroy(ev);
         return hip_fail(e, "hipEventRecord");
     }
-    auto deadline = std::chrono::steady_clock::now() + std::chrono::seconds(DRH_WAIT_TIMEOUT_S);
-    int spins = 0;
+    const auto start = std::chrono::steady_clock::now();
     for (;;) {
         e = hipEventQuery(ev);
         if (e == hipSuccess) break;
@@ -132,12 +131,13 @@ int wait_stream(hipStream_t s) {
             (void)hipEventDestroy(ev);
             return hip_fail(e, "device execution");
         }
-        if (std::chrono::steady_clock::now() > deadline) {
+        const auto waited = std::chrono::steady_clock::now() - start;
+        if (waited > std::chrono::seconds(DRH_WAIT_TIMEOUT_S)) {
             (void)hipEventDestroy(ev);
             return fail(DRH_ERR_TIMEOUT, "the GPU did not finish within " + std::to_string(DRH_WAIT_TIMEOUT_S) +
                                              " s; it may be busy with another process (check rocm-smi)");
         }
-        if (++spins > 64) std::this_thread::sleep_for(std::chrono::microseconds(50));
+        if (waited > std::chrono::microseconds(WAIT_SPIN_US)) std::this_thread::sleep_for(std::chrono::microseconds(50));
     }
     (void)hipEventDestroy(ev);
     return DRH_OK;
@@ -159,7 +159,82 @@ int check_shape(drh_ctx* ctx, int64_t B, int64_t T, int64_t H, int64_t W, float 
     return check_sizes(B, T, H, W);
 }
 
-int stage_in(drh_ctx* ctx, Staged& st, uint64_t kind, const float* src, size_t n, bool host, hipStream_t s) {
+HostStage::HostStage(drh_ctx* ctx, hipStream_t s, size_t bytes) : ctx_(ctx), s_(s) {
+    if (bytes == 0) return;
+    size_t want = PINNED_MIN;
+    while (want < bytes && want < PINNED_MAX) want *= 2;
+    {
+        std::lock_guard<std::mutex> g(ctx->mu);
+        for (size_t i = 0; i < ctx->free_pinned.size(); i++)
+            if (ctx->free_pinned[i].bytes == want) {
+                buf_ = ctx->free_pinned[i];
+                ctx->free_pinned.erase(ctx->free_pinned.begin() + (long)i);
+                ctx->pinned_bytes -= want;
+                return;
+            }
+    }
+    // without the buffer the arrays are copied as they are
+    if (hipHostMalloc(reinterpret_cast<void**>(&buf_.ptr), want, hipHostMallocDefault) == hipSuccess)
+        buf_.bytes = want;
+    else
+        buf_ = PinnedBuf{}, (void)hipGetLastError();
+}
+
+HostStage::~HostStage() {
+    if (!buf_.ptr) return;
+    if (pending_) (void)hipStreamSynchronize(s_);  // a call that failed half-way
+    {
+        std::lock_guard<std::mutex> g(ctx_->mu);
+        if (ctx_->pinned_bytes + buf_.bytes <= PINNED_KEEP) {
+            ctx_->free_pinned.push_back(buf_);
+            ctx_->pinned_bytes += buf_.bytes;
+            return;
+        }
+    }
+    (void)hipHostFree(buf_.ptr);
+}
+
+char* HostStage::take(size_t bytes) {
+    const size_t at = (used_ + 255) & ~(size_t)255;
+    if (!buf_.ptr || at > buf_.bytes || bytes > buf_.bytes - at) return nullptr;
+    used_ = at + bytes;
+    return buf_.ptr + at;
+}
+
+int HostStage::in(void* dev, const void* src, size_t bytes) {
+    if (char* p = take(bytes)) {
+        std::memcpy(p, src, bytes);
+        src = p;
+        pending_ = true;
+    }
+    HIP_TRY(hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, s_), "hipMemcpyAsync H2D");
+    return DRH_OK;
+}
+
+int HostStage::out(void* dst, const void* dev, size_t bytes) {
+    void* to = dst;
+    char* const p = nback_ < (int)(sizeof back_ / sizeof back_[0]) ? take(bytes) : nullptr;
+    if (p) {
+        back_[nback_++] = Back{dst, p, bytes};
+        to = p;
+        pending_ = true;
+    }
+    hipError_t e = hipMemcpyAsync(to, dev, bytes, hipMemcpyDeviceToHost, s_);
+    if (e != hipSuccess) return fail(DRH_ERR_READBACK, std::string("hipMemcpyAsync D2H: ") + hipGetErrorString(e));
+    return DRH_OK;
+}
+
+int HostStage::finish() {
+    int rc = wait_stream(s_);
+    if (rc) return rc;
+    pending_ = false;
+    for (int i = 0; i < nback_; i++) std::memcpy(back_[i].dst, back_[i].src, back_[i].bytes);
+    nback_ = 0;
+    return DRH_OK;
+}
+
+int stage_in(drh_ctx* ctx, Staged& st, uint64_t kind, const float* src, size_t n, bool host, hipStream_t s,
+             HostStage& hs) {
     if (n == 0) {
         st.dev = src;
         return DRH_OK;
@@ -170,8 +245,7 @@ int stage_in(drh_ctx* ctx, Staged& st, uint64_t kind, const float* src, size_t n
         return DRH_OK;
     }
     int rc = st.lease.acquire(ctx, kind, n * sizeof(float), s);
-    if (rc) return rc;
-    HIP_TRY(hipMemcpyAsync(st.lease.get<float>(), src, n * sizeof(float), hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
+    if (rc || (rc = hs.in(st.lease.get<float>(), src, n * sizeof(float)))) return rc;
     st.dev = st.lease.get<float>();
     return DRH_OK;
 }
@@ -193,15 +267,14 @@ int stage_out(drh_ctx* ctx, Out& o, uint64_t kind, float* dst, size_t n, bool ho
     return DRH_OK;
 }
 
-int copy_back(Out& o, hipStream_t s) {
+int copy_back(Out& o, HostStage& hs) {
     if (!o.host_dst || o.n == 0) return DRH_OK;
-    hipError_t e = hipMemcpyAsync(o.host_dst, o.dev, o.n * sizeof(float), hipMemcpyDeviceToHost, s);
-    if (e != hipSuccess) return fail(DRH_ERR_READBACK, std::string("hipMemcpyAsync D2H: ") + hipGetErrorString(e));
-    return DRH_OK;
+    return hs.out(o.host_dst, o.dev, o.n * sizeof(float));
 }
 
-int finish(uint32_t flags, hipStream_t s) {
-    if (flags & (DRH_HOST_PTRS | DRH_SYNC | DRH_PHASES)) return wait_stream(s);
+int finish(uint32_t flags, hipStream_t s, HostStage& hs) {
+    if (flags & DRH_HOST_PTRS) return hs.finish();
+    if (flags & (DRH_SYNC | DRH_PHASES)) return wait_stream(s);
     return DRH_OK;
 }
 
@@ -737,6 +810,9 @@ int drh_clear_pool(drh_ctx* ctx) {
     }
     ctx->free_bufs.clear();
     ctx->bytes = 0;
+    for (auto& p : ctx->free_pinned) (void)hipHostFree(p.ptr);
+    ctx->free_pinned.clear();
+    ctx->pinned_bytes = 0;
     return DRH_OK;
 }
 
@@ -797,11 +873,12 @@ int drh_render(drh_ctx* ctx, const float* params, const float* backgrounds, int6
     DeviceGuard dg(ctx->device);
     hipStream_t s = (hipStream_t)stream;
     bool host = flags & DRH_HOST_PTRS;
+    HostStage hs(ctx, s, host ? ((size_t)B * T * NP + (size_t)B * 3 + (size_t)B * H * W * 3) * sizeof(float) + HOST_PAD : 0);
     PhaseClock pc(flags, s);
     Staged p, bg;
     Out img;
-    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s))) return rc;
-    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s))) return rc;
+    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s, hs))) return rc;
     if ((rc = pc.lap(PH_PACK))) return rc;
     if ((rc = stage_out(ctx, img, K_OUT_IMAGES, out_images, (size_t)B * H * W * 3, host, s))) return rc;
     if ((rc = pc.lap(PH_ALLOC))) return rc;
@@ -809,8 +886,8 @@ int drh_render(drh_ctx* ctx, const float* params, const float* backgrounds, int6
                          img.dev, nullptr, nullptr, flags, s)))
         return rc;
     if ((rc = pc.lap(PH_DISPATCH))) return rc;
-    if ((rc = copy_back(img, s))) return rc;
-    if ((rc = finish(flags, s)) || (rc = pc.lap(PH_READBACK))) return rc;
+    if ((rc = copy_back(img, hs))) return rc;
+    if ((rc = finish(flags, s, hs)) || (rc = pc.lap(PH_READBACK))) return rc;
     pc.publish();
     return DRH_OK;
 }
@@ -826,13 +903,15 @@ int drh_fused_loss_backward(drh_ctx* ctx, const float* params, const float* back
     DeviceGuard dg(ctx->device);
     hipStream_t s = (hipStream_t)stream;
     bool host = flags & DRH_HOST_PTRS;
+    HostStage hs(ctx, s,
+                 host ? ((size_t)B * (2 * T * NP + 4) + (size_t)B * H * W * (out_images ? 6 : 3)) * sizeof(float) + HOST_PAD : 0);
     PhaseClock pc(flags, s);
     Staged p, bg, tg;
     Out losses, grads, img;
-    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s))) return rc;
-    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s))) return rc;
+    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s, hs))) return rc;
     if ((rc = pc.lap(PH_PACK))) return rc;
-    if ((rc = stage_in(ctx, tg, K_IN_IMAGES, targets, (size_t)B * H * W * 3, host, s))) return rc;
+    if ((rc = stage_in(ctx, tg, K_IN_IMAGES, targets, (size_t)B * H * W * 3, host, s, hs))) return rc;
     if ((rc = stage_out(ctx, losses, K_OUT_LOSSES, out_losses, (size_t)B, host, s))) return rc;
     if ((rc = stage_out(ctx, grads, K_OUT_GRADS, out_grads, (size_t)B * T * NP, host, s))) return rc;
     if ((rc = stage_out(ctx, img, K_OUT_IMAGES, out_images, (size_t)B * H * W * 3, host, s))) return rc;
@@ -841,8 +920,8 @@ int drh_fused_loss_backward(drh_ctx* ctx, const float* params, const float* back
                          grads.dev, losses.dev, flags, s)))
         return rc;
     if ((rc = pc.lap(PH_DISPATCH))) return rc;
-    if ((rc = copy_back(losses, s)) || (rc = copy_back(grads, s)) || (rc = copy_back(img, s))) return rc;
-    if ((rc = finish(flags, s)) || (rc = pc.lap(PH_READBACK))) return rc;
+    if ((rc = copy_back(losses, hs)) || (rc = copy_back(grads, hs)) || (rc = copy_back(img, hs))) return rc;
+    if ((rc = finish(flags, s, hs)) || (rc = pc.lap(PH_READBACK))) return rc;
     pc.publish();
     return DRH_OK;
 }
@@ -857,21 +936,22 @@ int drh_backward_from_grad(drh_ctx* ctx, const float* params, const float* backg
     DeviceGuard dg(ctx->device);
     hipStream_t s = (hipStream_t)stream;
     bool host = flags & DRH_HOST_PTRS;
+    HostStage hs(ctx, s, host ? ((size_t)B * (2 * T * NP + 3) + (size_t)B * H * W * 3) * sizeof(float) + HOST_PAD : 0);
     PhaseClock pc(flags, s);
     Staged p, bg, gi;
     Out grads;
-    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s))) return rc;
-    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s))) return rc;
+    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s, hs))) return rc;
     if ((rc = pc.lap(PH_PACK))) return rc;
-    if ((rc = stage_in(ctx, gi, K_IN_IMAGES, grad_images, (size_t)B * H * W * 3, host, s))) return rc;
+    if ((rc = stage_in(ctx, gi, K_IN_IMAGES, grad_images, (size_t)B * H * W * 3, host, s, hs))) return rc;
     if ((rc = stage_out(ctx, grads, K_OUT_GRADS, out_grads, (size_t)B * T * NP, host, s))) return rc;
     if ((rc = pc.lap(PH_ALLOC))) return rc;
     if ((rc = run_raster(ctx, drh::MODE_GRAD_IN, p.dev, bg.dev, gi.dev, (int)B, (int)T, (int)H, (int)W, sigma,
                          nullptr, grads.dev, nullptr, flags, s)))
         return rc;
     if ((rc = pc.lap(PH_DISPATCH))) return rc;
-    if ((rc = copy_back(grads, s))) return rc;
-    if ((rc = finish(flags, s)) || (rc = pc.lap(PH_READBACK))) return rc;
+    if ((rc = copy_back(grads, hs))) return rc;
+    if ((rc = finish(flags, s, hs)) || (rc = pc.lap(PH_READBACK))) return rc;
     pc.publish();
     return DRH_OK;
 }
@@ -896,10 +976,11 @@ int drh_render_record(drh_ctx* ctx, const float* params, const float* background
     DeviceGuard dg(ctx->device);
     hipStream_t s = (hipStream_t)stream;
     const bool host = flags & DRH_HOST_PTRS;
+    HostStage hs(ctx, s, host ? ((size_t)B * (T * NP + 3) + (size_t)B * H * W * 3) * sizeof(float) + HOST_PAD : 0);
     Staged p, bg;
     Out img;
-    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s))) return rc;
-    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s))) return rc;
+    if ((rc = stage_in(ctx, p, K_IN_PARAMS, params, (size_t)B * T * NP, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, bg, K_IN_BG, backgrounds, (size_t)B * 3, host, s, hs))) return rc;
     if ((rc = stage_out(ctx, img, K_OUT_IMAGES, out_images, (size_t)B * H * W * 3, host, s))) return rc;
     char* base = static_cast<char*>(record);
     drh::RasterArgs a{};
@@ -933,8 +1014,8 @@ int drh_render_record(drh_ctx* ctx, const float* params, const float* background
         KernelTimer kt(ctx, TK_RASTER);
         HIP_TRY(drh::launch_forward(drh::MODE_RECORD, !(flags & DRH_EXACT_MATH), a, s), "forward_kernel launch");
     }
-    if ((rc = copy_back(img, s))) return rc;
-    return finish(flags, s);
+    if ((rc = copy_back(img, hs))) return rc;
+    return finish(flags, s, hs);
 }
 
 int drh_backward_recorded(drh_ctx* ctx, const void* record, uint64_t record_bytes, const float* grad_images,
@@ -951,10 +1032,11 @@ int drh_backward_recorded(drh_ctx* ctx, const void* record, uint64_t record_byte
     if ((rc = check_record_head(ctx, record, make_head(B, T, H, W, sigma, flags), s))) return rc;
     const bool host = flags & DRH_HOST_PTRS;
     const bool det = (flags & DRH_DETERMINISTIC) != 0;
+    HostStage hs(ctx, s, host ? ((size_t)B * T * NP + (size_t)B * H * W * 3) * sizeof(float) + HOST_PAD : 0);
     Staged gi;
     Out grads;
     Lease partials;
-    if ((rc = stage_in(ctx, gi, K_IN_IMAGES, grad_images, (size_t)B * H * W * 3, host, s))) return rc;
+    if ((rc = stage_in(ctx, gi, K_IN_IMAGES, grad_images, (size_t)B * H * W * 3, host, s, hs))) return rc;
     if ((rc = stage_out(ctx, grads, K_OUT_GRADS, out_grads, (size_t)B * T * NP, host, s))) return rc;
     const dim3 grid = drh::raster_grid((int)B, (int)W, (int)H);
     const int nblk = (int)(grid.x * grid.y);
@@ -994,8 +1076,8 @@ int drh_backward_recorded(drh_ctx* ctx, const void* record, uint64_t record_byte
         HIP_TRY(drh::launch_reduce(a.partials, nullptr, a.B, nblk, 1, a.T, 3.0 * a.H * (double)a.W, grads.dev, nullptr, s),
                 "reduce_partials launch");
     }
-    if ((rc = copy_back(grads, s))) return rc;
-    return finish(flags, s);
+    if ((rc = copy_back(grads, hs))) return rc;
+    return finish(flags, s, hs);
 }
 
 int drh_adam_project_step(drh_ctx* ctx, float* params, const float* grads, float* m, float* v, const float* lr,
@@ -1010,16 +1092,17 @@ int drh_adam_project_step(drh_ctx* ctx, float* params, const float* grads, float
     DeviceGuard dg(ctx->device);
     hipStream_t s = (hipStream_t)stream;
     bool host = flags & DRH_HOST_PTRS;
+    HostStage hs(ctx, s, host ? 8 * (size_t)n * sizeof(float) + HOST_PAD : 0);
     // optim.rs:309-310 bias corrections
     float bc1 = 1.0f - powi_f32(beta1, (int32_t)step);
     float bc2 = 1.0f - powi_f32(beta2, (int32_t)step);
     int rc;
     Staged g, l, pin, min_, vin;
-    if ((rc = stage_in(ctx, g, K_IN_IMAGES, grads, (size_t)n, host, s))) return rc;
-    if ((rc = stage_in(ctx, l, K_IN_BG, lr, (size_t)n, host, s))) return rc;
-    if ((rc = stage_in(ctx, pin, K_IN_PARAMS, params, (size_t)n, host, s))) return rc;
-    if ((rc = stage_in(ctx, min_, K_FIT_F32, m, (size_t)n, host, s))) return rc;
-    if ((rc = stage_in(ctx, vin, K_OUT_GRADS, v, (size_t)n, host, s))) return rc;
+    if ((rc = stage_in(ctx, g, K_IN_IMAGES, grads, (size_t)n, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, l, K_IN_BG, lr, (size_t)n, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, pin, K_IN_PARAMS, params, (size_t)n, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, min_, K_FIT_F32, m, (size_t)n, host, s, hs))) return rc;
+    if ((rc = stage_in(ctx, vin, K_OUT_GRADS, v, (size_t)n, host, s, hs))) return rc;
     float* dp = const_cast<float*>(pin.dev);
     float* dm = const_cast<float*>(min_.dev);
     float* dv = const_cast<float*>(vin.dev);
@@ -1029,11 +1112,10 @@ int drh_adam_project_step(drh_ctx* ctx, float* params, const float* grads, float
                 "adam_project launch");
     }
     if (host) {
-        HIP_TRY(hipMemcpyAsync(params, dp, n * sizeof(float), hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
-        HIP_TRY(hipMemcpyAsync(m, dm, n * sizeof(float), hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
-        HIP_TRY(hipMemcpyAsync(v, dv, n * sizeof(float), hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
+        const size_t bytes = (size_t)n * sizeof(float);
+        if ((rc = hs.out(params, dp, bytes)) || (rc = hs.out(m, dm, bytes)) || (rc = hs.out(v, dv, bytes))) return rc;
     }
-    return finish(flags, s);
+    return finish(flags, s, hs);
 }
 
 int drh_encode_srgb(drh_ctx* ctx, const float* values, int64_t n, uint8_t* out, void* stream, uint32_t flags) {
@@ -1044,9 +1126,10 @@ int drh_encode_srgb(drh_ctx* ctx, const float* values, int64_t n, uint8_t* out, 
     DeviceGuard dg(ctx->device);
     hipStream_t s = (hipStream_t)stream;
     const bool host = flags & DRH_HOST_PTRS;
+    HostStage hs(ctx, s, host ? (size_t)n * 5 + HOST_PAD : 0);
     Staged in;
     int rc;
-    if ((rc = stage_in(ctx, in, K_SRGB_F32, values, (size_t)n, host, s))) return rc;
+    if ((rc = stage_in(ctx, in, K_SRGB_F32, values, (size_t)n, host, s, hs))) return rc;
     Lease ob;
     uint8_t* dout = out;
     if (host) {
@@ -1054,11 +1137,8 @@ int drh_encode_srgb(drh_ctx* ctx, const float* values, int64_t n, uint8_t* out, 
         dout = ob.get<uint8_t>();
     }
     HIP_TRY(drh::launch_encode_srgb(in.dev, n, dout, srgb_tables().encode, s), "encode_srgb launch");
-    if (host) {
-        hipError_t e = hipMemcpyAsync(out, dout, (size_t)n, hipMemcpyDeviceToHost, s);
-        if (e != hipSuccess) return fail(DRH_ERR_READBACK, std::string("hipMemcpyAsync D2H: ") + hipGetErrorString(e));
-    }
-    return finish(flags, s);
+    if (host && (rc = hs.out(out, dout, (size_t)n))) return rc;
+    return finish(flags, s, hs);
 }
 
 int drh_decode_srgb(drh_ctx* ctx, const uint8_t* bytes, int64_t n, float* out, void* stream, uint32_t flags) {
@@ -1069,19 +1149,19 @@ int drh_decode_srgb(drh_ctx* ctx, const uint8_t* bytes, int64_t n, float* out, v
     DeviceGuard dg(ctx->device);
     hipStream_t s = (hipStream_t)stream;
     const bool host = flags & DRH_HOST_PTRS;
+    HostStage hs(ctx, s, host ? (size_t)n * 5 + HOST_PAD : 0);
     Lease ib;
     const uint8_t* din = bytes;
     int rc;
     if (host) {
-        if ((rc = ib.acquire(ctx, K_SRGB_U8, (size_t)n, s))) return rc;
-        HIP_TRY(hipMemcpyAsync(ib.get<uint8_t>(), bytes, (size_t)n, hipMemcpyHostToDevice, s), "hipMemcpyAsync H2D");
+        if ((rc = ib.acquire(ctx, K_SRGB_U8, (size_t)n, s)) || (rc = hs.in(ib.get<uint8_t>(), bytes, (size_t)n))) return rc;
         din = ib.get<uint8_t>();
     }
     Out o;
     if ((rc = stage_out(ctx, o, K_SRGB_F32, out, (size_t)n, host, s))) return rc;
     HIP_TRY(drh::launch_decode_srgb(din, n, o.dev, srgb_tables().values, s), "decode_srgb launch");
-    if ((rc = copy_back(o, s))) return rc;
-    return finish(flags, s);
+    if ((rc = copy_back(o, hs))) return rc;
+    return finish(flags, s, hs);
 }
 
 }  // extern "C"
