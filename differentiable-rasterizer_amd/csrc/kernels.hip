@@ -3,7 +3,7 @@
 // Semantics follow the reference CPU path (crates/diffrast/src/raster.rs,
 // grad.rs, optim.rs, fit.rs); the work decomposition is this file's own:
 //
-//   setup_records : one thread per (scene, triangle). Computes the padded
+//   setup_records : four threads per (scene, triangle). Computes the padded
 //                   integer bounding box exactly as raster.rs:144-168 does,
 //                   the edge vectors and the data for a conservative
 //                   far-outside / deep-inside classification.
@@ -235,33 +235,21 @@ __device__ inline void reach_rows(const Reach r, const OrderArgs& o, int j, int 
     }
 }
 
-// The record of triangle i (scene-major index) from its parameters p.
-__device__ inline void setup_from(const float* __restrict__ p, size_t i, int W, int H, float sigma, int setup_mode,
-                                  float* __restrict__ rec) {
-    float* r = rec + i * REC;
-
+// A quarter of the record of triangle i (scene-major index) from its parameters
+// p: part 0-2 writes what belongs to the edge from vertex `part` to the next,
+// part 3 the rest. The quarters of a triangle run on neighbouring lanes (or on
+// waves of their own). A record on one lane was a serial chain of three edges'
+// roots and divisions, on waves that have a SIMD to themselves, and of 19 stores
+// of 64 cache lines each: B=1 383x509 T=400 whole calls 39.0 -> 38.5 us in four
+// runs of about that difference, a fit's iterations 21.1 -> 20.9 with its other
+// kernel's stop test off the path; beside an order or row lists, which take
+// longer than the records, the same time, as with 200 000 triangles.
+__device__ inline void setup_part(const float* __restrict__ p, size_t i, int part, int W, int H, float sigma,
+                                  int setup_mode, float* __restrict__ rec) {
+    float* const r = rec + i * REC;
     float v[6];
     for (int j = 0; j < 6; j++) v[j] = p[j];
-    float alpha = rust_clamp(p[9], 0.0f, 1.0f);
-
-    bool finite = true;
-    for (int j = 0; j < 6; j++) finite = finite && isfinite(v[j]);
-    const PixBox box = pix_box(v, W, H, sigma);
-    const bool taped = box.any() && drawn(alpha, SETUP_TAPE);
-    const bool live = box.any() && drawn(alpha, setup_mode);
-
-    // Edges in the reference's order: (v0,v1), (v1,v2), (v2,v0); e = b - a.
-    float e[6];
-    for (int j = 0; j < 3; j++) {
-        int a = j, b = (j + 1) % 3;
-        e[2 * j] = v[2 * b] - v[2 * a];
-        e[2 * j + 1] = v[2 * b + 1] - v[2 * a + 1];
-    }
-    float len2[3], rlen2[3];
-    for (int j = 0; j < 3; j++) {
-        len2[j] = e[2 * j] * e[2 * j] + e[2 * j + 1] * e[2 * j + 1];
-        rlen2[j] = (len2[j] <= 1e-20f) ? 0.0f : 1.0f / len2[j];
-    }
+    const float alpha = rust_clamp(p[9], 0.0f, 1.0f);
 
     // Conservative classification data. With s the orientation sign, the
     // outward distance of a point to edge line j is l_j = pt.n_j - off_j, and
@@ -269,23 +257,62 @@ __device__ inline void setup_from(const float* __restrict__ p, size_t i, int W, 
     // or the distance to the boundary from above (inside). It is only trusted
     // for a triangle whose area is large against the rounding of the
     // reference's cross products, so that its inside test cannot flip.
+    bool finite = true;
     float m = 0.0f;
-    for (int j = 0; j < 6; j++) m = fmaxf(m, fabsf(v[j]));
-    float area2 = e[0] * (v[5] - v[1]) - e[1] * (v[4] - v[0]);
-    float slack = 1e-5f * (1.0f + m);
-    bool fast = finite && (alpha == alpha) && m <= 1e4f &&
-                fabsf(area2) >= 1e-4f * (1.0f + m) * (1.0f + m);
-    float s = area2 >= 0.0f ? 1.0f : -1.0f;
-    float n[6], off[3];
-    for (int j = 0; j < 3; j++) {
-        float len = sqrtf(len2[j]);
-        float inv = (fast && len > 0.0f) ? s / len : 0.0f;
-        n[2 * j] = e[2 * j + 1] * inv;
-        n[2 * j + 1] = -e[2 * j] * inv;
-        off[j] = v[2 * j] * n[2 * j] + v[2 * j + 1] * n[2 * j + 1];
+    for (int j = 0; j < 6; j++) {
+        finite = finite && isfinite(v[j]);
+        m = fmaxf(m, fabsf(v[j]));
     }
-    float sig = fmaxf(sigma, 1e-8f);
+    const float area2 = (v[2] - v[0]) * (v[5] - v[1]) - (v[3] - v[1]) * (v[4] - v[0]);
+    const bool fast = finite && (alpha == alpha) && m <= 1e4f &&
+                      fabsf(area2) >= 1e-4f * (1.0f + m) * (1.0f + m);
+    const float s = area2 >= 0.0f ? 1.0f : -1.0f;
 
+    if (part < 3) {
+        // Edges in the reference's order: (v0,v1), (v1,v2), (v2,v0); e = b - a.
+        const float ax = part == 0 ? v[0] : (part == 1 ? v[2] : v[4]), bx = part == 0 ? v[2] : (part == 1 ? v[4] : v[0]);
+        const float ay = part == 0 ? v[1] : (part == 1 ? v[3] : v[5]), by = part == 0 ? v[3] : (part == 1 ? v[5] : v[1]);
+        const float ex = bx - ax, ey = by - ay;
+        const float len2 = ex * ex + ey * ey;
+        const float rlen2 = (len2 <= 1e-20f) ? 0.0f : 1.0f / len2;
+        const float len = sqrtf(len2);
+        const bool unit = fast && len > 0.0f;
+        const float inv = unit ? 1.0f / len : 0.0f, ninv = unit ? s * inv : 0.0f;
+        const float nx = ey * ninv, ny = -ex * ninv;
+        // Along-edge coordinate s_j = p . d_j - a_j . d_j, with d_j the unit edge
+        // direction: with the edge-line distance it bounds the distance of a whole
+        // tile to each edge segment when the tile's list is built.
+        const float dx = ex * inv, dy = ey * inv;
+        float* const re = r + R_E + 2 * part;
+        re[0] = ex;
+        re[1] = ey;
+        r[R_LEN2 + part] = len2;
+        r[R_RLEN2 + part] = rlen2;
+        float* const rn = r + R_N + 2 * part;
+        rn[0] = nx;
+        rn[1] = ny;
+        r[R_OFF + part] = ax * nx + ay * ny;
+        float* const rd = r + R_D + 2 * part;
+        rd[0] = dx;
+        rd[1] = dy;
+        r[R_SOFF + part] = ax * dx + ay * dy;
+        r[R_LEN + part] = len;
+        float* const eb = r + R_EB + 8 * part;
+        eb[0] = ax;
+        eb[1] = ay;
+        eb[2] = ex;
+        eb[3] = ey;
+        eb[4] = len2;
+        eb[5] = rlen2;
+        eb[6] = s;  // F_CCW as a factor: c eb[6] >= 0 inside
+        eb[7] = 0.0f;
+        return;
+    }
+    const PixBox box = pix_box(v, W, H, sigma);
+    const bool taped = box.any() && drawn(alpha, SETUP_TAPE);
+    const bool live = box.any() && drawn(alpha, setup_mode);
+    const float slack = 1e-5f * (1.0f + m);
+    const float sig = fmaxf(sigma, 1e-8f);
     for (int j = 0; j < 6; j++) r[R_V + j] = v[j];
     for (int j = 0; j < 3; j++) r[R_C + j] = p[6 + j];
     r[R_A] = alpha;
@@ -294,55 +321,20 @@ __device__ inline void setup_from(const float* __restrict__ p, size_t i, int W, 
     ri[R_BOX + 1] = live ? box.y0 : 0;
     ri[R_BOX + 2] = live ? box.x1 : 0;
     ri[R_BOX + 3] = live ? box.y1 : 0;
-    bool active = p[9] > 0.0f && p[9] < 1.0f;  // grad.rs:145
+    const bool active = p[9] > 0.0f && p[9] < 1.0f;  // grad.rs:145
     ri[R_FLAGS] = (live ? F_LIVE : 0) | (active ? F_ACTIVE : 0) | (fast && live ? F_FAST : 0) |
                   (area2 >= 0.0f ? F_CCW : 0) | (taped ? F_TAPE : 0);
     r[R_SPARE] = 0.0f;
-    for (int j = 0; j < 6; j++) r[R_E + j] = e[j];
-    for (int j = 0; j < 3; j++) r[R_LEN2 + j] = len2[j];
-    for (int j = 0; j < 3; j++) r[R_RLEN2 + j] = rlen2[j];
-    for (int j = 0; j < 6; j++) r[R_N + j] = n[j];
-    for (int j = 0; j < 3; j++) r[R_OFF + j] = off[j];
     // Far outside: at a true distance d >= sigma (ln(alpha / MIN_WEIGHT) + 0.05)
     // the weight is alpha * sigmoid(-d / sigma) < alpha e^(-d / sigma)
     // <= 0.951 MIN_WEIGHT, which the f32 rounding of the reference's sigmoid
     // and product (a few ulp) cannot lift to MIN_WEIGHT: it skips the pair too.
     // Deep inside: at a distance to the edge above 17 sigma, exp(-x) < 4.2e-8
     // < 2^-24, so the reference's 1 / (1 + exp(-x)) rounds to exactly 1.0f.
-    float xfar = fmaxf(logf(alpha * (1.0f / MIN_WEIGHT)) + 0.05f, 0.0f);
+    const float xfar = fmaxf(logf(alpha * (1.0f / MIN_WEIGHT)) + 0.05f, 0.0f);
     r[R_FAR] = (xfar == xfar ? xfar : 0.0f) * sig + slack;
     r[R_DEEP] = -(17.0f * sig + slack);
     r[R_SLACK] = slack;
-    // Along-edge coordinate s_j = p . d_j - a_j . d_j, with d_j the unit edge
-    // direction: with the edge-line distance it bounds the distance of a whole
-    // tile to each edge segment when the tile's list is built.
-    for (int j = 0; j < 3; j++) {
-        float len = sqrtf(len2[j]);
-        float inv = (fast && len > 0.0f) ? 1.0f / len : 0.0f;
-        float dx = e[2 * j] * inv, dy = e[2 * j + 1] * inv;
-        r[R_D + 2 * j] = dx;
-        r[R_D + 2 * j + 1] = dy;
-        r[R_SOFF + j] = v[2 * j] * dx + v[2 * j + 1] * dy;
-        r[R_LEN + j] = len;
-        float* eb = r + R_EB + 8 * j;
-        eb[0] = v[2 * j];
-        eb[1] = v[2 * j + 1];
-        eb[2] = e[2 * j];
-        eb[3] = e[2 * j + 1];
-        eb[4] = len2[j];
-        eb[5] = rlen2[j];
-        eb[6] = area2 >= 0.0f ? 1.0f : -1.0f;  // F_CCW as a factor: c eb[6] >= 0 inside
-        eb[7] = 0.0f;
-    }
-}
-
-// Setup of triangle i: its record from params[i * NP ...].
-__device__ inline void setup_one(const float* __restrict__ params, size_t i, int W, int H, float sigma,
-                                 int setup_mode, float* __restrict__ rec, float* __restrict__ zero_grads) {
-    // The backward kernel adds into the gradients: they start at zero.
-    if (zero_grads)
-        for (int j = 0; j < NP; j++) zero_grads[i * NP + j] = 0.0f;
-    setup_from(params + i * NP, i, W, H, sigma, setup_mode, rec);
 }
 
 // The raster kernels' block order, heaviest first. A block's time follows its
@@ -357,9 +349,8 @@ __device__ inline void setup_one(const float* __restrict__ params, size_t i, int
 // slot i to rank i / B of scene i % B, so the heaviest blocks of every scene go
 // first. Nothing crosses workgroups: a device-wide hand-off would cost more
 // than the order saves. The records then come from workgroups of
-// SETUP_REC_PER triangles: a wave stores each record as 19 16-byte pieces at a
-// 304-byte stride, a cache line per lane and store, and one CU issues about one
-// line per cycle, so 512 records on one CU took ~6 us and on four ~1.5.
+// SETUP_REC_PER triangles: one CU issues the stores' cache lines at about one per
+// cycle, so 512 records on one CU took ~6 us and on four ~1.5.
 constexpr int SETUP_THREADS = 1024, ORD_BUCKETS = 1024, ORD_REACH = 512, SETUP_REC_PER = 128;
 static_assert(ORD_BUCKETS == 16 * 64 && SETUP_THREADS % 64 == 0 && ORD_REACH <= SETUP_THREADS,
               "order workgroup shape: 16 buckets per lane of one wave");
@@ -505,8 +496,8 @@ __device__ inline void list_row(const float* __restrict__ params, int b, int y, 
 //    so that the order workgroups, the longest, are dispatched before the rest;
 //  with ra.rows, ra.parts that list its tile rows, a team of waves each;
 //  the rest the records of triangles [x per, x per + per) (and every nx per
-//    after, nx the records workgroups per scene), per = SETUP_REC_PER beside an
-//    order or rows, else the workgroup's threads.
+//    after, nx the records workgroups per scene), per a quarter of the workgroup's
+//    threads (setup_part), at most SETUP_REC_PER.
 __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __restrict__ params, int T, int W,
                                                                int H, float sigma, int setup_mode,
                                                                float* __restrict__ rec, float* __restrict__ zero_grads,
@@ -519,7 +510,7 @@ __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __re
     __shared__ __attribute__((aligned(16))) int hist[ORD_BUCKETS];
     if (halt && *halt >= 0) return;
     const int b = blockIdx.x, part = blockIdx.y, pitch = o.gx + 1;
-    const int per = min((int)blockDim.x, SETUP_REC_PER);  // records per workgroup
+    const int per = min((int)blockDim.x / 4, SETUP_REC_PER);  // records per workgroup
     if (head && b == 0 && part == 0 && threadIdx.x == 0) *head = head_val;
     // A record kept for a later backward holds its own copy of the backgrounds.
     if (bg_dst && part == 0 && threadIdx.x < 3) bg_dst[b * 3 + threadIdx.x] = bg_src[b * 3 + threadIdx.x];
@@ -541,9 +532,15 @@ __global__ __launch_bounds__(SETUP_THREADS) void setup_records(const float* __re
         x -= ra.parts;
         // grid rows are capped at 65535: a records workgroup strides over the rest
         const int nparts = (int)gridDim.y - (o.perm ? 1 : 0) - ra.parts;
-        if ((int)threadIdx.x < per)
-            for (int k = x * per + (int)threadIdx.x; k < T; k += nparts * per)
-                setup_one(params, (size_t)b * T + k, W, H, sigma, setup_mode, rec, zero_grads);
+        for (int k0 = x * per; k0 < T; k0 += nparts * per) {
+            const int k1 = min(k0 + per, T), t = (int)threadIdx.x;
+            // the backward kernel adds into the gradients: they start at zero
+            if (zero_grads)
+                for (int j = k0 * NP + t; j < k1 * NP; j += (int)blockDim.x) zero_grads[(size_t)b * T * NP + j] = 0.0f;
+            const int k = k0 + (t >> 2);
+            if (k < k1)
+                setup_part(params + ((size_t)b * T + k) * NP, (size_t)b * T + k, t & 3, W, H, sigma, setup_mode, rec);
+        }
         return;
     }
     // Triangles in batches of up to ORD_REACH: each one's Reach made by one
@@ -2251,9 +2248,10 @@ __global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const f
     static_assert(2 * SEG_BLOCK <= 64, "a block's entries are held one per lane");
     __shared__ int count[S];
     extern __shared__ __attribute__((aligned(16))) float seg_lds[];
-    if (a.halt && *a.halt >= 0) return;
+    // a stopped fit: tested once the list is made, which need not wait for the load
+    const int halted = a.halt ? *a.halt : -1;
     if (MODE == MODE_LOSS && !DET && a.loss_tail && (int)blockIdx.x >= (int)gridDim.x - a.B) {
-        if (threadIdx.x < 64) loss_tail(a, (int)blockIdx.x - ((int)gridDim.x - a.B));
+        if (threadIdx.x < 64 && halted < 0) loss_tail(a, (int)blockIdx.x - ((int)gridDim.x - a.B));
         return;
     }
     const int W = a.W, H = a.H, T = a.T, tpad = seg_tpad(T);
@@ -2294,6 +2292,7 @@ __global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const f
         }
         if (lane == 0) count[s] = n;
     }
+    if (halted >= 0) return;
     __syncthreads();
     int N = 0, first = 0;  // entries of the tile, and before this wave's
     for (int q = 0; q < S; q++) {
@@ -2689,9 +2688,9 @@ __global__ __launch_bounds__(RED_WAVES * 64) void fit_step(const float* __restri
         // setup_records would make them from the updated parameters (handed
         // over in LDS instead of read back)
         __syncthreads();
-        const int k = blockIdx.x * FIT_TRIS + (int)threadIdx.x;
-        if ((int)threadIdx.x < FIT_TRIS && k < T)
-            setup_from(newp + threadIdx.x * NP, (size_t)k, ft.W, ft.H, ft.sigma_next, SETUP_TAPE, ft.rec);
+        const int k = blockIdx.x * FIT_TRIS + lane;
+        if (wave < 4 && lane < FIT_TRIS && k < T)  // a wave for each part of the records
+            setup_part(newp + lane * NP, (size_t)k, wave, ft.W, ft.H, ft.sigma_next, SETUP_TAPE, ft.rec);
     }
 }
 
@@ -2805,7 +2804,7 @@ hipError_t launch_setup(const float* params, int B, int T, int W, int H, float s
     // whole team per row where one wave would take several rounds of passes: B=1
     // 512x512 T=1024 setup 9.4 -> 5.3 us); with one, a workgroup per scene makes it
     const int n = o.perm ? SETUP_THREADS : (rows.rows && T > 64 * ROW_PASSES ? 64 * ROW_TEAM : 64);
-    const int per = min(n, SETUP_REC_PER);  // records per workgroup (setup_records' `per`)
+    const int per = min(n / 4, SETUP_REC_PER);  // records per workgroup (setup_records' `per`)
     RowArgs ra = rows;
     const int teams = n / 64 / min(n / 64, ROW_TEAM);  // rows a workgroup lists at a time
     ra.parts = rows.rows ? min((rows.gy + teams - 1) / teams, 16384) : 0;
