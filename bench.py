@@ -13,7 +13,7 @@ evaluations per second, ms per batch, the dominant kernel's roofline position
 (fused_tile_kernel: its algorithmic FLOP per launch over its event-timed average
 duration, against the FP32 vector peak; under "two_kernel_path" the same step
 with forward_kernel and backward_kernel, DRH_UNFUSED=1, and their rooflines;
-configurations that take the two kernels report them directly), the CPU
+a configuration that takes the two kernels would report them directly), the CPU
 baseline (the C oracle, one thread per scene, on this host's cores), and under
 "configs" the same measurements for every benchmark workload: c0 (B=1 64x64 T=32), c1 (B=16 128x128 T=128), c2 (the
 headline), c3 (B=8 256x256 T=512 small triangles) and c4 (the 800-iteration
@@ -136,11 +136,12 @@ def time_fused(torch, ctx, cfg, p, bg, targets, steps, warmup, dev):
 
 def fused_kernel_name(B, H, W, T, deterministic=False):
     """The kernel the library's fused gradient path takes for this shape: the
-    segmented kernel for grids of at most 2048 8x8 tiles with 16 to 160
-    triangles (runtime.h: use_segments), else the one-wave tile kernel (the
-    four-wave block kernel with fixed-order sums)."""
+    segmented kernel for 16 to 1024 triangles on grids of at most 2048 8x8 tiles
+    (below 6144 for a batch without fixed-order sums; runtime.h: segment_waves),
+    else the one-wave tile kernel (the four-wave block kernel with fixed-order
+    sums)."""
     tiles = B * ((W + 15) // 16) * ((H + 15) // 16) * 4
-    if 16 <= T <= 160 and tiles <= 2048:
+    if 16 <= T <= 1024 and (tiles <= 2048 or (B > 1 and not deterministic and tiles < 6144)):
         return "fused_seg_kernel" + (" (fixed order)" if deterministic else "")
     return "fused_kernel (fixed order)" if deterministic else "fused_tile_kernel"
 
