@@ -80,6 +80,7 @@ struct PoolBuf {
 struct PinnedBuf {
     char* ptr = nullptr;
     size_t bytes = 0;
+    hipEvent_t ev = nullptr;  // of a parked buffer: recorded behind the copies that use it
 };
 
 enum TimedKernel : int { TK_SETUP = 0, TK_RASTER, TK_REDUCE, TK_ADAM, TK_BACKWARD, TK_COUNT };
@@ -112,6 +113,10 @@ struct drh_ctx {
     std::unordered_map<const void*, drh::RecordHead> records;
     std::vector<drh_rt::PinnedBuf> free_pinned;  // at most PINNED_KEEP bytes, freed by drh_clear_pool
     size_t pinned_bytes = 0;
+    // Buffers of calls that gave up waiting: queued copies may still use them.
+    // They come back once their event is done.
+    std::vector<drh_rt::PinnedBuf> parked_pinned;
+    size_t parked_bytes = 0;
 };
 
 namespace drh_rt {
@@ -171,7 +176,10 @@ int wait_stream(hipStream_t s);
 // most) are copied as they are. in() may be followed by changes to the caller's
 // array at once; out()'s arrays hold their values once finish() has waited for
 // the stream. The buffer goes back to the context only when nothing queued uses
-// it: after finish(), or else after a wait in the destructor.
+// it: after finish(), or (a call that failed half-way) after a bounded wait in the
+// destructor. A wait that times out parks it in the context instead, and the call
+// returns: a later call takes it back once the copies are done. With PINNED_KEEP
+// bytes parked the context stages no more.
 constexpr size_t PINNED_MIN = 1ull << 20, PINNED_MAX = 16ull << 20, PINNED_KEEP = 64ull << 20;
 class HostStage {
   public:
@@ -186,6 +194,7 @@ class HostStage {
 
   private:
     char* take(size_t bytes);
+    void park();
     struct Back {
         void* dst;
         const char* src;
@@ -195,11 +204,16 @@ class HostStage {
     hipStream_t s_;
     PinnedBuf buf_;
     size_t used_ = 0;
-    bool pending_ = false;
+    bool pending_ = false;   // queued copies may use the buffer
+    bool gave_up_ = false;   // finish() could not wait for them
     Back back_[4];
     int nback_ = 0;
 };
 constexpr size_t HOST_PAD = 8 * 256;  // the arrays' alignment in a HostStage's buffer
+
+// Parked buffers whose copies are done go to the free ones (within PINNED_KEEP)
+// or are freed. The caller holds ctx->mu.
+void reclaim_parked(drh_ctx* ctx);
 
 // Argument checks shared by the raster entry points, with the reference
 // binding's messages (crates/diffrast-py/src/lib.rs:162-195).

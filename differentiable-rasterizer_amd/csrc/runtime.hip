@@ -159,12 +159,34 @@ int check_shape(drh_ctx* ctx, int64_t B, int64_t T, int64_t H, int64_t W, float 
     return check_sizes(B, T, H, W);
 }
 
+void reclaim_parked(drh_ctx* ctx) {
+    for (size_t i = 0; i < ctx->parked_pinned.size();) {
+        PinnedBuf b = ctx->parked_pinned[i];
+        if (hipEventQuery(b.ev) != hipSuccess) {
+            i++;
+            continue;
+        }
+        ctx->parked_pinned.erase(ctx->parked_pinned.begin() + (long)i);
+        ctx->parked_bytes -= b.bytes;
+        (void)hipEventDestroy(b.ev);
+        b.ev = nullptr;
+        if (ctx->pinned_bytes + b.bytes <= PINNED_KEEP) {
+            ctx->free_pinned.push_back(b);
+            ctx->pinned_bytes += b.bytes;
+        } else {
+            (void)hipHostFree(b.ptr);
+        }
+    }
+}
+
 HostStage::HostStage(drh_ctx* ctx, hipStream_t s, size_t bytes) : ctx_(ctx), s_(s) {
     if (bytes == 0) return;
     size_t want = PINNED_MIN;
     while (want < bytes && want < PINNED_MAX) want *= 2;
     {
         std::lock_guard<std::mutex> g(ctx->mu);
+        if (!ctx->parked_pinned.empty()) reclaim_parked(ctx);
+        if (ctx->parked_bytes >= PINNED_KEEP) return;
         for (size_t i = 0; i < ctx->free_pinned.size(); i++)
             if (ctx->free_pinned[i].bytes == want) {
                 buf_ = ctx->free_pinned[i];
@@ -182,7 +204,15 @@ HostStage::HostStage(drh_ctx* ctx, hipStream_t s, size_t bytes) : ctx_(ctx), s_(
 
 HostStage::~HostStage() {
     if (!buf_.ptr) return;
-    if (pending_) (void)hipStreamSynchronize(s_);  // a call that failed half-way
+    if (pending_ && !gave_up_) {  // a call that failed half-way: its error stays the thread's last one
+        const std::string err = last_error_text();
+        pending_ = wait_stream(s_) != DRH_OK;
+        g_err = err;
+    }
+    if (pending_) {
+        park();
+        return;
+    }
     {
         std::lock_guard<std::mutex> g(ctx_->mu);
         if (ctx_->pinned_bytes + buf_.bytes <= PINNED_KEEP) {
@@ -192,6 +222,19 @@ HostStage::~HostStage() {
         }
     }
     (void)hipHostFree(buf_.ptr);
+}
+
+// Never waits. Where no event can be recorded nothing tells when the copies are
+// done: the buffer is given up.
+void HostStage::park() {
+    if (hipEventCreateWithFlags(&buf_.ev, hipEventDisableTiming) != hipSuccess) return;
+    if (hipEventRecord(buf_.ev, s_) != hipSuccess) {
+        (void)hipEventDestroy(buf_.ev);
+        return;
+    }
+    std::lock_guard<std::mutex> g(ctx_->mu);
+    ctx_->parked_pinned.push_back(buf_);
+    ctx_->parked_bytes += buf_.bytes;
 }
 
 char* HostStage::take(size_t bytes) {
@@ -226,6 +269,7 @@ int HostStage::out(void* dst, const void* dev, size_t bytes) {
 
 int HostStage::finish() {
     int rc = wait_stream(s_);
+    gave_up_ = rc != DRH_OK;
     if (rc) return rc;
     pending_ = false;
     for (int i = 0; i < nback_; i++) std::memcpy(back_[i].dst, back_[i].src, back_[i].bytes);
@@ -810,6 +854,7 @@ int drh_clear_pool(drh_ctx* ctx) {
     }
     ctx->free_bufs.clear();
     ctx->bytes = 0;
+    reclaim_parked(ctx);  // what is still in use stays parked: freeing it would wait for the device
     for (auto& p : ctx->free_pinned) (void)hipHostFree(p.ptr);
     ctx->free_pinned.clear();
     ctx->pinned_bytes = 0;

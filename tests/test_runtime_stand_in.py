@@ -1,0 +1,148 @@
+"""The library's host code on the CPU, over a stand-in for the HIP runtime
+(fake_hip.cpp): each test is a program of its own in which the stand-in's functions,
+loaded first, take the place of the runtime's. Kernels do not run.
+"""
+
+import shutil
+import subprocess
+import sys
+import textwrap
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+PKG = HERE.parent / "differentiable-rasterizer_amd"
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
+fake.fake_pinned_bytes.restype = ctypes.c_size_t
+fake.fake_malloc_limit.argtypes = [ctypes.c_size_t]
+fake.fake_launches.restype = ctypes.c_char_p
+sys.modules["torch"] = None  # its runtime is not wanted here
+sys.path.insert(0, {pkg!r})
+import numpy as np
+from diffrast import _lib
+
+MIB = 1 << 20
+
+def code(f):
+    try:
+        f()
+    except _lib.DiffrastError as e:
+        return e.code
+    return 0
+
+ctx = _lib.Context()
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("no g++")
+    so = tmp_path_factory.mktemp("fake") / "libfake_hip.so"
+    # the headers want the platform named where hipcc does not compile them
+    subprocess.run([gxx, "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    str(HERE / "fake_hip.cpp"), "-o", str(so)], check=True)
+
+    def run(text):
+        body = PRELUDE.format(fake=str(so), pkg=str(PKG)) + textwrap.dedent(text)
+        res = subprocess.run([sys.executable, "-c", body], capture_output=True, text=True, timeout=100)
+        assert res.returncode == 0, res.stderr
+
+    return run
+
+
+def test_timed_out_calls_return(program):
+    """A wait that times out ends the call with the time-out; nothing waits without a limit."""
+    program("""
+        v = np.linspace(0, 1, 1000, dtype=np.float32)
+        target, init = np.zeros((24, 24, 3), np.float32), np.full((5, 10), .5, np.float32)
+        fit = _lib.Fitter(ctx, target, init, np.zeros(3, np.float32), iters=4)
+        fake.fake_stuck(1)
+        assert code(lambda: ctx.encode_srgb(v)) == 2
+        assert code(lambda: ctx.render(init[None], 24, 24, .01)) == 2
+        assert code(lambda: ctx.fused_loss_backward(init[None], target[None], .01, want_images=True)) == 2
+        assert code(lambda: _lib.Fitter(ctx, target, init, np.zeros(3, np.float32), iters=4)) == 2
+        assert code(fit.step) == 2
+        assert code(lambda: ctx.resize_lanczos3(np.zeros((30, 30, 3), np.uint8), 7, 8)) == 2
+        assert fake.fake_unbounded_waits() == 0
+        parked = fake.fake_pinned_bytes()
+        fake.fake_stuck(0)
+        # the parked buffers are used again
+        ctx.encode_srgb(v)
+        assert fake.fake_pinned_bytes() == parked
+        fit.close()
+        ctx.clear_pool()
+        assert fake.fake_pinned_bytes() == 0
+    """)
+
+
+def test_parked_buffers_are_bounded(program):
+    program("""
+        fake.fake_stuck(1)
+        v = np.zeros(3 * MIB, np.float32)  # 15 MiB both ways: a buffer of 16
+        for _ in range(4):
+            assert code(lambda: ctx.encode_srgb(v)) == 2
+        assert fake.fake_unbounded_waits() == 0 and fake.fake_pinned_bytes() == 64 * MIB
+        code(lambda: ctx.encode_srgb(v))  # no buffer is left: copied as it is
+        assert fake.fake_pinned_bytes() == 64 * MIB
+        fake.fake_stuck(0)
+        ctx.encode_srgb(v)
+        ctx.clear_pool()
+        assert fake.fake_pinned_bytes() == 0
+    """)
+
+
+@pytest.mark.parametrize("stuck", [0, 1])
+@pytest.mark.parametrize("copy", [0, 1, 2, 4])
+def test_call_that_fails_half_way(program, copy, stuck):
+    """The failed copy's error is the call's, also where the wait for the others times out."""
+    program(f"""
+        init, target = np.full((1, 5, 10), .5, np.float32), np.zeros((1, 24, 24, 3), np.float32)
+        call = lambda: ctx.fused_loss_backward(init, target, .01)  # three copies in, two out
+        fake.fake_copy_fails({copy})
+        fake.fake_stuck({stuck})
+        rc = code(call)
+        assert rc == ({copy} < 3 and 3 or 4), (rc, _lib.last_error())
+        assert "stand-in error" in _lib.last_error()
+        assert fake.fake_unbounded_waits() == 0
+        fake.fake_stuck(0)
+        assert code(call) == 0
+        assert fake.fake_pinned_bytes() == MIB
+    """)
+
+
+@pytest.mark.parametrize("n", [10, 12800, 1 << 20, 5 << 20])
+def test_arrays_go_through_the_buffer_or_past_it(program, n):
+    """Adam's arrays in and out unchanged (its kernel does not run): all of them staged, the
+    first four of eight, none."""
+    program(f"""
+        fake.fake_polls(5)
+        n = {n} // 10 * 10
+        p, g, m, v, lr = (np.random.default_rng(i).random((n // 10, 10), dtype=np.float32) for i in range(5))
+        want = p.copy(), m.copy(), v.copy()
+        for _ in range(2):
+            out = ctx.adam_project_step(p, g, m, v, lr, step=1)
+            for a, b in zip((p, m, v), want):
+                assert np.array_equal(a, b)
+        assert fake.fake_pinned_bytes() <= 16 * MIB
+    """)
+
+
+def test_free_buffers_are_bounded_and_given_back(program):
+    program("""
+        import threading
+        fake.fake_polls(3)
+        for n in (1, MIB // 4, MIB // 2, MIB, 3 * MIB, 20 * MIB):
+            ctx.encode_srgb(np.zeros(n, np.float32))
+        assert fake.fake_pinned_bytes() == 31 * MIB  # a buffer each of 1, 2, 4, 8 and 16
+        ctx.clear_pool()
+        assert fake.fake_pinned_bytes() == 0
+        ctx.encode_srgb(np.zeros(5, np.float32))
+        ctx.close()
+        assert fake.fake_pinned_bytes() == 0
+    """)
