@@ -574,15 +574,6 @@ int run_raster(drh_ctx* ctx, int mode, const float* params, const float* bgs, co
         if ((rc = order.acquire(ctx, K_ORDER, cells * sizeof(int), s))) return rc;
         bufs.order = order.get<int>();
     }
-    // the tile rows' lists, where the call's kernel reads them
-    const size_t trows = (size_t)B * 2 * grid.y;
-    const int rows_min_t = mode == drh::MODE_RENDER ? ROW_LISTS_MIN_T_RENDER : ROW_LISTS_MIN_T_FUSED;
-    if ((mode == drh::MODE_RENDER || (bufs.fused && !bufs.segw && !det)) && T >= rows_min_t && W <= drh::ROWS_MAX_W &&
-        trows * T * sizeof(int2) <= ROW_LISTS_BUDGET) {
-        if ((rc = rows.acquire(ctx, K_ROWS, trows * T * sizeof(int2) + trows * sizeof(int), s))) return rc;
-        bufs.rows = rows.get<int2>();
-        bufs.row_n = reinterpret_cast<int*>(bufs.rows + trows * T);
-    }
     if (mode != drh::MODE_RENDER) {
         const size_t prows = (size_t)B * nblk * (bufs.segw ? drh::WAVES : 1);  // per block, or per tile
         if (det && (rc = partials.acquire(ctx, K_PARTIALS, prows * T * NP * sizeof(float), s))) return rc;
@@ -596,6 +587,22 @@ int run_raster(drh_ctx* ctx, int mode, const float* params, const float* bgs, co
                 return rc;
             if ((rc = pze.acquire(ctx, K_PIX_ZE, ntiles * 64 * sizeof(int2), s))) return rc;
             if ((rc = tn.acquire(ctx, K_TILE_N, ntiles * 2 * sizeof(int), s))) return rc;
+        }
+    }
+    // the tile rows' lists, where the call's kernel reads them (last: they leave the rest their memory)
+    const size_t trows = (size_t)B * 2 * grid.y;
+    const int rows_min_t = mode == drh::MODE_RENDER ? ROW_LISTS_MIN_T_RENDER : ROW_LISTS_MIN_T_FUSED;
+    if ((mode == drh::MODE_RENDER || (bufs.fused && !bufs.segw && !det)) && T >= rows_min_t && W <= drh::ROWS_MAX_W &&
+        trows * T * sizeof(int2) <= ROW_LISTS_BUDGET) {
+        // they only save time: without room for them the kernel scans every triangle
+        rc = rows.acquire(ctx, K_ROWS, trows * T * sizeof(int2) + trows * sizeof(int), s);
+        if (rc == DRH_OK) {
+            bufs.rows = rows.get<int2>();
+            bufs.row_n = reinterpret_cast<int*>(bufs.rows + trows * T);
+        } else if (rc == DRH_ERR_TOO_LARGE) {
+            (void)hipGetLastError();  // the failed allocation's, which the launches' checks would find
+        } else {
+            return rc;
         }
     }
     bufs.rec = tail && tail->rec ? tail->rec : rec.get<float>();

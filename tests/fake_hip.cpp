@@ -20,7 +20,7 @@ namespace {
 std::vector<std::function<void()>> g_queue;
 bool g_stuck = false;
 int g_polls = 0, g_polls_left = 0;  // a wait finds its event done after this many looks
-size_t g_malloc_limit = SIZE_MAX;   // larger device allocations fail
+size_t g_malloc_fails = 0;          // device allocations of this many bytes fail
 int g_copy_fails = -1;              // the copy of this number (from now, from 0) fails
 int g_unbounded = 0;                // waits without a limit
 std::map<void*, size_t> g_pinned;
@@ -54,7 +54,7 @@ extern "C" {
 // controls of the tests
 void fake_stuck(int on) { g_stuck = on != 0; }
 void fake_polls(int n) { g_polls = g_polls_left = n; }
-void fake_malloc_limit(size_t n) { g_malloc_limit = n ? n : SIZE_MAX; }
+void fake_malloc_fails(size_t n) { g_malloc_fails = n; }
 void fake_copy_fails(int n) { g_copy_fails = n; }
 int fake_unbounded_waits() { return g_unbounded; }
 size_t fake_pinned_bytes() {
@@ -99,7 +99,7 @@ hipError_t hipGetLastError() {
 hipError_t hipGetSymbolAddress(void** p, const void* s) { return *p = const_cast<void*>(s), hipSuccess; }
 
 hipError_t hipMalloc(void** p, size_t n) {
-    if (n > g_malloc_limit) return ret(hipErrorOutOfMemory);
+    if (n == g_malloc_fails) return ret(hipErrorOutOfMemory);
     *p = std::calloc(1, n);
     return hipSuccess;
 }

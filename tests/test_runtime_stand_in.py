@@ -18,7 +18,7 @@ PRELUDE = """
 import ctypes, sys
 fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
 fake.fake_pinned_bytes.restype = ctypes.c_size_t
-fake.fake_malloc_limit.argtypes = [ctypes.c_size_t]
+fake.fake_malloc_fails.argtypes = [ctypes.c_size_t]
 fake.fake_launches.restype = ctypes.c_char_p
 sys.modules["torch"] = None  # its runtime is not wanted here
 sys.path.insert(0, {pkg!r})
@@ -26,6 +26,14 @@ import numpy as np
 from diffrast import _lib
 
 MIB = 1 << 20
+
+def launched(f):
+    fake.fake_launches()
+    f()
+    return fake.fake_launches().decode().split()
+
+def addr(a):  # device memory is host memory here
+    return a.ctypes.data
 
 def code(f):
     try:
@@ -145,4 +153,27 @@ def test_free_buffers_are_bounded_and_given_back(program):
         ctx.encode_srgb(np.zeros(5, np.float32))
         ctx.close()
         assert fake.fake_pinned_bytes() == 0
+    """)
+
+
+@pytest.mark.parametrize("B,H,W,T", [(1, 520, 500, 300), (2, 1000, 1000, 128), (8, 256, 256, 200)])
+def test_call_without_room_for_row_lists(program, B, H, W, T):
+    """The tile rows' lists only save time: a call that finds no memory for them scans every
+    triangle."""
+    program(f"""
+        B, H, W, T = {B}, {H}, {W}, {T}
+        params, bg = np.full((B, T, 10), .5, np.float32), np.zeros((B, 3), np.float32)
+        img, losses, grads = np.zeros((B, H, W, 3), np.float32), np.zeros(B, np.float32), np.zeros((B, T, 10), np.float32)
+        render = lambda: ctx.render_ptr(addr(params), addr(bg), B, T, H, W, .002, addr(img))
+        fused = lambda: ctx.fused_ptr(addr(params), addr(bg), addr(img), B, T, H, W, .002, addr(losses), addr(grads))
+        rows = 2 * B * ((H + 15) // 16)
+        for call in (render, fused):
+            listed = launched(call)
+            ctx.clear_pool()
+            fake.fake_malloc_fails(rows * T * 8 + rows * 4)
+            scanned = launched(call)
+            fake.fake_malloc_fails(0)
+            assert len(scanned) == len(listed) and scanned != listed, (scanned, listed)
+            assert launched(call) == listed
+            ctx.clear_pool()
     """)
