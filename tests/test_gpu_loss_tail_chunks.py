@@ -32,3 +32,18 @@ def test_tail_chunks(ctx, B, H, W):
     tail = ctx.fused_loss_backward(params, targets, sigma, bgs)[0]
     fixed = ctx.fused_loss_backward(params, targets, sigma, bgs, deterministic=True)[0]
     assert np.array_equal(tail, fixed)
+
+
+# 1, 2, 16, 63, 64, 65, 128 and 130 blocks a scene: the last lanes and loads of a chunk have none
+@pytest.mark.parametrize("H,W", [(9, 16), (17, 5), (64, 64), (112, 131), (128, 128), (80, 200), (128, 256), (160, 208)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("B", [1, 9])
+def test_tail_of_small_scenes(ctx, B, H, W):
+    T, sigma = 8, 0.01
+    params = synth.batch("random", B, T, 2300)
+    bgs = synth.uniforms(2307, B * 3).reshape(B, 3).astype(np.float32)
+    targets = np.stack([synth.blob_target(2300 + b, H, W) for b in range(B)])
+    print(f"tail of small scenes B={B} {H}x{W}", flush=True)
+    tail = ctx.fused_loss_backward(params, targets, sigma, bgs)[0]
+    fixed = ctx.fused_loss_backward(params, targets, sigma, bgs, deterministic=True)[0]
+    assert np.array_equal(tail, fixed)
