@@ -137,11 +137,11 @@ def time_fused(torch, ctx, cfg, p, bg, targets, steps, warmup, dev):
 def fused_kernel_name(B, H, W, T, deterministic=False):
     """The kernel the library's fused gradient path takes for this shape: the
     segmented kernel for 16 to 1024 triangles on grids of at most 2048 8x8 tiles
-    (below 6144 for a batch without fixed-order sums; runtime.h: segment_waves),
-    else the one-wave tile kernel (the four-wave block kernel with fixed-order
-    sums)."""
+    (below 6144 for a batch of at least 48 triangles a scene without fixed-order
+    sums; runtime.h: segment_waves), else the one-wave tile kernel (the four-wave
+    block kernel with fixed-order sums)."""
     tiles = B * ((W + 15) // 16) * ((H + 15) // 16) * 4
-    if 16 <= T <= 1024 and (tiles <= 2048 or (B > 1 and not deterministic and tiles < 6144)):
+    if 16 <= T <= 1024 and (tiles <= 2048 or (B > 1 and T >= 48 and not deterministic and tiles < 6144)):
         return "fused_seg_kernel" + (" (fixed order)" if deterministic else "")
     return "fused_kernel (fixed order)" if deterministic else "fused_tile_kernel"
 

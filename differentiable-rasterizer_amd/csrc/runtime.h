@@ -310,29 +310,43 @@ struct RasterBufs {
 // fused_seg_kernel's waves per tile for a gradient call (fused) of `ntiles` 8x8
 // tiles, 0: the other kernels. Up to about a tile per SIMD a wave per tile is
 // bound by each tile's chain of dependent waits, and splitting a tile's entries
-// over waves shortens it: eight waves up to 3 tiles per CU, four up to 8 (10 for
-// a batch), two below 24, where a batch otherwise splits its heaviest blocks'
+// over waves shortens it: eight waves up to 768 tiles, four up to 2048 (2560 for
+// a batch), two below 6144, where a batch otherwise splits its heaviest blocks'
 // backward (SPLIT_*); from there on the one-wave kernel fills the device and its
-// tiles' fixed costs are less. Measured on 256 CUs, us per call, T = 128 large
-// triangles (uniform) / medium ones (random, sigma 0.01) / the same with sigma
-// 0.0015:
-//   tiles           other kernels        8 waves              4 waves              2 waves
-//    676 B=1      59 /  33 /  20      27 /  22 /  21      32 /  21 /  21      45 /  26 /  21
-//   1024 B=1      57 /  31 /  21      28 /  24 /  20      32 /  21 /  20      45 /  25 /  20
-//   2048 B=8      60 /  39 /  28      47 /  36 /  29      35 /  28 /  21      51 /  28 /  20
-//   4096 B=16     64 /  42 /  29      78 /  62 /  47      53 /  43 /  31      49 /  37 /  25
-//   5120 B=5      64 /  49 /  31      88 /  72 /  55      57 /  47 /  34      49 /  38 /  26
-//   6144 B=6      67 /  37 /  25     102 /  83 /  63      65 /  54 /  38      56 /  43 /  28
-//   4096 B=1      71 /  42 /  23      76 /  64 /  51      62 /  46 /  28      64 /  43 /  23
-// Past SEG2_MAX_T triangles two waves' LDS (20 bytes a triangle) leaves few
-// workgroups a CU: four there (B=4 256x256 T=800: 333 / 169 / 88 with the other
-// kernels, 203 / 144 / 68 with four waves, 247 / 176 / 75 with two). In the
-// fixed-order mode the tiles' partial rows grow with them: none past 8 tiles per
-// CU. From SEG_MIN_T triangles (a couple per wave) up to drh::SEG_MAX_T.
+// tiles' fixed costs are less. The limits are counts of tiles, measured on the 256
+// CUs of an MI355X, us per call, T = 128 large triangles (uniform) / medium ones
+// (random, sigma 0.004) / small ones:
+//   tiles        other kernels    8 waves         4 waves         2 waves
+//    676 B=1     49 / 23 / 15     23 / 16 / 13    27 / 16 / 12    38 / 19 / 13
+//   1024 B=1     48 / 24 / 16     28 / 20 / 16    27 / 17 / 13    38 / 20 / 14
+//   2048 B=8     57 / 31 / 25     44 / 30 / 26    32 / 22 / 18    43 / 22 / 17
+//   2304 B=9     59 / 34 / 27     50 / 35 / 29    35 / 25 / 20    46 / 23 / 19
+//   4096 B=16    61 / 32 / 26     74 / 50 / 41    51 / 34 / 25    46 / 28 / 20
+//   5120 B=5     61 / 36 / 26     85 / 58 / 47    55 / 37 / 28    46 / 29 / 20
+//   6144 B=6     61 / 27 / 19     98 / 67 / 53    63 / 42 / 31    53 / 32 / 22
+//   2116 B=1     49 / 24 / 16     41 / 29 / 22    38 / 22 / 16    41 / 21 / 14
+//   2704 B=1     55 / 26 / 16     49 / 34 / 26    45 / 25 / 17    52 / 22 / 15
+//   4096 B=1     69 / 28 / 17     71 / 47 / 35    62 / 31 / 21    63 / 30 / 17
+// One scene of a little more than 2048 tiles would gain from two or four waves
+// with large triangles (T = 512 at 2704 tiles: 165 -> 95 us) and lose with small
+// ones (21 -> 25): not taken. Past SEG2_MAX_T triangles two waves' LDS (20 bytes a
+// triangle) leaves few workgroups a CU: four there (B=4 256x256 T=800: 330 / 109 /
+// 62 with the other kernels, 204 / 91 / 47 with four waves, 249 / 106 / 49 with
+// two). In the fixed-order mode the tiles' partial rows grow with them: none past
+// 2048 tiles. From SEG_MIN_T triangles (a couple per wave) up to drh::SEG_MAX_T,
+// and past 2048 tiles only from SEG_BATCH_MIN_T: below, nothing is split otherwise
+// and a wave per tile is the faster (B=16 128x128 T=16 medium 14.5 us, 15.7 with
+// two waves; B=5 256x256 T=32 18.7, 20.2; T=48 19.5, split 26.8, two waves 21.5).
+// `noalloc`: drh_fused_loss_backward_noalloc, which never splits, so its other
+// kernel is the one-wave one (over every triangle): two waves end at
+// SEG2_NOALLOC_TILES. B=3 256x256, 3072 tiles: faster for every kind from T = 48
+// to 800 (7 to 80%); 4096 to 5632 tiles: large triangles up to 45% faster, small
+// ones up to 13% slower.
 // DRH_NO_SEGMENTS=1 in the environment keeps the other kernels (for comparing).
-constexpr size_t SEG8_MAX_TILES = 768, SEG4_MAX_TILES = 2048, SEG4_MAX_TILES_BATCH = 2560, SEG2_END_TILES = 6144;
-constexpr int SEG_MIN_T = 16, SEG2_MAX_T = 512;
-int segment_waves(int mode, int B, size_t ntiles, int T, bool det);
+constexpr size_t SEG8_MAX_TILES = 768, SEG4_MAX_TILES = 2048, SEG4_MAX_TILES_BATCH = 2560, SEG2_END_TILES = 6144,
+                 SEG2_NOALLOC_TILES = 3072;
+constexpr int SEG_MIN_T = 16, SEG_BATCH_MIN_T = 48, SEG2_MAX_T = 512;
+int segment_waves(int mode, int B, size_t ntiles, int T, bool det, bool noalloc = false);
 
 // From these many triangles on the one-wave fused kernel's and renders' lists scan
 // the triangles of their tile row (RowArgs), which setup_records lists beside the

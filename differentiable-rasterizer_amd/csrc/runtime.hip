@@ -428,13 +428,15 @@ bool fused_gradients(int mode, int nseg, int cap2, int T) {
     return !(e && e[0] == '1');
 }
 
-int segment_waves(int mode, int B, size_t ntiles, int T, bool det) {
+int segment_waves(int mode, int B, size_t ntiles, int T, bool det, bool noalloc) {
     if ((mode != drh::MODE_LOSS && mode != drh::MODE_GRAD_IN) || T < SEG_MIN_T || T > drh::SEG_MAX_T) return 0;
     const char* e = std::getenv("DRH_NO_SEGMENTS");
     if (e && e[0] == '1') return 0;
     if (ntiles <= SEG8_MAX_TILES) return 8;
-    if (ntiles <= (B > 1 && !det ? SEG4_MAX_TILES_BATCH : SEG4_MAX_TILES)) return 4;
-    if (B > 1 && !det && ntiles < SEG2_END_TILES) return T <= SEG2_MAX_T ? 2 : 4;
+    if (ntiles <= SEG4_MAX_TILES) return 4;
+    if (B == 1 || det || T < SEG_BATCH_MIN_T) return 0;
+    if (ntiles <= SEG4_MAX_TILES_BATCH) return 4;
+    if (noalloc ? ntiles <= SEG2_NOALLOC_TILES : ntiles < SEG2_END_TILES) return T <= SEG2_MAX_T ? 2 : 4;
     return 0;
 }
 

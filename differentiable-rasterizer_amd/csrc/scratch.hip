@@ -60,7 +60,7 @@ DeviceSlot* device_slot(int device) {
 struct ScratchLayout {
     size_t rec = 0, ploss = 0, pq = 0, pg0 = 0, pze = 0, tn = 0, order = 0, partials = 0, tent = 0, total = 0;
     int cap2 = 0;
-    int segw = 0;  // fused_seg_kernel, as drh_fused_loss_backward takes it
+    int segw = 0;  // fused_seg_kernel's waves per tile, or 0
     bool ordered = false;
 };
 
@@ -97,12 +97,12 @@ ScratchLayout scratch_layout(const drh_ctx* ctx, int B, int T, int H, int W, boo
     return L;
 }
 
-// fused_seg_kernel where drh_fused_loss_backward takes it and its partial rows
+// fused_seg_kernel where segment_waves says so and its partial rows
 // fit (with DRH_DETERMINISTIC they are per tile), else the other kernels.
 ScratchLayout scratch_layout(const drh_ctx* ctx, int B, int T, int H, int W, bool det) {
     const dim3 grid = drh::raster_grid(B, W, H);
     const int segw = fused_gradients(drh::MODE_LOSS, 1, (T + 8) & ~7, T)
-                         ? segment_waves(drh::MODE_LOSS, B, (size_t)B * grid.x * grid.y * drh::WAVES, T, det)
+                         ? segment_waves(drh::MODE_LOSS, B, (size_t)B * grid.x * grid.y * drh::WAVES, T, det, true)
                          : 0;
     if (segw) {
         const ScratchLayout L = scratch_layout(ctx, B, T, H, W, det, segw);

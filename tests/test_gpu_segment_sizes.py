@@ -29,13 +29,15 @@ CASES = [
     ("4w-T257", 3, 150, 155, 257, 0.004, "random"),
     ("4w-T600", 1, 230, 226, 600, 0.0015, "small"),
     ("4w-batch-T700", 12, 120, 130, 700, 0.003, "small"),
-    # 2 waves: a batch of 2560 to 6143 tiles
-    ("2w-T16", 11, 120, 130, 16, 0.004, "uniform"),
+    # 2 waves: a batch of 2560 to 6143 tiles, from 48 triangles
+    ("2w-T48", 11, 120, 130, 48, 0.004, "uniform"),
     ("2w-T66", 11, 120, 130, 66, 0.0015, "uniform"),
     ("2w-T200-long-lists", 11, 120, 130, 200, 0.002, "uniform"),
     ("2w-T512", 10, 121, 131, 512, 0.004, "random"),
     # just past the rule: the other kernels either way
     ("T1025", 1, 24, 24, 1025, 0.003, "small"),
+    ("batch-T47", 11, 120, 130, 47, 0.004, "uniform"),
+    ("batch-T16", 9, 128, 128, 16, 0.004, "random"),
 ]
 
 

@@ -177,3 +177,38 @@ def test_call_without_room_for_row_lists(program, B, H, W, T):
             assert launched(call) == listed
             ctx.clear_pool()
     """)
+
+
+# waves a tile of fused_seg_kernel (0: another kernel) for one call of drh_fused_loss_backward and of
+# drh_fused_loss_backward_noalloc; tiles are 8x8, four to a 16x16 block
+@pytest.mark.parametrize("B,H,W,T,pooled,noalloc", [
+    (1, 64, 64, 15, 0, 0), (1, 64, 64, 16, 8, 8), (1, 64, 64, 1024, 8, 8), (1, 64, 64, 1025, 0, 0),
+    (3, 128, 128, 16, 8, 8), (4, 128, 96, 16, 8, 8), (4, 128, 112, 16, 4, 4), (1, 224, 240, 150, 4, 4),
+    (8, 128, 128, 16, 4, 4), (1, 256, 512, 300, 4, 4), (1, 272, 496, 300, 0, 0),
+    # a batch past 2048 tiles, from 48 triangles
+    (9, 128, 128, 16, 0, 0), (9, 128, 128, 47, 0, 0), (9, 128, 128, 48, 4, 4), (10, 128, 128, 300, 4, 4),
+    (11, 128, 128, 47, 0, 0), (11, 128, 128, 48, 2, 2), (12, 128, 128, 512, 2, 2), (12, 128, 128, 513, 4, 4),
+    (13, 128, 128, 200, 2, 0), (16, 128, 128, 32, 0, 0), (16, 128, 128, 128, 2, 0), (16, 128, 128, 1024, 4, 0),
+    (5, 256, 256, 512, 2, 0), (6, 256, 256, 128, 0, 0), (23, 128, 128, 128, 2, 0), (24, 128, 128, 128, 0, 0),
+])
+def test_waves_per_tile(program, B, H, W, T, pooled, noalloc):
+    """Which kernel a gradient call takes, also without atomics (no batch past 2048 tiles) and in
+    the IEEE mode."""
+    program(f"""
+        import re
+        B, H, W, T = {B}, {H}, {W}, {T}
+        params, bg = np.full((B, T, 10), .5, np.float32), np.zeros((B, 3), np.float32)
+        img, losses, grads = np.zeros((B, H, W, 3), np.float32), np.zeros(B, np.float32), np.zeros((B, T, 10), np.float32)
+        def waves(call, flags):
+            names = launched(lambda: call(addr(params), addr(bg), addr(img), B, T, H, W, .002, addr(losses),
+                                          addr(grads), flags=flags))
+            found = [re.search(r"fused_seg_kernelILi\\d+ELb\\dELb\\dELi(\\d)E", n) for n in names]
+            return sum(int(m.group(1)) for m in found if m)
+        tiles = 4 * B * ((H + 15) // 16) * ((W + 15) // 16)
+        for flags in (0, _lib.EXACT_MATH, _lib.DETERMINISTIC):
+            off = flags == _lib.DETERMINISTIC and tiles > 2048
+            assert waves(ctx.fused_ptr, flags) == (0 if off else {pooled}), flags
+            assert waves(ctx.fused_noalloc_ptr, flags) == (0 if off else {noalloc}), flags
+        bwd = lambda p, b, i, B, T, H, W, s, l, g, flags: ctx.from_grad_ptr(p, b, i, B, T, H, W, s, g, flags=flags)
+        assert waves(bwd, 0) == {pooled}
+    """)
