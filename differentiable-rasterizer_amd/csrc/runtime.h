@@ -353,12 +353,23 @@ int segment_waves(int mode, int B, size_t ntiles, int T, bool det, bool noalloc 
 // records: a tile's box tests then read a few coalesced words instead of every
 // triangle's record. us per call without and with, large (uniform) / medium
 // (random, sigma 0.004) / small triangles: fused B=16 256x256 T=64 54.9 / 34.7 /
-// 25.3 -> 51.4 / 34.5 / 24.8, T=512 308 / 127 / 62.6 -> 301 / 123 / 50.1; renders
+// 25.3 -> 51.4 / 34.5 / 24.8, T=512 302 / 127 / 60.0 -> 296 / 121 / 46.2; renders
 // B=1 512x512 T=1024 107 / 48.8 / 29.3 -> 111 / 39.5 / 22.7, 1024x1024 T=150 41.1
 // / 30.6 / 20.9 -> 36.9 / 25.4 / 20.7, T=64 unchanged. The segmented kernel's
 // waves share the scan, and waiting for a row first cost it up to 10%: it scans
 // every triangle.
-constexpr int ROW_LISTS_MIN_T_FUSED = 64, ROW_LISTS_MIN_T_RENDER = 128;
+// Many rows are listed in many scenes' setup at the call's expense, and a scene of
+// few rows gains little from them: with more than ROW_LISTS_FREE rows in all, only
+// where triangles times a scene's rows reach ROW_LISTS_MIN_WORK. Fused, 64x64:
+// B=256 T=64 83.5 / 48.4 / 32.9 -> 87.7 / 52.3 / 36.8, T=128 154 / 80.3 / 47.7 ->
+// 158 / 84.0 / 51.1, B=96 T=256 152 / 67.8 / 39.6 -> 154 / 66.1 / 38.0; renders
+// B=256 64x64 T=128 71.0 / 42.7 / 31.2 -> 73.8 / 46.2 / 34.7, T=256 134 / 74.4 /
+// 53.6 -> 138 / 72.2 / 49.7. What stays slower with them is large triangles in
+// renders of 96 or more small scenes, whose records are more than the L2s hold and
+// were read ahead by the scan: B=128 64x64 T=1000 478 / 188 / 128 -> 525 / 165 /
+// 94.7. The sizes do not tell, and the other kinds gain more.
+constexpr int ROW_LISTS_MIN_T_FUSED = 64, ROW_LISTS_MIN_T_RENDER = 128, ROW_LISTS_MIN_WORK = 2048;
+constexpr size_t ROW_LISTS_FREE = 512;
 constexpr size_t ROW_LISTS_BUDGET = 256ull << 20;  // bytes
 
 // Split of the backward's sweep over a tile's recorded entries. A tile's sweep

@@ -595,6 +595,7 @@ int run_raster(drh_ctx* ctx, int mode, const float* params, const float* bgs, co
     const size_t trows = (size_t)B * 2 * grid.y;
     const int rows_min_t = mode == drh::MODE_RENDER ? ROW_LISTS_MIN_T_RENDER : ROW_LISTS_MIN_T_FUSED;
     if ((mode == drh::MODE_RENDER || (bufs.fused && !bufs.segw && !det)) && T >= rows_min_t && W <= drh::ROWS_MAX_W &&
+        (trows <= ROW_LISTS_FREE || T * 2 * (int64_t)grid.y >= ROW_LISTS_MIN_WORK) &&
         trows * T * sizeof(int2) <= ROW_LISTS_BUDGET) {
         // they only save time: without room for them the kernel scans every triangle
         rc = rows.acquire(ctx, K_ROWS, trows * T * sizeof(int2) + trows * sizeof(int), s);

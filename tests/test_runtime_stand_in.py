@@ -212,3 +212,30 @@ def test_waves_per_tile(program, B, H, W, T, pooled, noalloc):
         bwd = lambda p, b, i, B, T, H, W, s, l, g, flags: ctx.from_grad_ptr(p, b, i, B, T, H, W, s, g, flags=flags)
         assert waves(bwd, 0) == {pooled}
     """)
+
+
+@pytest.mark.parametrize("B,H,W,T,render,fused", [
+    (1, 512, 512, 63, 0, 0), (1, 512, 512, 64, 0, 1), (1, 512, 512, 127, 0, 1), (1, 512, 512, 128, 1, 1),
+    (1, 40, 4096, 128, 1, 1), (6, 256, 256, 64, 0, 1), (16, 256, 256, 64, 0, 1), (17, 256, 256, 64, 0, 1),
+    # up to 512 tile rows in all, past them from 2048 triangles times a scene's rows
+    (24, 128, 128, 64, 0, 1), (32, 128, 128, 64, 0, 1), (33, 128, 128, 127, 0, 0), (33, 128, 128, 128, 1, 1),
+    (64, 64, 128, 128, 1, 1), (96, 64, 64, 128, 0, 0), (96, 64, 64, 255, 0, 0), (96, 64, 64, 256, 1, 1),
+    (65, 64, 128, 255, 0, 0), (128, 32, 128, 128, 1, 1), (512, 32, 32, 511, 0, 0), (512, 32, 32, 512, 1, 1),
+    (128, 64, 64, 4096, 1, 1), (128, 64, 64, 32800, 0, 0),  # 256 MiB of lists at most
+])
+def test_row_lists_rule(program, B, H, W, T, render, fused):
+    """Whether a render and a fused call outside the segmented kernel's share list the tile rows."""
+    program(f"""
+        import re
+        B, H, W, T = {B}, {H}, {W}, {T}
+        params, bg = np.zeros((B, T, 10), np.float32), np.zeros((B, 3), np.float32)
+        img, losses, grads = np.zeros((B, H, W, 3), np.float32), np.zeros(B, np.float32), np.zeros((B, T, 10), np.float32)
+        names = launched(lambda: ctx.render_ptr(addr(params), addr(bg), B, T, H, W, .002, addr(img)))
+        lists = [re.search(r"forward_kernelILi\\d+ELb\\dELb\\dELb(\\d)E", n) for n in names]
+        assert [int(m.group(1)) for m in lists if m] == [{render}], names
+        names = launched(lambda: ctx.fused_ptr(addr(params), addr(bg), addr(img), B, T, H, W, .002, addr(losses),
+                                               addr(grads)))
+        lists = [re.search(r"fused_tile_kernelILi\\d+ELb\\dELb(\\d)E", n) for n in names]
+        lists = [int(m.group(1)) for m in lists if m]
+        assert lists == [{fused}] or not lists and T > 1024, names
+    """)
