@@ -2,18 +2,19 @@
 
 setup_records orders the blocks of a batch (B > 1) whose grid has more blocks than
 the device has CUs (256 on MI355X): the backward kernel always follows the order, the
-forward kernel when T <= 256, and the one-wave fused kernel an order of 8x8 tiles where
-the scene's tile grid fits the order's cells (else the block order, four tiles per
-block). The order only changes which tile a launch slot works on, so every result must
-equal the oracle's at this path's bars (images 1e-5, gradients 1e-4 of the scene's
-gradient norm), and, with DRH_DETERMINISTIC, be bit-identical from call to call. The
-cases are sized to take the ordered paths: 4 scenes of 160 x 200 px are 4 x 10 x 13 =
-520 blocks; 2 scenes of 720 x 768 px have 90 x 96 tiles each, past the tile order's
+forward kernel when T <= 256, and the one-wave fused kernel and the segmented one an
+order of 8x8 tiles where the scene's tile grid fits the order's cells (else the block
+order, four tiles per block). The order only changes which tile a launch slot works on,
+so every result must equal the oracle's at this path's bars (images 1e-5, gradients 1e-4
+of the scene's gradient norm), and, with DRH_DETERMINISTIC, be bit-identical from call to
+call. The cases are sized to take the ordered paths: 4 scenes of 160 x 200 px are 4 x 10 x
+13 = 520 blocks; 2 scenes of 720 x 768 px have 90 x 96 tiles each, past the tile order's
 8192 cells, so their one-wave fused kernel takes the block order; 2 scenes of 1100
 small triangles take the order workgroup's triangles in three batches of up to 512
-and the records in nine workgroups of 128. From 256 triangles on, the one-wave
-fused kernel's lists scan only the triangles of their tile row, which setup_records
-lists (the small-triangle cases, and 300 large triangles at 256 x 256).
+and the records in nine workgroups of 128; 6 scenes of 256 x 256 px are past the
+segmented kernel's share, with the lists of their tile rows. Each runs as it does by
+default and with DRH_NO_SEGMENTS=1, where the smaller grids split their heaviest blocks'
+backward.
 """
 
 import numpy as np
@@ -51,13 +52,18 @@ def scenes(kind, B, T, seed):
 # (kind, B, H, W, T, sigma): forward and backward ordered; backward only (T > 256)
 CASES = [("uniform", 4, 160, 200, 100, 0.002), ("small", 3, 200, 208, 300, 0.003),
          ("uniform", 2, 720, 768, 40, 0.002), ("small", 2, 256, 256, 1100, 0.002),
-         ("uniform", 2, 256, 256, 300, 0.002)]
+         ("uniform", 2, 256, 256, 300, 0.002), ("uniform", 6, 250, 256, 100, 0.002),
+         ("small", 6, 256, 245, 300, 0.002)]
 
 
+@pytest.mark.parametrize("segments", [True, False], ids=["default", "no-segments"])
 @pytest.mark.parametrize("kind,B,H,W,T,sigma", CASES,
-                         ids=["ordered", "backward-ordered", "large-block-order", "many-triangles", "row-lists-large"])
-def test_ordered_render_fused_and_from_grad_match_oracle(ctx, orc, kind, B, H, W, T, sigma):
+                         ids=["ordered", "backward-ordered", "large-block-order", "many-triangles", "large",
+                              "tile-order", "tile-order-row-lists"])
+def test_ordered_render_fused_and_from_grad_match_oracle(ctx, orc, kind, B, H, W, T, sigma, segments, monkeypatch):
     assert B * -(-H // 16) * -(-W // 16) > 256  # more blocks than CUs: the order is made
+    if not segments:
+        monkeypatch.setenv("DRH_NO_SEGMENTS", "1")
     params, bgs = scenes(kind, B, T, 50)
     print(f"order {kind} B={B} {H}x{W} T={T}", flush=True)
     img = ctx.render(params, H, W, sigma, bgs)

@@ -92,8 +92,8 @@ def test_fused_and_two_kernel_paths_agree(ctx, orc, name, B, H, W, T, sigma, kin
     # and image come from the same per-block sums (bit-equal); the gradients
     # differ only in the order of their float atomics, and not at all with
     # fixed-order sums. On grids this small the default would take
-    # fused_seg_kernel (tests/test_gpu_segments.py), which composites in
-    # segments and rounds differently: DRH_NO_SEGMENTS=1 keeps the others.
+    # fused_seg_kernel (tests/test_gpu_segments.py): DRH_NO_SEGMENTS=1 keeps
+    # the others.
     monkeypatch.setenv("DRH_NO_SEGMENTS", "1")
     params, bgs = make_case(B, H, W, T, kind)
     targets = orc.render_batch(synth.batch(kind, B, T, 100, target_offset=1000), H, W, sigma, bgs[::-1].copy())
@@ -120,12 +120,14 @@ def test_fused_and_two_kernel_paths_agree(ctx, orc, name, B, H, W, T, sigma, kin
 
 
 @pytest.mark.parametrize("mode", ["loss", "from_grad"])
-def test_split_backward_matches_oracle(ctx, orc, mode):
+def test_split_backward_matches_oracle(ctx, orc, mode, monkeypatch):
     # Six 128x128 scenes of large triangles: 384 blocks, under six per compute
     # unit, so the backward splits the sweep of the heaviest quarter of blocks
     # over three waves per tile from the forward kernel's checkpoints (tiles
     # with up to ~60 recorded entries). Against the oracle, and against the
-    # fixed-order mode, which never splits.
+    # fixed-order mode, which never splits. By default such grids take
+    # fused_seg_kernel up to 1024 triangles: DRH_NO_SEGMENTS=1 keeps the split.
+    monkeypatch.setenv("DRH_NO_SEGMENTS", "1")
     B, H, W, T, sigma = 6, 128, 128, 128, 0.0015
     params = synth.batch("uniform", B, T, 41)
     bgs = synth.uniforms(47, B * 3).reshape(B, 3).astype(np.float32)
@@ -512,8 +514,8 @@ def test_random_shapes_match_oracle(ctx, orc, i, monkeypatch):
     dl, dg = ctx.fused_loss_backward(params, targets, sigma, bgs, deterministic=True)
     assert np.array_equal(dl, losses[False])
     assert_grads(dg, cg, label=f"case {i} fixed-order")
-    # the fused kernels other than fused_seg_kernel (which small grids take by
-    # default and which rounds its segment composite differently)
+    # the fused kernels other than fused_seg_kernel, which small grids take by
+    # default
     monkeypatch.setenv("DRH_NO_SEGMENTS", "1")
     nl, ng = ctx.fused_loss_backward(params, targets, sigma, bgs)
     check_losses(nl, cl, label=f"case {i} no segments")

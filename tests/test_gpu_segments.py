@@ -1,7 +1,8 @@
 """fused_seg_kernel: the gradient calls on grids of few tiles (a single scene of
-a few hundred 8x8 tiles, the fit), where each tile's triangles are split over
+a few hundred 8x8 tiles, the fit), where each tile's entries are split over
 eight waves that evaluate their weights and sweep their gradients in parallel,
-while the composite between them runs in scene order.
+while the composite between them runs in scene order. Its other shares are in
+test_gpu_segment_sizes.py.
 
 Against the oracle at the usual bars (tests/bars.py); against the other fused
 kernels (DRH_NO_SEGMENTS=1): the same image and losses bit for bit (the
@@ -19,7 +20,7 @@ from diffrast import synth
 pytestmark = pytest.mark.gpu
 
 # (name, B, H, W, T, sigma, kind): every one within the segmented kernel's
-# share (at most 2048 tiles, 16 to 160 triangles)
+# share of eight waves (at most 768 tiles, 16 to 1024 triangles)
 CASES = [
     ("64x64-T32", 1, 64, 64, 32, 0.0015, "uniform"),
     ("fit-176-T150", 1, 176, 176, 150, 0.02, "uniform"),

@@ -239,3 +239,39 @@ def test_row_lists_rule(program, B, H, W, T, render, fused):
         lists = [int(m.group(1)) for m in lists if m]
         assert lists == [{fused}] or not lists and T > 1024, names
     """)
+
+
+SEG, ONE_WAVE, ONE_WAVE_ROWS = "fused_seg_kernel", r"fused_tile_kernelILi\\d+ELb\\dELb0E", r"fused_tile_kernelILi\\d+ELb\\dELb1E"
+SPLIT = r"forward_kernelILi\\d+ELb\\dELb1E"  # with checkpoints
+
+
+@pytest.mark.parametrize("name,B,H,W,T,segments,entry,kernel", [
+    ("split backward", 6, 128, 128, 128, False, "fused_ptr", SPLIT),
+    ("split backward from gradients", 6, 128, 128, 128, False, "from_grad_ptr", SPLIT),
+    ("merged lists", 1, 480, 512, 300, True, "fused_noalloc_ptr", ONE_WAVE),
+    ("merged lists, full region", 1, 480, 512, 304, True, "fused_noalloc_ptr", ONE_WAVE),
+    ("merged lists of rows", 1, 480, 512, 304, True, "fused_ptr", ONE_WAVE_ROWS),
+    ("ordered", 4, 160, 200, 100, True, "fused_ptr", SEG),
+    ("ordered, split", 4, 160, 200, 100, False, "fused_ptr", SPLIT),
+    ("backward-ordered, split", 3, 200, 208, 300, False, "fused_ptr", SPLIT),
+    ("large-block-order", 2, 720, 768, 40, True, "fused_ptr", ONE_WAVE),
+    ("many-triangles", 2, 256, 256, 1100, True, "fused_ptr", SPLIT),
+    ("tile-order", 6, 250, 256, 100, True, "fused_ptr", ONE_WAVE_ROWS),
+    ("tile-order-row-lists", 6, 256, 245, 300, True, "fused_ptr", ONE_WAVE_ROWS),
+    ("tail, 48 scenes", 48, 40, 56, 20, False, "fused_ptr", ONE_WAVE),
+    ("tail, 1254 blocks", 1, 600, 520, 40, False, "fused_ptr", ONE_WAVE),
+    ("tail, odd", 2, 301, 333, 47, False, "fused_ptr", ONE_WAVE),
+], ids=lambda v: v if isinstance(v, str) and " " in v else None)
+def test_gpu_tests_reach_their_kernels(program, name, B, H, W, T, segments, entry, kernel):
+    """The sizes of GPU tests that name a kernel launch it."""
+    program(f"""
+        import os, re
+        if not {segments}:
+            os.environ["DRH_NO_SEGMENTS"] = "1"
+        B, H, W, T = {B}, {H}, {W}, {T}
+        params, bg = np.zeros((B, T, 10), np.float32), np.zeros((B, 3), np.float32)
+        img, losses, grads = np.zeros((B, H, W, 3), np.float32), np.zeros(B, np.float32), np.zeros((B, T, 10), np.float32)
+        out = (addr(grads),) if "{entry}" == "from_grad_ptr" else (addr(losses), addr(grads))
+        names = launched(lambda: ctx.{entry}(addr(params), addr(bg), addr(img), B, T, H, W, .002, *out))
+        assert any(re.search("{kernel}", n) for n in names), names
+    """)
