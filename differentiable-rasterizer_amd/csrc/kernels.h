@@ -37,13 +37,14 @@ enum RecField : int {
     R_D = 40,      // 6: unit edge directions (fast path only)
     R_SOFF = 46,   // 3: a . d per edge
     R_LEN = 49,    // 3: |e|
-    R_EB = 52,     // 3 x 8: per edge a.x a.y e.x e.y |e|^2 1/|e|^2 (+-1: F_CCW) 0 (scalar-loaded by edge index)
+    R_EB = 52,     // 3 x 8: per edge a.x a.y e.x e.y |e|^2 1/|e|^2 s 0 (scalar-loaded by edge index); s = +-1: the orientation
 };
-// F_CCW: the cross products of inside points are >= 0 (else <= 0).
+// The orientation s (R_EB): +1 where the cross products of inside points are >= 0,
+// else -1 (they are <= 0).
 // F_LIVE: drawn by this call's forward pass. F_TAPE: live for the taped forward
 // of the gradient paths, which culls a NaN alpha that a render composites; it
 // differs from F_LIVE only in records made by a render kept for a backward.
-enum : int { F_LIVE = 1, F_ACTIVE = 2, F_FAST = 4, F_CCW = 8, F_TAPE = 16 };
+enum : int { F_LIVE = 1, F_ACTIVE = 2, F_FAST = 4, F_TAPE = 8 };
 
 // MODE_RECORD is a forward pass only: MODE_RENDER's image plus MODE_GRAD_IN's
 // hand-over to the backward kernel, for a render whose backward comes later.

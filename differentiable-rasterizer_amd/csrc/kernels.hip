@@ -304,7 +304,7 @@ __device__ inline void setup_part(const float* __restrict__ p, size_t i, int par
         eb[3] = ey;
         eb[4] = len2;
         eb[5] = rlen2;
-        eb[6] = s;  // F_CCW as a factor: c eb[6] >= 0 inside
+        eb[6] = s;  // c eb[6] >= 0 inside
         eb[7] = 0.0f;
         return;
     }
@@ -322,8 +322,7 @@ __device__ inline void setup_part(const float* __restrict__ p, size_t i, int par
     ri[R_BOX + 2] = live ? box.x1 : 0;
     ri[R_BOX + 3] = live ? box.y1 : 0;
     const bool active = p[9] > 0.0f && p[9] < 1.0f;  // grad.rs:145
-    ri[R_FLAGS] = (live ? F_LIVE : 0) | (active ? F_ACTIVE : 0) | (fast && live ? F_FAST : 0) |
-                  (area2 >= 0.0f ? F_CCW : 0) | (taped ? F_TAPE : 0);
+    ri[R_FLAGS] = (live ? F_LIVE : 0) | (active ? F_ACTIVE : 0) | (fast && live ? F_FAST : 0) | (taped ? F_TAPE : 0);
     r[R_SPARE] = 0.0f;
     // Far outside: at a true distance d >= sigma (ln(alpha / MIN_WEIGHT) + 0.05)
     // the weight is alpha * sigmoid(-d / sigma) < alpha e^(-d / sigma)
