@@ -2218,8 +2218,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void fu
 // LDS (dynamic, seg_lds_bytes): the entries' words and lanes (20 bytes each, at
 // most T) and one area that holds the waves' lists, then the block buffers, the
 // S handed-over states and the totals, then phase C's transposition areas. Small
-// blocks keep it small (S = 2: 8.7 KB and 20 bytes a triangle): a grid of 4096
-// tiles of two waves is one round of a device with 24 of them on a CU.
+// blocks keep it small, S = 2: 8.7 KB and 20 bytes a triangle, 14 workgroups on a
+// CU at T = 128 (3584 of a grid's tiles at once on 256 CUs), 8 at T = 512.
 //
 // An earlier form gave each of eight waves an eighth of the triangles for all
 // three phases, with every wave compositing all entries: its LDS held every
