@@ -2036,10 +2036,12 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(DET 
 // once, each chunk waited for before the next: when the last tile stores, the
 // earlier chunks are summed. Polling every slot of a large scene before summing
 // any (its loads one block after another) took ~13 us at 512x512 (B=1, T = 128
-// medium triangles: 36.1 -> 22.9 us per call). A chunk loads only the blocks that
-// there are: polling its 64 TAIL_U for scenes of 16 blocks, every lane the last
-// one's, took memory from the tiles (T = 8 small triangles, 64x64: B=64 14.0 ->
-// 12.5 us, B=256 21.6 -> 19.8).
+// medium triangles: 36.1 -> 22.9 us per call). The last chunk
+// loads one or two blocks a lane where it has no more: polling 64 TAIL_U for scenes
+// of 16 blocks, every lane the last one's, took memory from the tiles (T = 8 small
+// triangles, 64x64: B=64 13.8 -> 13.1 us; medium, B=256 22.5 -> 21.3). The kernels
+// mark its branch unlikely, which lays its code out behind the tiles' (B=16 256x256
+// T=128: 79.4 us with it in front, 78.9 behind).
 constexpr int TAIL_U = 4;           // blocks per lane and chunk (scenes of up to 256 blocks: one chunk)
 constexpr int TAIL_SPIN = 1 << 22;  // polls in all, each at least one round trip to memory
 __device__ inline double tail_load(const double* p) {
@@ -2047,42 +2049,51 @@ __device__ inline double tail_load(const double* p) {
 }
 __device__ inline bool tail_pending(double v) { return (uint64_t)__double_as_longlong(v) == LOSS_PENDING; }
 
+// U blocks per lane from block r0 on, polled until none is pending and added to l:
+// false if that takes too long.
+template <int U>
+__device__ inline bool tail_chunk(const double* pl, int r0, int nblk, int& spin, double& l) {
+    double v[U][WAVES];
+    for (;;) {
+        bool pending = false;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int r = min(r0 + 64 * u, nblk - 1);  // past the end: the last block's, not added
+#pragma unroll
+            for (int q = 0; q < WAVES; q++) v[u][q] = tail_load(pl + (size_t)r * WAVES + q);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int q = 0; q < WAVES; q++) pending = pending || tail_pending(v[u][q]);
+        if (lane_mask(pending) == 0) break;
+        if (++spin >= TAIL_SPIN) return false;
+        __builtin_amdgcn_s_sleep(2);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        double lb = v[u][0];
+#pragma unroll
+        for (int q = 1; q < WAVES; q++) lb += v[u][q];
+        l = r0 + 64 * u < nblk ? l + lb : l;
+    }
+    return true;
+}
+
 __device__ inline void loss_tail(const RasterArgs& a, int b) {
     const int lane = threadIdx.x & 63, nblk = a.gx * a.gy;
     const double* pl = a.partial_loss + (size_t)b * nblk * WAVES;
     double l = 0.0;
     bool ok = true;
     int spin = 0;
-    for (int r0 = lane; __builtin_amdgcn_readfirstlane(r0) < nblk && ok; r0 += 64 * TAIL_U) {
-        const int left = nblk - __builtin_amdgcn_readfirstlane(r0);  // blocks from this chunk on
-        double v[TAIL_U][WAVES] = {};
-        for (;;) {
-            bool pending = false;
-#pragma unroll
-            for (int u = 0; u < TAIL_U; u++) {
-                if (64 * u >= left) break;
-                const int r = min(r0 + 64 * u, nblk - 1);  // past the end: the last block's, not added
-#pragma unroll
-                for (int q = 0; q < WAVES; q++) v[u][q] = tail_load(pl + (size_t)r * WAVES + q);
-            }
-#pragma unroll
-            for (int u = 0; u < TAIL_U; u++)
-#pragma unroll
-                for (int q = 0; q < WAVES; q++) pending = pending || tail_pending(v[u][q]);
-            if (lane_mask(pending) == 0) break;
-            if (++spin >= TAIL_SPIN) {
-                ok = false;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
-        }
-#pragma unroll
-        for (int u = 0; u < TAIL_U; u++) {
-            double lb = v[u][0];
-#pragma unroll
-            for (int q = 1; q < WAVES; q++) lb += v[u][q];
-            l = r0 + 64 * u < nblk ? l + lb : l;
-        }
+    for (int r0 = 0; r0 < nblk && ok; r0 += 64 * TAIL_U) {
+        const int left = nblk - r0;
+        if (left > 128)
+            ok = tail_chunk<TAIL_U>(pl, r0 + lane, nblk, spin, l);
+        else if (left > 64)
+            ok = tail_chunk<2>(pl, r0 + lane, nblk, spin, l);
+        else
+            ok = tail_chunk<1>(pl, r0 + lane, nblk, spin, l);
     }
     l = wave_sum_f64(l);
     if (lane == 0) a.losses[b] = ok ? (float)(l / (3.0 * (double)a.H * (double)a.W)) : __builtin_nanf("");
@@ -2097,7 +2108,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) void fu
     if (a.halt && *a.halt >= 0) return;
     if (MODE == MODE_LOSS && a.loss_tail) {
         // the last B workgroups: the last row of a two-dimensional grid
-        if (gridDim.y > 1 ? blockIdx.y == gridDim.y - 1 : (int)blockIdx.x >= (int)gridDim.x - a.B) {
+        if (__builtin_expect(gridDim.y > 1 ? blockIdx.y == gridDim.y - 1 : (int)blockIdx.x >= (int)gridDim.x - a.B, 0)) {
             loss_tail(a, gridDim.y > 1 ? (int)blockIdx.x : (int)blockIdx.x - ((int)gridDim.x - a.B));
             return;
         }
@@ -2254,7 +2265,7 @@ __global__ __launch_bounds__(S * 64) void fused_seg_kernel(RasterArgs a, const f
     extern __shared__ __attribute__((aligned(16))) float seg_lds[];
     // a stopped fit: tested once the list is made, which need not wait for the load
     const int halted = a.halt ? *a.halt : -1;
-    if (MODE == MODE_LOSS && !DET && a.loss_tail && (int)blockIdx.x >= (int)gridDim.x - a.B) {
+    if (MODE == MODE_LOSS && !DET && __builtin_expect(a.loss_tail && (int)blockIdx.x >= (int)gridDim.x - a.B, 0)) {
         if (threadIdx.x < 64 && halted < 0) loss_tail(a, (int)blockIdx.x - ((int)gridDim.x - a.B));
         return;
     }

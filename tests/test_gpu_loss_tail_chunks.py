@@ -34,9 +34,9 @@ def test_tail_chunks(ctx, B, H, W):
     assert np.array_equal(tail, fixed)
 
 
-# 1, 2, 16, 63, 64, 65, 128 and 130 blocks a scene: the last lanes and loads of a chunk have none
-@pytest.mark.parametrize("H,W", [(9, 16), (17, 5), (64, 64), (112, 131), (128, 128), (80, 200), (128, 256), (160, 208)],
-                         ids=lambda v: str(v))
+# 1, 2, 16, 63, 64, 65, 128, 130 and 357 blocks a scene: one, two and four loads a lane, the last lanes without
+@pytest.mark.parametrize("H,W", [(9, 16), (17, 5), (64, 64), (112, 131), (128, 128), (80, 200), (128, 256), (160, 208),
+                                 (336, 272)], ids=lambda v: str(v))
 @pytest.mark.parametrize("B", [1, 9])
 def test_tail_of_small_scenes(ctx, B, H, W):
     T, sigma = 8, 0.01
