@@ -351,6 +351,7 @@ __device__ inline void setup_part(const float* __restrict__ p, size_t i, int par
 // SETUP_REC_PER triangles: one CU issues the stores' cache lines at about one per
 // cycle, so 512 records on one CU took ~6 us and on four ~1.5.
 constexpr int SETUP_THREADS = 1024, ORD_BUCKETS = 1024, ORD_REACH = 512, SETUP_REC_PER = 128;
+constexpr int SETUP_ROUND = 512;  // workgroups that run at once on 256 CUs
 static_assert(ORD_BUCKETS == 16 * 64 && SETUP_THREADS % 64 == 0 && ORD_REACH <= SETUP_THREADS,
               "order workgroup shape: 16 buckets per lane of one wave");
 
@@ -2823,7 +2824,15 @@ hipError_t launch_setup(const float* params, int B, int T, int W, int H, float s
     RowArgs ra = rows;
     const int teams = n / 64 / min(n / 64, ROW_TEAM);  // rows a workgroup lists at a time
     ra.parts = rows.rows ? min((rows.gy + teams - 1) / teams, 16384) : 0;
-    const int gx = min((T + per - 1) / per, 65534 - ra.parts) + ra.parts + (o.perm || T == 0 ? 1 : 0);
+    int recs = min((T + per - 1) / per, 65534 - ra.parts);
+    // Without an order, one round of the device (two workgroups a CU by their LDS)
+    // where that takes the records at most two strides: a second round of a few
+    // workgroups left the one-wave kernel's waves of a 1024-tile grid on uneven
+    // SIMDs (B=16 64x64 T=2000 large triangles: 1257 -> 1192 us, setup 10.7 of it
+    // either way; IEEE mode 1982 -> 1764).
+    const int round = SETUP_ROUND / B - ra.parts;
+    if (!o.perm && recs > round && recs <= 2 * round) recs = round;
+    const int gx = recs + ra.parts + (o.perm || T == 0 ? 1 : 0);
     OrderArgs oa = o;
     const float cs = (float)(1 << o.shift);
     oa.r_h = 1.0f / (float)H;

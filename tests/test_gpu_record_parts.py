@@ -7,7 +7,7 @@ three give equal images, bit for bit.
 import numpy as np
 import pytest
 
-from bars import check_image
+from bars import assert_grads, check_image, check_losses
 from diffrast import synth
 
 pytestmark = pytest.mark.gpu
@@ -39,3 +39,25 @@ def test_record_counts(ctx, orc, T):
         assert np.array_equal(many[i], two[i % 2])
     for b in range(2):
         assert np.array_equal(ctx.render(params[b:b + 1], H, W, SIGMA, bgs[b:b + 1])[0], two[b])
+
+
+@pytest.mark.parametrize("T", [1537, 1700, 3000])
+def test_records_in_two_strides(ctx, orc, T):
+    # 16 scenes of 8 tile rows: 8 + T / 64 setup workgroups each, past 512 in all from 1537
+    # triangles (64 a workgroup); a scene alone takes its records in one stride
+    H, W = 64, 60
+    print(f"record strides T={T}", flush=True)
+    params = synth.batch("small", 2, T, 4200)
+    bgs = synth.uniforms(4207, 6).reshape(2, 3).astype(np.float32)
+    targets = np.stack([synth.blob_target(4200 + b, H, W) for b in range(2)])
+    many = [np.tile(x, (8,) + (1,) * (x.ndim - 1)) for x in (params, targets, bgs)]
+    img = ctx.render(many[0], H, W, SIGMA, many[2])
+    losses, grads = ctx.fused_loss_backward(many[0], many[1], SIGMA, many[2])
+    want = orc.loss_backward_batch(params, targets, SIGMA, bgs)
+    for b in range(2):
+        one = ctx.render(params[b:b + 1], H, W, SIGMA, bgs[b:b + 1])[0]
+        check_image(one[None], orc.render_batch(params[b:b + 1], H, W, SIGMA, bgs[b:b + 1]))
+        for i in range(b, 16, 2):
+            assert np.array_equal(img[i], one)
+            check_losses(losses[i:i + 1], want[0][b:b + 1])
+            assert_grads(grads[i:i + 1], want[1][b:b + 1])
