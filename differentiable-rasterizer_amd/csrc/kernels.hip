@@ -623,7 +623,11 @@ struct Soft {
 // raster.rs:79-87 of sd / sigma. The reference's two branches are one function,
 // 1 / (1 + e^-x): formed from one hardware exponential it is as exact on both
 // sides (1 + e^-x rounds once, and where e^-x overflows the result is 0), in
-// five instructions instead of nine with both branches and a select.
+// five instructions instead of nine with both branches and a select. Against 64
+// bits over 17 sigma on both sides, sigma 0.001 to 0.02: relative error 1.9e-7 to
+// 3.6e-7 rms and at most 1.6e-6; with both branches 3.0e-7 to 3.5e-7 and 2.3e-6
+// (the exponent's factor was rounded twice). A fit differs by it, as by any last
+// bit (after 96 iterations 1e-6 to 6e-5 of the losses, and as near to 64 bits).
 template <bool FAST>
 __device__ inline float coverage_of(float sd, const Soft& so) {
     if (FAST) return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(sd * so.nl2));

@@ -301,7 +301,7 @@ struct RasterBufs {
     float* ckpt = nullptr;          // split backward's checkpoints, or null: no split
     int nseg = 1, seg_m = 0, nsplit = 0;  // its segments, entries per segment, split blocks per scene
     bool fused = false;             // one fused kernel (fused_gradients); pq, pg0, pze, tn unused
-    bool order_tiles = false;       // `order` ranks 8x8 tiles (one-wave fused kernel only), not blocks
+    bool order_tiles = false;       // `order` ranks 8x8 tiles (one-wave and segmented kernels), not blocks
     int2* rows = nullptr;           // B*2gy*T entries of the tile rows' lists (RowArgs), or null
     int* row_n = nullptr;           // B*2gy counts
     int segw = 0;                   // fused_seg_kernel's waves per tile (RasterArgs::segw), or 0
